@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "mcpi_internal.h"
+#include "pair_rows.h"
 
 namespace mcpi {
 
@@ -102,6 +103,49 @@ __global__ void k_rank_states(int N, int M, int64_t n_states, const int32_t *__r
     for (int i = M - 1; i > 0; i--)
         for (int p = w[i]; p > 0; p--) { k += NCmat[n_left + (N + 1) * i]; n_left--; }
     out[t] = k;
+}
+
+// Occupations of the states with N - 2 particles, one byte per orbital in rows
+// of two (M <= 16) or four 64-bit words: one thread per state, greedy over the
+// rank table B of the basis with N particles.
+__global__ __launch_bounds__(256) void k_unrank_occ(int N, int M, int64_t nu, const int32_t *__restrict__ B,
+                                                    uint64_t *__restrict__ occ)
+{
+    extern __shared__ int32_t occ_bt[];
+    const int NB1 = N + 1;
+    for (int x = threadIdx.x; x < M * NB1; x += 256) occ_bt[x] = B[x];
+    __syncthreads();
+    const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (u >= nu) return;
+    uint64_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
+    auto put = [&](int j, int v) {
+        const uint64_t z = (uint64_t)v << (8 * (j & 7));
+        w0 |= j < 8 ? z : 0;
+        w1 |= j >= 8 && j < 16 ? z : 0;
+        w2 |= j >= 16 && j < 24 ? z : 0;
+        w3 |= j >= 24 ? z : 0;
+    };
+    int64_t R = nu - 1 - u;
+    int p = N - 2, above = N - 2, j = M - 1;
+    while (j >= 1) {
+        const int64_t bj = occ_bt[j * NB1 + p];
+        if (bj > R) {
+            p--;
+        } else {
+            put(j, above - p);
+            above = p;
+            R -= bj;
+            j--;
+        }
+    }
+    put(0, above);
+    uint64_t *o = occ + u * (M <= 16 ? 2 : 4);
+    o[0] = w0;
+    o[1] = w1;
+    if (M > 16) {
+        o[2] = w2;
+        o[3] = w3;
+    }
 }
 
 // Single-jump map (OneOneMap, configurationsMap.h:348-417): one thread per
@@ -561,7 +605,8 @@ static void free_basis(mcpi_basis b)
 {
     if (!b) return;
     void *ptrs[] = {b->d.IF,     b->d.Map,    b->d.MapOT,  b->d.MapTT,  b->d.strideOT, b->d.strideTT,
-                    b->d.B,      b->d.NCmat,  b->d.packOT, b->d.packTT, b->d.poffOT,   b->d.poffTT};
+                    b->d.B,      b->d.NCmat,  b->d.packOT, b->d.packTT, b->d.poffOT,   b->d.poffTT,
+                    b->d.occ2};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (PatternTables &t : b->patterns) {
@@ -593,6 +638,27 @@ static mcpi_status alloc_dev(void **p, int64_t bytes, int64_t *acct)
         return MCPI_ERR_ALLOC;
     }
     *acct += bytes;
+    return MCPI_OK;
+}
+
+// The occupation table of the states with N - 2 particles (BasisDev::occ2),
+// unranked once here: 16 or 32 bytes a state, about an eighth of IF.  A
+// device without the memory for it goes without.
+static mcpi_status build_occ2(mcpi_basis b)
+{
+    const int N = b->d.N, M = b->d.M;
+    if (N < 2) return MCPI_OK;
+    const int64_t nu = mcpi::nc_of(N - 2, M), bytes = nu * occ_stride(M);
+    void *p = nullptr;
+    if (hipMalloc(&p, (size_t)bytes + 64) != hipSuccess) {
+        (void)hipGetLastError();
+        return MCPI_OK;
+    }
+    b->device_bytes += bytes;
+    b->d.occ2 = (uint8_t *)p;
+    hipLaunchKernelGGL(k_unrank_occ, dim3((unsigned)((nu + 255) / 256)), dim3(256), sizeof(int32_t) * M * (N + 1), 0,
+                       N, M, nu, b->d.B, (uint64_t *)p);
+    MCPI_HIP(hipGetLastError());
     return MCPI_OK;
 }
 
@@ -635,6 +701,11 @@ static mcpi_status basis_init(int N, int M, const int32_t *IF_host, const int32_
             free_basis(b);
             return hip_fail(e, "unrank kernel", __FILE__, __LINE__);
         }
+    }
+    const mcpi_status so = build_occ2(b);
+    if (so != MCPI_OK) {
+        free_basis(b);
+        return so;
     }
     *out = b;
     return MCPI_OK;
@@ -996,6 +1067,16 @@ mcpi_status mcpi_hip_basis_create(int N, int M, int maps, mcpi_basis *out)
         return st;
     }
     *out = b;
+    return MCPI_OK;
+}
+
+// Frees the occupation table, as if the device had had no memory for it when
+// the basis was created (for tests; not part of the public interface).
+mcpi_status mcpi_hip_basis_drop_occ2(mcpi_basis b)
+{
+    MCPI_ARG(b, "null basis");
+    if (b->d.occ2) MCPI_HIP(hipFree(b->d.occ2));
+    b->d.occ2 = nullptr;
     return MCPI_OK;
 }
 

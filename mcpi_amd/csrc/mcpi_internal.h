@@ -95,6 +95,10 @@ struct BasisDev {
     int64_t *strideTT;  // nc+1 entries (last = |MapTT|) or null
     int32_t *B;         // (M) x (N+1) table B[j*(N+1) + p], row 0 unused
     int32_t *NCmat;     // (N+1)*(M+1), reference layout
+    // occupations of the states with N - 2 particles, one byte per orbital in
+    // rows of 16 (M <= 16) or 32 bytes; null for N < 2, or when the device had
+    // no memory for it (the pair amplitudes then unrank their rows)
+    uint8_t *occ2;
     // Wave-packed double-jump targets (full maps only; see basis.hip): for
     // each wavefront of 64 consecutive rows w, the slots of the jumps active
     // in any of its lanes, from int offset poffOT[w] / poffTT[w]

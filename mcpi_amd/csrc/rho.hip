@@ -35,18 +35,36 @@
 // combinatorial number system) and its two difference tables are kept in
 // LDS, so a gather costs two LDS reads and two subtractions.
 //
-// Kernel: a block owns one tile pair (TI, TJ) of 80 x 80 entries of the
-// Gram matrix and loops over tiles of U rows of Phi (32 for rho2, 128 for
-// rho1, whose Phi has at most 32 columns): it unranks the rows (one thread
-// per row), gathers the U x 16 NG (x 2 off the diagonal) entries of Phi
-// into LDS (lanes over consecutive rows of one column: neighbouring
-// targets; GB loads in flight per thread), then every thread adds its
-// entry of each 16 x 16 sub-block (the sub-blocks i <= j of a diagonal
-// tile pair, all of them off it) with FP64 FMAs.  Each block writes its
-// tile once; two fixed-order stages sum the blocks (deterministic result),
-// and a last kernel expands the Gram matrix into the full rho1 / rho2
-// arrays on the device.  No map is read, so the densities run on every
-// storage mode, and the vectors are in the reference order.
+// Kernel k_gram: a block owns one tile pair (TI, TJ) of 80 x 80 entries of
+// the Gram matrix and loops over tiles of U rows of Phi (32 for rho2, 128
+// for rho1, whose Phi has at most 32 columns).  The tile's rows are
+// unranked (one thread per row, during the previous tile's products), its
+// entries gathered into LDS (lanes over consecutive rows of one column:
+// neighbouring targets; GB loads in flight per thread), and the product
+// runs on the FP64 matrix cores in 16 x 16 sub-blocks: the sub-blocks i <= j
+// of a diagonal tile pair, all of them off it, dealt out to the block's four
+// wavefronts.  Phi stays in LDS in one layout for both operands, because
+// v_mfma_f64_16x16x4f64 takes A[i][k] and B[k][j] from the same lanes
+// (i or j = lane % 16, k = lane / 16): lane (i, k) of step s reads column i of
+// row 4 s + k.
+// The bound is FP64: a complex product is three real ones here (Gauss), 6
+// operations for each entry of the sub-blocks and row, against 8 on the vector
+// units.  Eight wavefronts a block with at most two sub-blocks each leave room
+// for two blocks a CU, so that one block's gathers and row tables run beside
+// the other's products (four wavefronts with four sub-blocks each: 2.34 ms at
+// N = 16, M = 12; three such blocks without gathers in flight over the
+// products: 2.38 ms).  rho1 and rho2 together, kernels, sums and expansion, at
+// M = 12: N = 12 (352,716 rows of 78 columns) 0.45 -> 0.20 ms, of which the
+// product 0.32 -> 0.18; N = 16 (4,457,400 rows) 5.26 -> 2.12 ms, the product
+// 4.2 -> 2.1 ms or 49 TFLOP/s issued (before: vector FMAs, unranked rows and a
+// Gram product of its own for rho1).
+// Each block writes its sub-blocks once; two fixed-order stages sum the
+// blocks (deterministic result), the second one inside the kernel that
+// expands the Gram matrix into the full rho1 / rho2 arrays on the device.
+// With rho2 at hand rho1 needs no Gram product of its own: on N >= 2
+// particles sum_s a*_k a*_s a_s a_l = (N - 1) a*_k a_l.  No map is read, so
+// the densities run on every storage mode, and the vectors are in the
+// reference order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -56,6 +74,7 @@
 #include <vector>
 
 #include "mcpi_internal.h"
+#include "pair_rows.h"
 
 namespace mcpi {
 
@@ -65,23 +84,33 @@ constexpr int GT = 80;            // Gram tile side (columns of Phi per tile)
 constexpr int GG = GT / 16;       // 16 x 16 sub-blocks per tile side
 constexpr int GU2 = 32;           // rows of Phi per LDS tile, rho2
 constexpr int GU1 = 128;          // rows of Phi per LDS tile, rho1 (16 or 32 columns)
-constexpr int GTHREADS = 256;     // 16 x 16 threads: one entry of each sub-block
-constexpr int GTILE = GT * GT;    // entries of one tile
-constexpr int GB = 5;             // gathers in flight per thread
-constexpr int GSEG = 32;          // segments of the first stage of the block sums
+constexpr int GWAVES = 8;         // wavefronts of a block
+constexpr int GTHREADS = 64 * GWAVES;
+constexpr int GSEG = 8;           // segments of the first stage of the block sums
+
+typedef double mcpi_v4d __attribute__((ext_vector_type(4)));
+
+// sub-blocks of a tile pair with ng column groups a side
+__host__ __device__ constexpr int gram_subblocks(int ng, bool diag) { return diag ? ng * (ng + 1) / 2 : ng * ng; }
+
+// LDS row stride of a tile of Phi in complex entries: odd, so that the lanes
+// of a gather write rows on distinct banks
+__host__ __device__ constexpr int gram_stride(int ng) { return 16 * ng + 1; }
 
 struct GramArgs {
     int N, M, ord;       // particles and orbitals of the basis; annihilators (1: rho1, 2: rho2)
     int np;              // columns of Phi: M (ord 1) or M(M+1)/2 (ord 2)
     int ntile;           // tiles of GT columns
-    int rs;              // LDS row stride of a Phi tile in complex entries (16 * groups + 1)
     int ng;              // 16-column groups of a full tile (<= GG)
     int64_t nc;          // states of the basis
     int64_t nu;          // rows of Phi: states of B(N - ord, M)
     int64_t nut;         // tiles of U rows
     const int32_t *B;    // rank table B[j*(N+1) + p]
+    const uint8_t *occ;  // occupations of the rows (null: unrank them)
     const cplx *C;       // vector, reference order
-    cplx *partial;       // [tile pair][block][GTILE]
+    cplx *partial;       // [block][entries]: the sub-blocks of the diagonal
+                         // tile pairs, then of the others, 256 entries each
+    int64_t entries;     // entries of one block's partial
 };
 
 __device__ inline cplx ldc(const cplx *p)
@@ -106,12 +135,14 @@ __host__ __device__ inline int off_index(int TI, int TJ, int T)
     return TI * (2 * T - TI - 1) / 2 + (TJ - TI - 1);
 }
 
-// LDS layout of a block (dynamic shared memory, in this order)
+// LDS layout of a block (dynamic shared memory, in this order); red: the
+// wavefronts' sums where they split the rows, over the tiles (which are
+// done with by then)
 struct GramLds {
-    size_t phiA, phiB, tt, dq, dl, sq, bt, ql, pp, bytes;
+    size_t phiA, phiB, g, sq, ql, tt, dd, bt, bytes;
 };
 
-__host__ __device__ inline GramLds gram_lds(int N, int M, int np, int rs, bool diag, int GU, int ord)
+__host__ __device__ inline GramLds gram_lds(int N, int M, int np, int ng, bool diag, int GU, int ord, size_t red)
 {
     GramLds L;
     size_t o = 0;
@@ -121,241 +152,363 @@ __host__ __device__ inline GramLds gram_lds(int N, int M, int np, int rs, bool d
         o += n;
         return r;
     };
-    L.phiA = take(sizeof(cplx) * GU * rs, 16);
-    L.phiB = diag ? L.phiA : take(sizeof(cplx) * GU * rs, 16);
-    L.tt = take(sizeof(int64_t) * GU, 8);
-    L.dq = take(sizeof(int64_t) * GU * M, 8);
-    L.dl = take(sizeof(int64_t) * GU * M * (ord == 2), 8);
+    L.phiA = take(sizeof(cplx) * GU * gram_stride(ng), 16);
+    L.phiB = diag ? L.phiA : take(sizeof(cplx) * GU * gram_stride(ng), 16);
+    if (o < red) o = red;
+    L.g = take(sizeof(double) * GU * M * ord, 8);
     L.sq = take(sizeof(double) * (N + 3), 8);
+    L.ql = take(sizeof(uint2) * np, 8);
+    L.tt = take(sizeof(int32_t) * GU, 4);
+    L.dd = take(sizeof(int32_t) * GU * M * ord, 4);
     L.bt = take(sizeof(int32_t) * M * (N + 1), 4);
-    L.ql = take(sizeof(uint16_t) * np, 2);
-    L.pp = take((size_t)GU * (M + 1), 1);
     L.bytes = (o + 15) / 16 * 16;
     return L;
 }
 
+// How the wavefronts share the sub-blocks of a tile pair: WK of them split
+// the rows (steps of four) and GWAVES / WK split the sub-blocks, at most NB
+// each.  Few sub-blocks leave wavefronts without one, so they split the rows
+// there and add their sums in LDS at the end.
+template <bool DIAG, int NG>
+struct GramSplit {
+    static constexpr int SB = gram_subblocks(NG, DIAG);
+    static constexpr int WK = SB <= 3 ? 8 : (SB <= 6 ? 4 : (SB <= 10 ? 2 : 1));
+    static constexpr int WB = GWAVES / WK;
+    static constexpr int NB = (SB + WB - 1) / WB;
+    static constexpr size_t red = WK > 1 ? sizeof(cplx) * 256 * NB * WB * (WK - 1) : 0;
+    // per SIMD: sub-blocks take 24 registers each, and 4 wavefronts (two
+    // blocks of a CU in turn) leave 128
+    static constexpr int WAVES = NB <= 2 ? 4 : 2;
+};
+
 // Block partials of one tile pair of Phi^H Phi.  DIAG: tile pair (TI, TI)
 // from blockIdx.y, sub-blocks i <= j; else the off-diagonal pair
-// off_pair(blockIdx.y), all sub-blocks.
-template <bool DIAG, int GU, int NG>
-__global__ __launch_bounds__(GTHREADS) __attribute__((amdgpu_waves_per_eu(DIAG ? 3 : 2))) void k_gram(GramArgs a)
+// off_pair(blockIdx.y), all sub-blocks.  OW > 0: the rows come
+// from the occupation table, OW words each (rho2 only), else they are
+// unranked.
+template <bool DIAG, int GU, int NG, int OW>
+__global__ __launch_bounds__(GTHREADS) __attribute__((amdgpu_waves_per_eu(GramSplit<DIAG, NG>::WAVES))) void
+k_gram(GramArgs a)
 {
+    using S = GramSplit<DIAG, NG>;
+    constexpr int NB = S::NB, RS = gram_stride(NG);
     extern __shared__ __align__(16) unsigned char lds[];
-    const GramLds L = gram_lds(a.N, a.M, a.np, a.rs, DIAG, GU, a.ord);
+    const GramLds L = gram_lds(a.N, a.M, a.np, NG, DIAG, GU, a.ord, S::red);
     cplx *phiA = (cplx *)(lds + L.phiA);
     cplx *phiB = (cplx *)(lds + L.phiB);
-    int64_t *tt = (int64_t *)(lds + L.tt);
-    int64_t *dq = (int64_t *)(lds + L.dq);
-    int64_t *dl = (int64_t *)(lds + L.dl);
+    double *g = (double *)(lds + L.g);        // sqrt(u_o + 1), then sqrt(u_o + 2): [orbital][row]
     double *sq = (double *)(lds + L.sq);
+    uint2 *ql = (uint2 *)(lds + L.ql);        // a column's places in dd and g (see below)
+    int32_t *tt = (int32_t *)(lds + L.tt);    // rank(u + ord e_0), -1 past the last row
+    int32_t *dd = (int32_t *)(lds + L.dd);    // S_0 - S_1, then S_1 - S_2: [orbital][row]
     int32_t *Bt = (int32_t *)(lds + L.bt);
-    uint16_t *ql = (uint16_t *)(lds + L.ql);
-    uint8_t *pp = lds + L.pp;
 
     const int t = threadIdx.x;
-    const int N = a.N, M = a.M, NB = N + 1, Np = N - a.ord;
+    const int N = a.N, M = a.M, NB1 = N + 1, Np = N - a.ord;
     int TI, TJ;
     if (DIAG) TI = TJ = blockIdx.y;
     else off_pair(blockIdx.y, a.ntile, TI, TJ);
-    const int tp = DIAG ? TI : a.ntile + (int)blockIdx.y;
 
-    for (int x = t; x < M * NB; x += GTHREADS) Bt[x] = a.B[x];
+    for (int x = t; x < M * NB1; x += GTHREADS) Bt[x] = a.B[x];
     for (int x = t; x < N + 3; x += GTHREADS) sq[x] = sqrt((double)x);
+    // column p = pair (q, l) or orbital q: its entries of dd at x (low half
+    // q, high half l), the second root at y (sqrt(u_l + 1), or sqrt(u_l + 2)
+    // for q = l; the first is at q)
     for (int x = t; x < a.np; x += GTHREADS) {
+        int q = x, l = 0;
         if (a.ord == 2) {
-            int l = 0;
             while ((l + 1) * (l + 2) / 2 <= x) l++;
-            ql[x] = (uint16_t)((x - l * (l + 1) / 2) | (l << 8));
-        } else {
-            ql[x] = (uint16_t)(x | (x << 8));
+            q = x - l * (l + 1) / 2;
         }
+        ql[x] = make_uint2((unsigned)(q * GU) | (unsigned)((M + l) * GU) << 16,
+                           (unsigned)((q == l ? M + l : l) * GU));
     }
+    __syncthreads();
     // columns of the two sides (NG groups of 16, a.ng == NG; the columns of
     // a narrower last tile past wA / wB hold zeros, so every sub-block is
     // computed without a test)
     const int wA = min(GT, a.np - TI * GT), wB = min(GT, a.np - TJ * GT);
-    const int r = t >> 4, c = t & 15;
 
-    cplx acc[NG][NG];
-#pragma unroll
-    for (int i = 0; i < NG; i++)
-#pragma unroll
-        for (int j = 0; j < NG; j++) acc[i][j] = cmake(0, 0);
-
-    constexpr int ncolA = 16 * NG, ncolB = DIAG ? 0 : 16 * NG;
-    const int nent = GU * (ncolA + ncolB);
-    for (int64_t tile = blockIdx.x; tile < a.nut; tile += gridDim.x) {
-        __syncthreads();   // the previous tile's Gram reads are done
-        const int64_t u0 = tile * GU;
-        // rows of the tile: unrank (greedy over B), difference tables
-        if (t < GU) {
-            const int64_t u = u0 + t;
-            uint8_t *P = pp + t * (M + 1);
-            if (u < a.nu) {
-                // one step per iteration (lower p, or settle orbital j and
-                // move down), so the lanes of a wavefront stay together:
-                // at most Np + M - 1 iterations
-                int64_t R = a.nu - 1 - u;
-                int pj = Np, j = M - 1;
-                P[M] = (uint8_t)Np;
-                while (j >= 1) {
-                    const int64_t bj = Bt[j * NB + pj];
-                    if (bj > R) {
-                        pj--;
-                    } else {
-                        P[j] = (uint8_t)pj;
-                        R -= bj;
-                        j--;
-                    }
-                }
-                P[0] = 0;
-                int64_t s0 = 0, s1 = 0, s2 = 0;
-                int64_t *Dq = dq + t * M;
-                Dq[0] = 0;
-                if (a.ord == 2) {   // the second table exists for rho2 only
-                    int64_t *Dl = dl + t * M;
-                    Dl[0] = 0;
-                    for (int j = 1; j < M; j++) {
-                        const int b = j * NB + P[j];
-                        s0 += Bt[b];
-                        s1 += Bt[b + 1];
-                        s2 += Bt[b + 2];
-                        Dq[j] = s0 - s1;
-                        Dl[j] = s1 - s2;
-                    }
-                } else {
-                    for (int j = 1; j < M; j++) {
-                        const int b = j * NB + P[j];
-                        s0 += Bt[b];
-                        s1 += Bt[b + 1];
-                        Dq[j] = s0 - s1;
-                    }
-                }
-                tt[t] = a.nc - 1 - (a.ord == 2 ? s2 : s1);
+    // row r of a tile without an occupation table: unrank (greedy over B),
+    // targets and roots
+    auto unrank_row = [&](int64_t tile, int r) {
+        const int64_t u = tile * GU + r;
+        if (u >= a.nu) {
+            tt[r] = -1;
+            return;
+        }
+        // one step per iteration (lower p, or settle orbital j and move
+        // down), so the lanes of a wavefront stay together: at most
+        // Np + M - 1 iterations.  P_j falls with j: the occupation of
+        // orbital j is known when P_j is.  dd holds P_j meanwhile.
+        int32_t *dq = dd + r, *dl = dd + M * GU + r;
+        double *gq = g + r, *gl = g + M * GU + r;
+        int32_t R = (int32_t)(a.nu - 1 - u);
+        int pj = Np, pa = Np, j = M - 1;
+        while (j >= 1) {
+            const int32_t bj = Bt[j * NB1 + pj];
+            if (bj > R) {
+                pj--;
             } else {
-                tt[t] = -1;
+                dq[j * GU] = pj;
+                gq[j * GU] = sq[pa - pj + 1];
+                if (a.ord == 2) gl[j * GU] = sq[pa - pj + 2];
+                pa = pj;
+                R -= bj;
+                j--;
             }
         }
-        __syncthreads();
-        // gather the tile of Phi: lanes over consecutive rows of one column,
-        // GB entries per thread at a time (their targets first, then all
-        // their loads in flight together, then the LDS stores: a store to
-        // the tile may alias the tables as far as the compiler knows, so
-        // one entry at a time would serialize the loads)
-        for (int e0 = t; e0 < nent; e0 += GB * GTHREADS) {
-            int64_t tg[GB];
-            double f[GB];
-#pragma unroll
-            for (int k = 0; k < GB; k++) {
-                const int e = e0 + k * GTHREADS;
-                tg[k] = -1;
-                f[k] = 0;
-                const bool sideB = e >= GU * ncolA;
-                const int e2 = sideB ? e - GU * ncolA : e;
-                const int col = e2 / GU, ul = e2 % GU;
-                const int64_t base = e < nent ? tt[ul] : -1;
-                if (base >= 0 && col < (sideB ? wB : wA)) {
-                    const int p = (sideB ? TJ : TI) * GT + col;
-                    const int q = ql[p] & 255, l = ql[p] >> 8;
-                    const uint8_t *P = pp + ul * (M + 1);
-                    const int uq = P[q + 1] - P[q];
-                    if (a.ord == 2) {
-                        const int ulo = P[l + 1] - P[l];
-                        tg[k] = base - dq[ul * M + q] - dl[ul * M + l];
-                        f[k] = sq[uq + 1] * sq[ulo + 1 + (q == l)];
-                    } else {
-                        tg[k] = base - dq[ul * M + q];
-                        f[k] = sq[uq + 1];
-                    }
-                }
-            }
-            cplx v[GB];
-#pragma unroll
-            for (int k = 0; k < GB; k++) v[k] = tg[k] >= 0 ? ldc(a.C + tg[k]) : cmake(0, 0);
-#pragma unroll
-            for (int k = 0; k < GB; k++) {
-                const int e = e0 + k * GTHREADS;
-                if (e < nent) {
-                    const bool sideB = e >= GU * ncolA;
-                    const int e2 = sideB ? e - GU * ncolA : e;
-                    (sideB ? phiB : phiA)[(e2 % GU) * a.rs + e2 / GU] = cscale(v[k], f[k]);
-                }
+        gq[0] = sq[pa + 1];
+        if (a.ord == 2) gl[0] = sq[pa + 2];
+        int32_t s0 = 0, s1 = 0, s2 = 0;
+        dq[0] = 0;
+        if (a.ord == 2) dl[0] = 0;
+        for (int o = 1; o < M; o++) {
+            const int b = o * NB1 + dq[o * GU];
+            s0 += Bt[b];
+            s1 += Bt[b + 1];
+            dq[o * GU] = s0 - s1;
+            if (a.ord == 2) {
+                s2 += Bt[b + 2];
+                dl[o * GU] = s1 - s2;
             }
         }
-        __syncthreads();
-        // Gram: acc[i][j] += conj(Phi[u][16i + r]) Phi[u][16j + c]
-        // rho1 tiles (one or two column groups) keep several rows' loads in flight
-        constexpr int UN = GU == GU1 ? 4 : 1;
-#pragma unroll UN
-        for (int ul = 0; ul < GU; ul++) {
-            const cplx *ra = phiA + ul * a.rs, *rb = phiB + ul * a.rs;
-            cplx av[NG], bv[NG];
+        tt[r] = (int32_t)(a.nc - 1) - (a.ord == 2 ? s2 : s1);
+    };
+    // rows of a tile from the occupation table (pair amplitudes only): two
+    // threads a row, one for each table of differences; occ_row's load is
+    // issued a tile earlier
+    const bool duty = t < 2 * GU;
+    const int dr = t % GU, dh = t / GU;
+    constexpr int NW = OW ? OW : 1;
+    uint32_t ow[NW];
+    auto occ_row = [&](int64_t tile) {
+        const int64_t u = min(tile * GU + dr, a.nu - 1);
+        const uint4 *o = reinterpret_cast<const uint4 *>(a.occ + u * occ_stride(M));
 #pragma unroll
-            for (int i = 0; i < NG; i++) {
-                av[i] = ra[16 * i + r];
-                bv[i] = rb[16 * i + c];
+        for (int k = 0; k < OW / 4; k++) {
+            const uint4 w = o[k];
+            ow[4 * k] = w.x;
+            ow[4 * k + 1] = w.y;
+            ow[4 * k + 2] = w.z;
+            ow[4 * k + 3] = w.w;
+        }
+    };
+    auto occ_tables = [&](int64_t tile) {
+        const int32_t s = pair_row_tables<NW>(ow, M, NB1, Bt, sq, dh, dd + dh * M * GU + dr, g + dh * M * GU + dr, GU);
+        if (dh == 1) tt[dr] = tile * GU + dr < a.nu ? (int32_t)(a.nc - 1) - s : -1;
+    };
+
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int il = lane & 15, kl = lane >> 4;
+    const int wk = wave / S::WB, wb = wave % S::WB;
+    // this wavefront's sub-blocks: NB, or one fewer
+    const int sb0 = wb * S::SB / S::WB;
+    const bool last = (wb + 1) * S::SB / S::WB - sb0 == NB;
+    int bi[NB], bj[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        const int b = min(sb0 + j, S::SB - 1);
+        int I = 0, J = b;
+        if (DIAG) {
+            while (J >= NG - I) {
+                J -= NG - I;
+                I++;
+            }
+            J += I;
+        } else {
+            I = b / NG;
+            J = b % NG;
+        }
+        bi[j] = 16 * I;
+        bj[j] = 16 * J;
+    }
+
+    mcpi_v4d T1[NB], T2[NB], T3[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) T1[j] = T2[j] = T3[j] = mcpi_v4d{0, 0, 0, 0};
+
+    constexpr int SIDES = DIAG ? 1 : 2;
+    constexpr int CS = GTHREADS / GU, NK = 16 * NG / CS;   // columns side by side, and a thread's columns
+    const int ul = t % GU, c0 = t / GU;
+    // Gathers of a tile of Phi: a thread keeps to one row and takes every
+    // CS-th column (lanes over consecutive rows of one column): targets and
+    // loads, all in flight together, then (put) the LDS stores
+    cplx v[SIDES][NK];
+    double f[SIDES][NK];
+    auto get = [&]() {
+        const int32_t base = tt[ul];
+#pragma unroll
+        for (int h = 0; h < SIDES; h++) {
+            const int p0 = (h ? TJ : TI) * GT + c0, pw = (h ? TJ : TI) * GT + (h ? wB : wA);
+            int32_t tg[NK];
+#pragma unroll
+            for (int k = 0; k < NK; k++) {
+                const int p = p0 + k * CS;
+                const uint2 x = ql[p < pw ? p : 0];
+                const int xq = x.x & 0xffff;
+                tg[k] = base - dd[xq + ul];
+                f[h][k] = g[xq + ul];
+                if (a.ord == 2) {
+                    tg[k] -= dd[(x.x >> 16) + ul];
+                    f[h][k] *= g[x.y + ul];
+                }
+                // columns and rows past the last: the load goes to entry 0, put
+                // stores zero (no branch: all loads are in flight together)
+                if (base < 0 || p >= pw) {
+                    tg[k] = 0;
+                    f[h][k] = -1;
+                }
             }
 #pragma unroll
-            for (int i = 0; i < NG; i++)
+            for (int k = 0; k < NK; k++) v[h][k] = ldc(a.C + tg[k]);
+        }
+    };
+    auto put = [&]() {
 #pragma unroll
-                for (int j = 0; j < NG; j++) {
-                    if (DIAG && j < i) continue;
-                    acc[i][j] = cfma_conj(av[i], bv[j], acc[i][j]);
-                }
+        for (int h = 0; h < SIDES; h++) {
+            cplx *row = (h ? phiB : phiA) + ul * RS + c0;
+#pragma unroll
+            for (int k = 0; k < NK; k++) row[k * CS] = f[h][k] < 0 ? cmake(0, 0) : cscale(v[h][k], f[h][k]);
+        }
+    };
+
+    auto rows = [&](int64_t tile) {
+        if (tile >= a.nut) return;
+        if (OW == 0) {
+            if (t < GU) unrank_row(tile, t);
+        } else if (duty) {
+            occ_tables(tile);
+            occ_row(tile + gridDim.x);
+        }
+    };
+    // The gathers of a tile are in flight during the previous tile's
+    // products, and the row tables of the one after are made beside them (by
+    // the wavefront with the fewest sub-blocks)
+    if (OW > 0 && duty) occ_row(blockIdx.x);
+    rows(blockIdx.x);
+    if (blockIdx.x < a.nut) {
+        __syncthreads();
+        get();
+        __syncthreads();
+        rows(blockIdx.x + gridDim.x);
+    }
+    for (int64_t tile = blockIdx.x; tile < a.nut; tile += gridDim.x) {
+        const int64_t next = tile + gridDim.x;
+        put();
+        __syncthreads();   // the tile and the next one's row tables are written
+        // (the loaded occupations are taken first: waiting for them after the
+        // gathers would wait for those too)
+        if (OW > 0)
+#pragma unroll
+            for (int k = 0; k < NW; k++) asm volatile("" : "+v"(ow[k]));
+        if (next < a.nut) get();
+        __syncthreads();   // the next tile's row tables are read
+        rows(next + gridDim.x);
+        // conj(x + iy) (u + iv) = (k1 + k3) + i (k1 + k2) with k1 = u (x - y),
+        // k2 = x (v - u), k3 = y (u + v)
+#pragma unroll 2
+        for (int s = 0; s < GU / 4 / S::WK; s++) {
+            const cplx *ra = phiA + (4 * (s * S::WK + wk) + kl) * RS + il;
+            const cplx *rb = phiB + (4 * (s * S::WK + wk) + kl) * RS + il;
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                if (j == NB - 1 && !last) continue;
+                const cplx x = ra[bi[j]], y = rb[bj[j]];
+                T1[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re - x.im, y.re, T1[j], 0, 0, 0);
+                T2[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.im - y.re, T2[j], 0, 0, 0);
+                T3[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.re + y.im, T3[j], 0, 0, 0);
+            }
+        }
+        __syncthreads();   // the tile's products are done
+    }
+    // re = T1 + T3, im = T1 + T2; register r of lane j + 16 g holds entry
+    // (g + 4 r, j) of the sub-block
+    const int at = kl * 16 + il;
+    cplx *out = a.partial + (int64_t)blockIdx.x * a.entries +
+                256 * ((int64_t)(DIAG ? 0 : a.ntile * gram_subblocks(GG, true)) + (int64_t)blockIdx.y * S::SB);
+    if (S::WK > 1) {
+        cplx *red = (cplx *)lds;   // [row split - 1][sub-block][256]
+        __syncthreads();
+        if (wk > 0) {
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    red[(((wk - 1) * S::WB + wb) * NB + j) * 256 + at + 64 * r] =
+                        cmake(T1[j][r] + T3[j][r], T1[j][r] + T2[j][r]);
+        }
+        __syncthreads();
+        if (wk > 0) return;
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        if (j == NB - 1 && !last) continue;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            cplx z = cmake(T1[j][r] + T3[j][r], T1[j][r] + T2[j][r]);
+            if (S::WK > 1) {
+                const cplx *red = (const cplx *)lds;
+#pragma unroll
+                for (int w = 0; w < S::WK - 1; w++)
+                    z = cadd(z, red[((w * S::WB + wb) * NB + j) * 256 + at + 64 * r]);
+            }
+            out[(sb0 + j) * 256 + at + 64 * r] = z;
         }
     }
-    cplx *out = a.partial + ((size_t)tp * gridDim.x + blockIdx.x) * GTILE;
-#pragma unroll
-    for (int i = 0; i < GG; i++)
-#pragma unroll
-        for (int j = 0; j < GG; j++)
-            out[(16 * i + r) * GT + 16 * j + c] = (i < NG && j < NG) ? acc[i < NG ? i : 0][j < NG ? j : 0] : cmake(0, 0);
 }
 
-// Block sums in two fixed-order stages.  Stage 1: segment s of the blocks
-// (blocks s*seg .. s*seg+seg-1, in order) summed into the partial of its
-// first block; stage 2: the segment sums, in order, into G[tp][e].
-__global__ void k_gram_sum1(int ntp, int nblocks, int seg, cplx *__restrict__ partial)
+// Block sums in two fixed-order stages.  Stage 1 (this kernel): segment s of
+// the blocks (blocks s*seg .. s*seg+seg-1), in four parts of consecutive
+// blocks side by side, summed into the partial of its first block; stage 2:
+// the segment sums, in order, where they are read (GramSums).
+__global__ __launch_bounds__(256) void k_gram_sum1(int64_t entries, int nblocks, int seg, cplx *__restrict__ partial)
 {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= (int64_t)ntp * GTILE) return;
-    const int64_t tp = x / GTILE, e = x % GTILE;
-    const int b0 = blockIdx.y * seg, b1 = min(nblocks, b0 + seg);
-    if (b0 >= b1) return;
-    cplx *p = partial + tp * nblocks * GTILE + e;
+    __shared__ cplx part[4][64];
+    const int64_t x = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    const int w = threadIdx.x >> 6;
+    const int s0 = blockIdx.y * seg, s1 = min(nblocks, s0 + seg), q = (seg + 3) / 4;
+    const int b0 = s0 + w * q, b1 = min(s1, b0 + q);
     double re = 0, im = 0;
     for (int b = b0; b < b1; b++) {
-        const cplx z = p[(int64_t)b * GTILE];
+        const cplx z = ldc(partial + b * entries + x);
         re += z.re;
         im += z.im;
     }
-    p[(int64_t)b0 * GTILE] = cmake(re, im);
-}
-
-__global__ void k_gram_sum2(int ntp, int nblocks, int seg, const cplx *__restrict__ partial, cplx *__restrict__ G)
-{
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= (int64_t)ntp * GTILE) return;
-    const int64_t tp = x / GTILE, e = x % GTILE;
-    const cplx *p = partial + tp * nblocks * GTILE + e;
-    double re = 0, im = 0;
-    for (int b = 0; b < nblocks; b += seg) {
-        const cplx z = p[(int64_t)b * GTILE];
-        re += z.re;
-        im += z.im;
+    part[w][threadIdx.x & 63] = cmake(re, im);
+    __syncthreads();
+    if (w || s0 >= s1) return;
+    for (int k = 1; k < 4; k++) {
+        re += part[k][threadIdx.x].re;
+        im += part[k][threadIdx.x].im;
     }
-    G[x] = cmake(re, im);
+    partial[s0 * entries + x] = cmake(re, im);
 }
 
-// entry (p1, p2) of the Hermitian Gram matrix held as the tiles of its upper
-// triangle (T tiles a side); a diagonal entry is real
-__device__ inline cplx gram_entry(const cplx *G, int T, int p1, int p2)
+// the segment sums of a Gram matrix held as the sub-blocks of its upper triangle
+struct GramSums {
+    const cplx *p;      // null: the matrix is zero
+    int64_t step;       // entries from one segment's sums to the next's
+    int nseg;
+    int T, ng;          // tiles a side, column groups of a tile
+};
+
+// entry (p1, p2) of the Hermitian Gram matrix; a diagonal entry is real
+__device__ inline cplx gram_entry(const GramSums &G, int p1, int p2)
 {
     const bool lower = p1 > p2;
     const int a = lower ? p2 : p1, b = lower ? p1 : p2;
-    const int TI = a / GT, TJ = b / GT;
-    const int tp = TI == TJ ? TI : T + off_index(TI, TJ, T);
-    const cplx z = G[(size_t)tp * GTILE + (a % GT) * GT + b % GT];
+    const int TI = a / GT, TJ = b / GT, I = a % GT / 16, J = b % GT / 16;
+    const int sb = gram_subblocks(G.ng, true);
+    const int at = TI == TJ ? TI * sb + I * G.ng - I * (I - 1) / 2 + (J - I)
+                            : G.T * sb + off_index(TI, TJ, G.T) * gram_subblocks(G.ng, false) + I * G.ng + J;
+    const cplx *p = G.p + (int64_t)at * 256 + (a % 16) * 16 + b % 16;
+    cplx y[GSEG];
+#pragma unroll
+    for (int s = 0; s < GSEG; s++) y[s] = s < G.nseg ? ldc(p + s * G.step) : cmake(0, 0);
+    cplx z = y[0];
+#pragma unroll
+    for (int s = 1; s < GSEG; s++) z = cadd(z, y[s]);
     if (a == b) return cmake(z.re, 0);
     return lower ? cmake(z.re, -z.im) : z;
 }
@@ -366,17 +519,33 @@ __device__ inline int pair_of(int x, int y)
     return hi * (hi + 1) / 2 + lo;
 }
 
-// rho1[k + M l] = G1(k, l) and rho2[a + bM + cM^2 + dM^3] = s2 * G2({a,b}, {c,d});
-// a null G gives zeros (fewer particles than annihilators)
-__global__ void k_gram_expand(int M, int T1, const cplx *__restrict__ G1, cplx *__restrict__ rho1, int T2,
-                              const cplx *__restrict__ G2, cplx *__restrict__ rho2, double s2)
+// rho1[k + M l] = G1(k, l), or with G2 at hand sum_s G2({k,s}, {s,l}) / (N -
+// 1) (the first blocks1 blocks, 32 lanes an entry, lane s the term of s); a
+// null matrix gives zeros (fewer particles than annihilators)
+// rho2[a + bM + cM^2 + dM^3] = s2 * G2({a,b}, {c,d}) (the other blocks)
+__global__ __launch_bounds__(256) void k_gram_expand(int N, int M, int blocks1, GramSums G1, cplx *__restrict__ rho1,
+                                                     GramSums G2, cplx *__restrict__ rho2, double s2)
 {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t M2 = (int64_t)M * M;
-    if (rho1 && x < M2) rho1[x] = G1 ? gram_entry(G1, T1, (int)(x % M), (int)(x / M)) : cmake(0, 0);
-    if (!rho2 || x >= M2 * M2) return;
+    if ((int)blockIdx.x < blocks1) {
+        const int x = blockIdx.x * 8 + threadIdx.x / 32, s = threadIdx.x % 32;
+        const int k = x % M, l = x / M;
+        cplx z = cmake(0, 0);
+        if (x < M2 && s < M) {
+            if (G2.p) z = gram_entry(G2, pair_of(k, s), pair_of(s, l));
+            else if (G1.p && s == 0) z = gram_entry(G1, k, l);
+        }
+        for (int o = 16; o > 0; o >>= 1) {
+            z.re += __shfl_xor(z.re, o, 64);
+            z.im += __shfl_xor(z.im, o, 64);
+        }
+        if (x < M2 && s == 0) rho1[x] = G2.p ? cmake(z.re / (N - 1), z.im / (N - 1)) : z;
+        return;
+    }
+    const int64_t x = (int64_t)(blockIdx.x - blocks1) * 256 + threadIdx.x;
+    if (x >= M2 * M2) return;
     const int a = (int)(x % M), b = (int)(x / M % M), c = (int)(x / M2 % M), d = (int)(x / (M2 * M));
-    rho2[x] = G2 ? cscale(gram_entry(G2, T2, pair_of(a, b), pair_of(c, d)), s2) : cmake(0, 0);
+    rho2[x] = G2.p ? cscale(gram_entry(G2, pair_of(a, b), pair_of(c, d)), s2) : cmake(0, 0);
 }
 
 }  // namespace
@@ -387,9 +556,7 @@ struct GramPlan {
     int U = GU2;         // rows of Phi per LDS tile
     int ntp = 0;         // tile pairs: ntile diagonal, then the off-diagonal ones
     int nblocks = 0;     // blocks per tile pair
-    size_t sm_diag = 0, sm_off = 0;
-    size_t partial_entries() const { return (size_t)ntp * nblocks * GTILE; }
-    size_t gram_entries() const { return (size_t)ntp * GTILE; }
+    size_t partial_entries() const { return (size_t)nblocks * a.entries; }
 };
 
 // plan Phi^H Phi for ord annihilators on basis b; nblocks at most max_blocks
@@ -402,34 +569,46 @@ static mcpi_status plan_gram(const BasisDev &b, int ord, int max_blocks, GramPla
     a.np = ord == 2 ? b.M * (b.M + 1) / 2 : b.M;
     a.ntile = (a.np + GT - 1) / GT;
     a.ng = std::min(GG, (a.np + 15) / 16);
-    a.rs = 16 * a.ng + 1;   // odd stride: the lanes of a gather write rows on distinct banks
     a.nc = b.nc;
     a.nu = b.N >= ord ? nc_of(b.N - ord, b.M) : 0;
     pl->U = ord == 2 ? GU2 : GU1;
     a.nut = (a.nu + pl->U - 1) / pl->U;
     a.B = b.B;
+    a.occ = ord == 2 ? b.occ2 : nullptr;
     a.C = nullptr;
     a.partial = nullptr;
-    pl->ntp = a.ntile * (a.ntile + 1) / 2;
+    const int noff = a.ntile * (a.ntile - 1) / 2;
+    pl->ntp = a.ntile + noff;
+    a.entries = 256 * ((int64_t)a.ntile * gram_subblocks(a.ng, true) + (int64_t)noff * gram_subblocks(a.ng, false));
     int dev = 0, ncu = 0;
     MCPI_HIP(hipGetDevice(&dev));
     MCPI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    // about three blocks per CU over all tile pairs, at most one per row tile
-    const int64_t want = std::max<int64_t>(1, (int64_t)3 * ncu / pl->ntp);
+    // two blocks per CU (their registers fill it) over all tile pairs, at most one per row tile
+    const int64_t want = std::max<int64_t>(1, (int64_t)2 * ncu / pl->ntp);
     pl->nblocks = (int)std::max<int64_t>(1, std::min<int64_t>({want, a.nut, (int64_t)max_blocks}));
-    pl->sm_diag = gram_lds(a.N, a.M, a.np, a.rs, true, pl->U, ord).bytes;
-    pl->sm_off = gram_lds(a.N, a.M, a.np, a.rs, false, pl->U, ord).bytes;
-    MCPI_ARG((a.ntile > 1 ? pl->sm_off : pl->sm_diag) <= 160 * 1024, "density-matrix tiles exceed LDS");
+    return MCPI_OK;
+}
+
+template <bool DIAG, int U, int NG, int OW>
+static mcpi_status launch_gram_k(const GramPlan &pl, int ny, hipStream_t s)
+{
+    const size_t sm =
+        gram_lds(pl.a.N, pl.a.M, pl.a.np, NG, DIAG, U, pl.a.ord, GramSplit<DIAG, NG>::red).bytes;
+    MCPI_ARG(sm <= 160 * 1024, "density-matrix tiles exceed LDS");
+    (void)hipFuncSetAttribute((const void *)k_gram<DIAG, U, NG, OW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
+    hipLaunchKernelGGL((k_gram<DIAG, U, NG, OW>), dim3(pl.nblocks, ny), dim3(GTHREADS), sm, s, pl.a);
+    MCPI_HIP(hipGetLastError());
     return MCPI_OK;
 }
 
 template <bool DIAG, int U, int NG>
-static mcpi_status launch_gram(const GramPlan &pl, int ny, size_t sm, hipStream_t s)
+static mcpi_status launch_gram(const GramPlan &pl, int ny, hipStream_t s)
 {
-    (void)hipFuncSetAttribute((const void *)k_gram<DIAG, U, NG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
-    hipLaunchKernelGGL((k_gram<DIAG, U, NG>), dim3(pl.nblocks, ny), dim3(GTHREADS), sm, s, pl.a);
-    MCPI_HIP(hipGetLastError());
-    return MCPI_OK;
+    if (U == GU2 && pl.a.occ) {
+        if (pl.a.M <= 16) return launch_gram_k<DIAG, U, NG, U == GU2 ? 4 : 0>(pl, ny, s);
+        return launch_gram_k<DIAG, U, NG, U == GU2 && NG == GG ? 8 : 0>(pl, ny, s);
+    }
+    return launch_gram_k<DIAG, U, NG, 0>(pl, ny, s);
 }
 
 // the block-partial kernels of a plan: rho1 (U = GU1, one tile of at most
@@ -439,35 +618,33 @@ static mcpi_status launch_gram_kernels(const GramPlan &pl, hipStream_t s)
     const int T = pl.a.ntile;
     if (pl.U == GU1) {
         MCPI_ARG(T == 1 && pl.a.ng <= 2, "one-body Gram matrix wider than two column groups");
-        return pl.a.ng == 1 ? launch_gram<true, GU1, 1>(pl, 1, pl.sm_diag, s)
-                            : launch_gram<true, GU1, 2>(pl, 1, pl.sm_diag, s);
+        return pl.a.ng == 1 ? launch_gram<true, GU1, 1>(pl, 1, s) : launch_gram<true, GU1, 2>(pl, 1, s);
     }
     switch (pl.a.ng) {
-    case 1: MCPI_CHECK((launch_gram<true, GU2, 1>(pl, T, pl.sm_diag, s))); break;
-    case 2: MCPI_CHECK((launch_gram<true, GU2, 2>(pl, T, pl.sm_diag, s))); break;
-    case 3: MCPI_CHECK((launch_gram<true, GU2, 3>(pl, T, pl.sm_diag, s))); break;
-    case 4: MCPI_CHECK((launch_gram<true, GU2, 4>(pl, T, pl.sm_diag, s))); break;
-    default: MCPI_CHECK((launch_gram<true, GU2, GG>(pl, T, pl.sm_diag, s))); break;
+    case 1: MCPI_CHECK((launch_gram<true, GU2, 1>(pl, T, s))); break;
+    case 2: MCPI_CHECK((launch_gram<true, GU2, 2>(pl, T, s))); break;
+    case 3: MCPI_CHECK((launch_gram<true, GU2, 3>(pl, T, s))); break;
+    case 4: MCPI_CHECK((launch_gram<true, GU2, 4>(pl, T, s))); break;
+    default: MCPI_CHECK((launch_gram<true, GU2, GG>(pl, T, s))); break;
     }
     // off-diagonal tile pairs exist only when the columns fill more than one tile
-    if (T > 1) MCPI_CHECK((launch_gram<false, GU2, GG>(pl, T * (T - 1) / 2, pl.sm_off, s)));
+    if (T > 1) MCPI_CHECK((launch_gram<false, GU2, GG>(pl, T * (T - 1) / 2, s)));
     return MCPI_OK;
 }
 
-// Phi^H Phi into G (pl.gram_entries()) through partial, on stream s
-static mcpi_status run_gram(GramPlan pl, const cplx *C, cplx *partial, cplx *G, hipStream_t s)
+// segment sums of Phi^H Phi in partial, on stream s
+static mcpi_status run_gram(GramPlan pl, const cplx *C, cplx *partial, GramSums *G, hipStream_t s)
 {
     pl.a.C = C;
     pl.a.partial = partial;
     MCPI_CHECK(launch_gram_kernels(pl, s));
-    const int64_t n = (int64_t)pl.ntp * GTILE;
     const int seg = (pl.nblocks + GSEG - 1) / GSEG, nseg = (pl.nblocks + seg - 1) / seg;
-    hipLaunchKernelGGL(k_gram_sum1, dim3((unsigned)((n + 255) / 256), (unsigned)nseg), dim3(256), 0, s, pl.ntp,
-                       pl.nblocks, seg, partial);
-    MCPI_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_gram_sum2, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, pl.ntp, pl.nblocks, seg,
-                       (const cplx *)partial, G);
-    MCPI_HIP(hipGetLastError());
+    if (seg > 1) {
+        hipLaunchKernelGGL(k_gram_sum1, dim3((unsigned)(pl.a.entries / 64), (unsigned)nseg), dim3(256), 0, s,
+                           pl.a.entries, pl.nblocks, seg, partial);
+        MCPI_HIP(hipGetLastError());
+    }
+    *G = GramSums{partial, (int64_t)seg * pl.a.entries, nseg, pl.a.ntile, pl.a.ng};
     return MCPI_OK;
 }
 
@@ -479,37 +656,26 @@ static mcpi_status densities_dev(const BasisDev &b, const cplx *C, bool want1, b
                                  double s2, cplx *ws, size_t ws_entries, size_t *need, hipStream_t s)
 {
     const int M = b.M;
-    GramPlan p1, p2;
-    const bool do1 = want1 && b.N >= 1, do2 = want2 && b.N >= 2;
-    int maxb = 1 << 20;
-    MCPI_CHECK(plan_gram(b, 1, maxb, &p1));
-    MCPI_CHECK(plan_gram(b, 2, maxb, &p2));
-    const size_t g1 = do1 ? p1.gram_entries() : 0, g2 = do2 ? p2.gram_entries() : 0;
-    auto partials = [&](const GramPlan &a, const GramPlan &c) {
-        return std::max(do1 ? a.partial_entries() : 0, do2 ? c.partial_entries() : 0);
-    };
+    // one product: rho2's where it exists (rho1 is its contraction), else rho1's
+    const bool do2 = want2 && b.N >= 2, do1 = want1 && b.N >= 1 && !do2;
+    GramPlan pl;
+    MCPI_CHECK(plan_gram(b, do2 ? 2 : 1, 1 << 20, &pl));
     if (!ws) {
-        *need = g1 + g2 + partials(p1, p2);
+        *need = do1 || do2 ? pl.partial_entries() : 1;
         return MCPI_OK;
     }
-    if (g1 + g2 + partials(p1, p2) > ws_entries) {
-        // fewer blocks: the partials take what the Gram tiles leave
-        MCPI_ARG(ws_entries > g1 + g2, "density workspace too small");
-        const size_t room = ws_entries - g1 - g2;
-        const size_t per1 = (size_t)p1.ntp * GTILE, per2 = (size_t)p2.ntp * GTILE;
-        const size_t per = std::max(do1 ? per1 : 0, do2 ? per2 : 0);
-        MCPI_ARG(per > 0 && room >= per, "density workspace too small");
-        maxb = (int)std::min<size_t>(room / per, 1 << 20);
-        MCPI_CHECK(plan_gram(b, 1, maxb, &p1));
-        MCPI_CHECK(plan_gram(b, 2, maxb, &p2));
+    GramSums none{}, G{};
+    if (do1 || do2) {
+        if (pl.partial_entries() > ws_entries) {
+            MCPI_ARG(ws_entries >= (size_t)pl.a.entries, "density workspace too small");
+            MCPI_CHECK(plan_gram(b, do2 ? 2 : 1, (int)(ws_entries / pl.a.entries), &pl));
+        }
+        MCPI_CHECK(run_gram(pl, C, ws, &G, s));
     }
-    cplx *G1 = ws, *G2 = ws + g1, *partial = ws + g1 + g2;
-    if (do1) MCPI_CHECK(run_gram(p1, C, partial, G1, s));
-    if (do2) MCPI_CHECK(run_gram(p2, C, partial, G2, s));
-    const int64_t M2 = (int64_t)M * M, n = want2 ? M2 * M2 : M2;
-    hipLaunchKernelGGL(k_gram_expand, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, M, p1.a.ntile,
-                       do1 ? (const cplx *)G1 : nullptr, want1 ? rho1 : nullptr, p2.a.ntile,
-                       do2 ? (const cplx *)G2 : nullptr, want2 ? rho2 : nullptr, s2);
+    const int64_t M2 = (int64_t)M * M;
+    const int blocks1 = want1 ? (int)((M2 + 7) / 8) : 0, blocks2 = want2 ? (int)((M2 * M2 + 255) / 256) : 0;
+    hipLaunchKernelGGL(k_gram_expand, dim3((unsigned)(blocks1 + blocks2)), dim3(256), 0, s, b.N, M, blocks1,
+                       do1 ? G : none, rho1, do2 ? G : none, rho2, s2);
     MCPI_HIP(hipGetLastError());
     return MCPI_OK;
 }
