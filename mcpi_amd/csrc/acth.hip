@@ -201,11 +201,34 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
             zoff = std::move(pf.zoff);
         }
     }
+    auto offsets = [](int x) {
+        const int l = pair_hi(x), q = x - l * (l + 1) / 2;
+        return PairOff{q * PAIR_ORB, l * PAIR_ORB, q == l ? PAIR_SLOT : 0, 0};
+    };
+    std::vector<PairRec> zrec;
+    for (size_t r = 0; r + 1 < zoff.size(); r++)
+        for (int j = zoff[r]; j < zoff[r + 1]; j++) {
+            const PairOff o = offsets(zord[j]);
+            zrec.push_back({zb[zord[j]].re, zb[zord[j]].im, o.oq, o.ol, o.e, j + 1 == zoff[r + 1]});
+        }
+    std::vector<PairRun> zrun;
+    if (!zoff.empty()) {
+        const int R = (int)zoff.size() - 1, n = zoff[R];
+        for (int g = 1; g <= PAIR_RUNS; g++)
+            for (int w = 0, r = 0; w <= 4 * g; w++) {
+                while (r < R && zoff[r] < n * w / (4 * g)) r++;
+                zrun.push_back({r, zoff[r]});
+            }
+    }
+    std::vector<PairOff> pql;
+    if (pair)
+        for (int x = 0; x < pair_count(M); x++) pql.push_back(offsets(x));
     // one device block: complex tables first (16-byte aligned), then integers
     size_t nC = dk.size() + d1.size() + d2.size() + A0.size() + A.size() + ot.size() + tt.size() + nz_c.size() +
                 otc.size() + ttc.size() + pw.size() + ph1.size() + za.size() + zb.size();
     size_t nB = nz1.size() + nzo.size() + nzt.size() + 4 * (m1j.size() + ot_off.size() + tt_off.size() +
-                                                           nz_e.size() + zblk.size() + zord.size() + zoff.size()) + 64;
+                                                           nz_e.size() + zblk.size() + zord.size() + zoff.size()) +
+                zrec.size() * sizeof(PairRec) + zrun.size() * sizeof(PairRun) + pql.size() * sizeof(PairOff) + 64;
     size_t bytes = (nC * sizeof(cplx) + nB + 64 + 255) & ~(size_t)255;
     char *dev = nullptr;
     MCPI_HIP(hipMalloc(&dev, bytes));
@@ -226,6 +249,9 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     const size_t o_ph1 = ph1.empty() ? 0 : put(ph1.data(), ph1.size() * sizeof(cplx));
     const size_t o_za = za.empty() ? 0 : put(za.data(), za.size() * sizeof(cplx));
     const size_t o_zb = zb.empty() ? 0 : put(zb.data(), zb.size() * sizeof(cplx));
+    const size_t o_zrec = zblk.empty() ? 0 : put(zrec.data(), zrec.size() * sizeof(PairRec));
+    const size_t o_zrun = zblk.empty() ? 0 : put(zrun.data(), zrun.size() * sizeof(PairRun));
+    const size_t o_pql = pql.empty() ? 0 : put(pql.data(), pql.size() * sizeof(PairOff));
     size_t o_m1 = put(m1j.data(), m1j.size() * 4);
     size_t o_oo = put(ot_off.data(), ot_off.size() * 4);
     size_t o_to = put(tt_off.data(), tt_off.size() * 4);
@@ -258,7 +284,10 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     c->pzblk = fac ? (int32_t *)(dev + o_zblk) : nullptr;
     c->pzord = fac ? (int32_t *)(dev + o_zord) : nullptr;
     c->pzoff = fac ? (int32_t *)(dev + o_zoff) : nullptr;
+    c->pzrec = fac ? (PairRec *)(dev + o_zrec) : nullptr;
+    c->pzrun = fac ? (PairRun *)(dev + o_zrun) : nullptr;
     c->pzR = fac ? (int)zoff.size() - 1 : 0;
+    c->pql = pair ? (PairOff *)(dev + o_pql) : nullptr;
     c->nz_1j = (uint8_t *)(dev + o_n1);
     c->nz_ot = (uint8_t *)(dev + o_no);
     c->nz_tt = (uint8_t *)(dev + o_nt);

@@ -96,20 +96,6 @@ __device__ inline cplx term(cplx coef, double x, cplx c, cplx acc)
     return acc;
 }
 
-// Hardware block b runs on XCD b % 8 as that XCD's (b / 8)-th block.  Chunks
-// of G consecutive row blocks dealt round-robin to the XCDs: each XCD gets
-// rows from the whole basis (the H.v work per row differs between regions
-// of the basis, so contiguous eighths leave XCDs idle at the end) while
-// neighbouring blocks still share an L2.  Blocks past the last full round
-// of chunks keep their index.
-__device__ inline unsigned chunk_xcd(unsigned b, unsigned n, unsigned G)
-{
-    const unsigned full = n / (8 * G) * (8 * G);
-    if (b >= full) return b;
-    const unsigned x = b % 8, k = b / 8;
-    return ((k / G) * 8 + x) * G + k % G;
-}
-
 // Per-row state kept in registers: the occupations packed 8 bits per orbital
 // (M <= 16) and sqrt(v + 1).  Everything else is derived on use (prefix
 // counts inside the rank tables, sqrt(v) and sqrt(v + 2) from the LDS table),

@@ -1,0 +1,997 @@
+// H.v through the pair space (schedules 6 and 7): every term of the
+// reference's operator (hamiltonianMatrix.h:1431-1970, the folded rules of
+// acth.hip), evaluated as two gathers around a pair-space step instead of
+// one gather per term.
+//
+// In pair form (build_coefficients) the operator is
+//   H = sum_{k,l} h1[k][l] a*_k a_l + sum_{P,Q} W[P][Q] a*_{P1} a*_{P2} a_{Q1} a_{Q2}
+// over unordered orbital pairs.  On N >= 2 particles the one-body part is a
+// pair term too (a*_k a_l = sum_s a*_k a*_s a_s a_l / (N - 1)).  Inserting
+// the identity over the basis with N-2 particles after the creators,
+//   (H C)(v) = sum_P <v|a*_{P1} a*_{P2}|u> Y2_u(P),  u = v - e_{P1} - e_{P2}
+//   Y2_u(P)  = sum_Q W[P][Q] X[Q][u],  X[Q][u] = <u|a_{Q1} a_{Q2}|C>
+// and <u|a_q a_l|C> = sqrt((u_q + 1)(u_l + 1 + [q = l])) C[rank(u + e_q + e_l)]
+// is the pair amplitude of the densities' Gram matrix (rho.hip).  At N = M =
+// 12 a row has up to 1,636 double-jump terms; here it costs 78 output
+// gathers, and the 352,716 rows of 10 particles cost 78 gathers and a 78 x
+// 78 complex matrix-vector product each, on the FP64 MFMA (schedule 6).
+// When W is block diagonal with rank-one blocks, W = a b^T on each block r
+// (a contact interaction that conserves a pair charge), and h1 is diagonal,
+// Y2_u(P) = a[P] Z[r(P)][u] with Z[r][u] = sum_{Q in r} b[Q] X[Q][u]: one
+// sum per block and no product (schedule 7).
+//
+// k_pair_amp<M>: X, gathered.  k_pair_mul<M>: Y2 = W X on the MFMA.
+// k_pairz_amp<>: Z, gathered and summed per block.
+// k_pair_out<M, FAC>: one thread per row v of the basis ranks the v - e_P
+// in the smaller basis from its prefix-count tables and sums the factors
+// times Y2 (or a[P] Z).  k_pair_y1<M, U>: for N = 1 only, the one-body
+// part over the empty basis of N - 1 particles.  Y2, Z and X are stored
+// column-major (Y[col * ld + u]) so that every pass reads and writes them
+// coalesced.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+#include "mcpi_internal.h"
+
+namespace mcpi {
+
+namespace {
+
+constexpr int PT = 256;   // threads per block
+
+struct PairArgs {
+    int N;                // particles of the basis
+    int64_t nc;           // its states
+    int64_t nu;           // states of the basis with N - 2 (or N - 1) particles
+    int64_t nut;          // tiles of U rows
+    const int32_t *B;     // rank table B[j*(N+1) + p]
+    const cplx *C;
+    const cplx *W;        // pair matrix pw[Q * PWS + P], or h1 as ph1[l * 16 + k] (M <= 12)
+    cplx *Y;              // Y[col * ld + u]
+    int64_t ld;           // row stride of Y (and of the pair amplitudes X), >= nu
+    const cplx *H1;       // pair product: h1 (ph1[l * 16 + k]) folded into W with weight h1s
+    double h1s;           // 1 / (N - 1), or 0
+    const uint8_t *occ;   // occupations of the N - 2 particle states (BasisDev::occ2)
+    const PairOff *ql;    // pairs: their places in the row tables
+    const PairRec *rec;   // factorized form: pairs block by block
+    const PairRun *run;   // 4 gridDim.y runs of blocks
+    int zR;               // blocks
+    unsigned G;           // tiles dealt to an XCD in one piece
+    int64_t mC, mY;       // factorized form, several members: entries between
+                          // the members' C vectors and between their Z tables
+};
+
+__device__ inline cplx ldcp(const cplx *p)
+{
+    double2 t = *reinterpret_cast<const double2 *>(p);
+    return cmake(t.x, t.y);
+}
+
+// 16-byte load at byte offset off of the buffer [p, p + bytes) (bytes <
+// 2^31); an offset at or past the end reads zero without a memory access
+__device__ inline cplx ldbuf(const cplx *p, int bytes, uint32_t off)
+{
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, bytes, 0x00020000);
+    const v4u w = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    return cmake(__builtin_bit_cast(double, (unsigned long long)w.x | ((unsigned long long)w.y << 32)),
+                 __builtin_bit_cast(double, (unsigned long long)w.z | ((unsigned long long)w.w << 32)));
+}
+
+template <int M, int U>
+struct PairLds {
+    static constexpr int RS = M + 1;   // LDS row stride of the tile (odd)
+    static size_t bytes(int N)
+    {
+        size_t o = sizeof(cplx) * ((size_t)M * 16 + (size_t)U * RS);
+        o += sizeof(int64_t) * ((size_t)U + (size_t)U * M);
+        o += sizeof(double) * (N + 3) + sizeof(int32_t) * M * (N + 1) + (size_t)U * (M + 1);
+        return (o + 15) / 16 * 16;
+    }
+};
+
+// Y1[k][u] = sum_l h1[k][l] <u|a_l|C> over the basis with N-1 particles
+template <int M, int U>
+__global__ __launch_bounds__(PT) void k_pair_y1(PairArgs a)
+{
+    using L = PairLds<M, U>;
+    constexpr int RS = L::RS, UR = U / 16;
+    extern __shared__ __align__(16) unsigned char lds[];
+    cplx *Wl = (cplx *)lds;                                   // [M][16]: h1[k][l] at l * 16 + k
+    cplx *phi = Wl + M * 16;                                   // [U][RS]
+    int64_t *tt = (int64_t *)(phi + U * RS);                  // [U]
+    int64_t *dq = tt + U;                                      // [U][M]
+    double *sq = (double *)(dq + U * M);                       // [N + 3]
+    int32_t *Bt = (int32_t *)(sq + a.N + 3);                   // [M][N + 1]
+    uint8_t *pp = (uint8_t *)(Bt + M * (a.N + 1));            // [U][M + 1]
+
+    const int t = threadIdx.x;
+    const int N = a.N, NB = N + 1, Np = N - 1;
+    for (int x = t; x < M * 16; x += PT) Wl[x] = ldcp(a.W + x);
+    for (int x = t; x < M * NB; x += PT) Bt[x] = a.B[x];
+    for (int x = t; x < N + 3; x += PT) sq[x] = sqrt((double)x);
+    const int pg = t & 15, ug = t >> 4;
+
+    for (int64_t tile = blockIdx.x; tile < a.nut; tile += gridDim.x) {
+        __syncthreads();   // the previous tile's product has read phi and the row tables
+        const int64_t u0 = tile * U;
+        if (t < U) {
+            const int64_t u = u0 + t;
+            uint8_t *P = pp + t * (M + 1);
+            if (u < a.nu) {
+                // greedy unranking, one step per iteration (lanes stay together)
+                int64_t R = a.nu - 1 - u;
+                int pj = Np, j = M - 1;
+                P[M] = (uint8_t)Np;
+                while (j >= 1) {
+                    const int64_t bj = Bt[j * NB + pj];
+                    if (bj > R) {
+                        pj--;
+                    } else {
+                        P[j] = (uint8_t)pj;
+                        R -= bj;
+                        j--;
+                    }
+                }
+                P[0] = 0;
+                int64_t s0 = 0, s1 = 0;
+                int64_t *Dq = dq + t * M;
+                Dq[0] = 0;
+                for (int j2 = 1; j2 < M; j2++) {
+                    const int b = j2 * NB + P[j2];
+                    s0 += Bt[b];
+                    s1 += Bt[b + 1];
+                    Dq[j2] = s0 - s1;
+                }
+                tt[t] = a.nc - 1 - s1;
+            } else {
+                tt[t] = -1;
+            }
+        }
+        __syncthreads();
+        // amplitudes of the tile: lanes over consecutive rows of one column,
+        // five loads in flight per thread
+        constexpr int NE = U * M, GBP = 5;
+        for (int e0 = t; e0 < NE; e0 += GBP * PT) {
+            int64_t tg[GBP];
+            double f[GBP];
+#pragma unroll
+            for (int k = 0; k < GBP; k++) {
+                const int e = e0 + k * PT;
+                const int col = e / U, ul = e % U;
+                const int64_t base = e < NE ? tt[ul] : -1;
+                tg[k] = -1;
+                f[k] = 0;
+                if (base >= 0) {
+                    const uint8_t *P = pp + ul * (M + 1);
+                    tg[k] = base - dq[ul * M + col];
+                    f[k] = sq[P[col + 1] - P[col] + 1];
+                }
+            }
+            cplx v[GBP];
+#pragma unroll
+            for (int k = 0; k < GBP; k++) v[k] = tg[k] >= 0 ? ldcp(a.C + tg[k]) : cmake(0, 0);
+#pragma unroll
+            for (int k = 0; k < GBP; k++) {
+                const int e = e0 + k * PT;
+                if (e < NE) phi[(e % U) * RS + e / U] = cscale(v[k], f[k]);
+            }
+        }
+        __syncthreads();
+        // thread (pg, ug) forms column pg (an orbital k < M) of the rows
+        // ug + 16 j
+        cplx acc[UR];
+#pragma unroll
+        for (int j = 0; j < UR; j++) acc[j] = cmake(0, 0);
+#pragma unroll 2
+        for (int l = 0; l < M; l++) {
+            const cplx w = Wl[l * 16 + pg];
+            cplx x[UR];
+#pragma unroll
+            for (int j = 0; j < UR; j++) x[j] = phi[(ug + 16 * j) * RS + l];
+#pragma unroll
+            for (int j = 0; j < UR; j++) acc[j] = cfma(w, x[j], acc[j]);
+        }
+        if (pg < M) {
+#pragma unroll
+            for (int j = 0; j < UR; j++) {
+                const int64_t u = u0 + ug + 16 * j;
+                if (u < a.nu) {
+                    double2 o;
+                    o.x = acc[j].re;
+                    o.y = acc[j].im;
+                    *reinterpret_cast<double2 *>(a.Y + (int64_t)pg * a.ld + u) = o;
+                }
+            }
+        }
+    }
+}
+
+// Row tables of a tile of PAIR_U states u of N - 2 particles in LDS, PAIR_ORB
+// bytes per orbital o: the differences of the rank sums for o the lower (dq)
+// and the higher (dl) orbital of a pair, sqrt(u_o + 1), and sqrt(u_o + 2) for
+// the pairs q = l.  A pair and row take two differences and two roots, at
+// offsets that depend on the pair alone (PairOff): four LDS reads.
+constexpr int PAIR_DL = 4, PAIR_G = PAIR_SLOT;   // of an orbital's entries: dl, the roots
+
+static size_t pair_amp_lds(int N, int M)
+{
+    const size_t o = (size_t)PAIR_ORB * M + sizeof(double) * (N + 3) + sizeof(int32_t) * (PAIR_U + M * (N + 1));
+    return (o + 15) / 16 * 16;
+}
+
+// tables the launches pass are read through constant pointers: uniform
+// indices then give scalar loads although the kernels write memory
+template <class T>
+__device__ inline const __attribute__((address_space(4))) T *kptr(const T *p)
+{
+    return (const __attribute__((address_space(4))) T *)p;
+}
+
+// The tables of a row with occupations w (NW words of bytes, orbital 0 first)
+// at tab; returns rank(u + 2 e_0).  Four orbitals' entries are in flight
+// together.
+template <int NW>
+__device__ inline int32_t pair_rows(const uint32_t (&w)[NW], int M, int NB1, int32_t top, const int32_t *Bt,
+                                    const double *sq, unsigned char *tab)
+{
+    int p = 0;
+    int32_t s01 = 0, s12 = 0, s2 = 0;
+#pragma unroll
+    for (int k = 0; k < NW; k++) {
+        if (4 * k >= M) continue;
+        int32_t b0[4], b1[4], b2[4];
+        double g[4], g2[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            // (orbitals past M - 1 read its entry again and are not stored)
+            const int o = 4 * k + j, b = (o < M ? o : M - 1) * NB1 + p;
+            const int v = (int)((w[k] >> (8 * j)) & 255u);
+            b0[j] = Bt[b];
+            b1[j] = Bt[b + 1];
+            b2[j] = Bt[b + 2];
+            g[j] = sq[v + 1];
+            g2[j] = sq[v + 2];
+            p += v;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int o = 4 * k + j;
+            if (o >= M) continue;
+            if (o) {
+                s01 += b0[j] - b1[j];
+                s12 += b1[j] - b2[j];
+                s2 += b2[j];
+            }
+            unsigned char *t = tab + o * PAIR_ORB;
+            *(int2 *)t = make_int2(s01, s12);
+            *(double *)(t + PAIR_G) = g[j];
+            *(double *)(t + PAIR_G + PAIR_SLOT) = g2[j];
+        }
+    }
+    return top - s2;
+}
+
+// target of a pair and row (tab: the row's entries) and its amplitude's factor
+__device__ inline uint32_t pair_target(const unsigned char *tab, int oq, int ol, int e, int32_t base, double &f)
+{
+    f = *(const double *)(tab + oq + PAIR_G) * *(const double *)(tab + ol + e + PAIR_G);
+    return (uint32_t)(base - *(const int32_t *)(tab + oq) - *(const int32_t *)(tab + ol + PAIR_DL));
+}
+
+// Z[r][u] = sum_{Q in block r} zb[Q] <u|a_{Q1} a_{Q2}|C> of the factorized pair
+// form; Z has R rows of ld entries.  MV > 1: the same for MV members that share
+// zb and the blocks, their C vectors mC and their Z tables mY entries apart
+// (the row tables and the targets are shared); grid row z serves members z MV
+// .. z MV + MV - 1.  RC: zb is real.
+//
+// A block tabulates 64 rows from the occupation table (one wavefront) and its
+// four wavefronts share the list of pairs (a.rec, block by block), cut at block
+// borders into 4 gridDim.y runs of about the same length (a.run): with few rows
+// gridDim.y > 1 gives every CU something to do.  A wavefront walks its run in
+// batches of BT pairs whose loads are in flight together, across the borders
+// of the blocks r.  Per pair and row: four LDS reads, two differences, one
+// gather.  What bounds it is the L2: neighbouring tiles gather from
+// neighbouring parts of C, so chunks of them go to one XCD each.
+// Measured (before: rows unranked in the kernel, two pairs in flight, tiles
+// dealt out one by one): N = 12, M = 12 88 -> 44 us; N = 16, M = 12 1220 -> 730
+// us (chunks of 128 tiles; single tiles 820); 24 members of N = 10, M = 13, four
+// at a time, 688 -> 567 us (chunks of 32 tiles, whose part of four C vectors an
+// L2 holds; 128: 770 with batches of four); N = 5, M = 21 60 -> 6 us (eleven
+// runs of 28 tiles).
+template <int NW, int MV, bool RC>
+__global__ __launch_bounds__(PT) void k_pairz_amp(PairArgs a, int M)
+{
+    constexpr int U = PAIR_U, BT = 8;
+
+    extern __shared__ __align__(16) unsigned char lds[];
+    double *sq = (double *)(lds + PAIR_ORB * M);               // [N + 3]
+    int32_t *tt = (int32_t *)(sq + a.N + 3);                   // [U]
+    int32_t *Bt = tt + U;                                      // [M][N + 1]
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int N = a.N, NB1 = N + 1;
+    const int64_t m0 = MV > 1 ? (int64_t)blockIdx.z * MV : 0;   // first member of this grid row
+    // one tile a block; its occupations' load goes first
+    const int64_t u = (int64_t)chunk_xcd(blockIdx.x, gridDim.x, a.G) * U + lane;
+    uint32_t w[NW];
+    if (wave == 0) {
+        const uint4 *o = reinterpret_cast<const uint4 *>(a.occ + (u < a.nu ? u : a.nu - 1) * (4 * NW));
+#pragma unroll
+        for (int k = 0; k < NW / 4; k++) {
+            const uint4 x = o[k];
+            w[4 * k] = x.x;
+            w[4 * k + 1] = x.y;
+            w[4 * k + 2] = x.z;
+            w[4 * k + 3] = x.w;
+        }
+    }
+    // this wavefront's run of blocks
+    const auto rec = kptr(a.rec);
+    const auto run = kptr(a.run) + 4 * blockIdx.y + wave;
+    const int r0 = run[0].r, j0 = run[0].j, j1 = run[1].j;
+    for (int x = t; x < M * NB1; x += PT) Bt[x] = a.B[x];
+    for (int x = t; x < N + 3; x += PT) sq[x] = sqrt((double)x);
+    unsigned char *tab = lds + 8 * lane;
+    __syncthreads();
+    if (wave == 0) tt[lane] = pair_rows<NW>(w, M, NB1, (int32_t)(a.nc - 1), Bt, sq, tab);
+    __syncthreads();
+    {
+        const int32_t base = tt[lane];
+        cplx acc[MV];
+#pragma unroll
+        for (int m = 0; m < MV; m++) acc[m] = cmake(0, 0);
+        int r = r0;
+        // B pairs from j on (past the run's end its last pair again, unused)
+        auto batch = [&](auto size, int j) {
+            constexpr int B = decltype(size)::value;
+            double f[B];
+            cplx v[MV][B];
+#pragma unroll
+            for (int k = 0; k < B; k++) {
+                const auto &x = rec[j + k < j1 ? j + k : j1 - 1];
+                const uint32_t tg = pair_target(tab, x.oq, x.ol, x.e, base, f[k]);
+#pragma unroll
+                for (int m = 0; m < MV; m++) v[m][k] = ldcp(a.C + (m0 + m) * a.mC + tg);
+            }
+#pragma unroll
+            for (int k = 0; k < B; k++) {
+                if (j + k >= j1) continue;
+                const auto &x = rec[j + k];
+#pragma unroll
+                for (int m = 0; m < MV; m++) {
+                    if (RC) {
+                        acc[m].re = fma(x.br * f[k], v[m][k].re, acc[m].re);
+                        acc[m].im = fma(x.br * f[k], v[m][k].im, acc[m].im);
+                    } else {
+                        acc[m] = cfma(cscale(cmake(x.br, x.bi), f[k]), v[m][k], acc[m]);
+                    }
+                }
+                if (x.last) {
+                    if (u < a.nu) {
+#pragma unroll
+                        for (int m = 0; m < MV; m++) {
+                            double2 o;
+                            o.x = acc[m].re;
+                            o.y = acc[m].im;
+                            *reinterpret_cast<double2 *>(a.Y + (m0 + m) * a.mY + (int64_t)r * a.ld + u) = o;
+                        }
+                    }
+#pragma unroll
+                    for (int m = 0; m < MV; m++) acc[m] = cmake(0, 0);
+                    r++;
+                }
+            }
+        };
+        int j = j0;
+        for (; j + BT <= j1; j += BT) batch(std::integral_constant<int, BT>(), j);
+#pragma clang loop unroll(disable)
+        for (; j < j1; j += 2) batch(std::integral_constant<int, 2>(), j);
+    }
+}
+
+// The pair amplitudes X[Q][u] = <u|a_{Q1} a_{Q2}|C> of the basis with N-2
+// particles, column-major (X[Q * ld + u]): the row tables as above, lanes over
+// the rows of one column at a time (neighbouring targets, coalesced stores),
+// GBP loads in flight per thread.
+template <int M>
+__global__ __launch_bounds__(PT) void k_pair_amp(PairArgs a)
+{
+    constexpr int NP = pair_count(M), U = PAIR_U;
+    static_assert(M <= 16, "16-byte rows");
+    extern __shared__ __align__(16) unsigned char lds[];
+    double *sq = (double *)(lds + PAIR_ORB * M);               // [N + 3]
+    int32_t *tt = (int32_t *)(sq + a.N + 3);                   // [U]
+    int32_t *Bt = tt + U;                                      // [M][N + 1]
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int N = a.N, NB1 = N + 1;
+    const auto ql = kptr(a.ql);
+    for (int x = t; x < M * NB1; x += PT) Bt[x] = a.B[x];
+    for (int x = t; x < N + 3; x += PT) sq[x] = sqrt((double)x);
+    unsigned char *tab = lds + 8 * lane;
+    for (int64_t tile = blockIdx.x; tile < a.nut; tile += gridDim.x) {
+        __syncthreads();
+        const int64_t u = tile * U + lane;
+        if (wave == 0) {
+            const uint4 x = *reinterpret_cast<const uint4 *>(a.occ + (u < a.nu ? u : a.nu - 1) * 16);
+            const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+            tt[lane] = pair_rows<4>(w, M, NB1, (int32_t)(a.nc - 1), Bt, sq, tab);
+        }
+        __syncthreads();
+        const int32_t base = tt[lane];
+        constexpr int GBP = 5;
+#pragma clang loop unroll(disable)
+        for (int p0 = wave; p0 < NP; p0 += 4 * GBP) {
+            double f[GBP];
+            cplx v[GBP];
+#pragma unroll
+            for (int k = 0; k < GBP; k++) {
+                const auto &x = ql[p0 + 4 * k < NP ? p0 + 4 * k : NP - 1];
+                v[k] = ldcp(a.C + pair_target(tab, x.oq, x.ol, x.e, base, f[k]));
+            }
+#pragma unroll
+            for (int k = 0; k < GBP; k++) {
+                const int p = p0 + 4 * k;
+                if (p >= NP || u >= a.nu) continue;
+                const cplx z = cscale(v[k], f[k]);
+                double2 o;
+                o.x = z.re;
+                o.y = z.im;
+                *reinterpret_cast<double2 *>(a.Y + (int64_t)p * a.ld + u) = o;
+            }
+        }
+    }
+}
+
+// Y2 = W X through FP64 MFMA (v_mfma_f64_16x16x4f64: lane i + 16k holds
+// A[i][k] and B[k][i]; the result D[g + 4r][j] sits in register r of lane
+// j + 16g), three real products per complex one (Gauss): T1 = (Xr + Xi)
+// Wr, T2 = Xr (Wi - Wr), T3 = Xi (Wr + Wi), then Re = T1 - T3 and Im = T1 +
+// T2.  The block stages W once in LDS as B fragments in the order the lanes
+// read them: Wa[s][g][lane] = (Wr, Wi - Wr) and Wb[s][g][lane] = Wr + Wi of
+// W[4s + k][16g + j], KS = ceil(NP/4) steps of four Q times NG groups of
+// 16 pair columns P, zero past NP; conflict-free reads.
+// Each wavefront takes 16-row blocks of X on its own and keeps the 16 x NP
+// result block in accumulators: per step one A fragment (four Q rows of 16
+// consecutive u, coalesced; loaded four steps ahead, across row blocks)
+// meets the NG fragments of W, three MFMAs each.
+typedef double mcpi_v4d __attribute__((ext_vector_type(4)));
+
+constexpr int PAIR_MUL_WAVES = 8;
+
+// The one-body operator in pair form: on states of N >= 2 particles
+//   a*_k a_l = (1 / (N - 1)) sum_s a*_k a*_s a_s a_l
+// (the number operator is N - 1 on a_l |v>), so h1 adds
+// h1[k][l] / (N - 1) to W[{k, s}][{s, l}] for every s.  This is the sum of
+// h1[k][l] over the orderings (k, s) of the pair P and (s, l) of the pair Q
+// that share s.
+__device__ inline cplx h1_pair(const cplx *h1, int P, int Q)
+{
+    const int p2 = pair_hi(P), p1 = P - p2 * (p2 + 1) / 2;
+    const int q2 = pair_hi(Q), q1 = Q - q2 * (q2 + 1) / 2;
+    cplx z = cmake(0, 0);
+    for (int o = 0; o < (p1 == p2 ? 1 : 2); o++) {
+        const int k = o ? p1 : p2, s = o ? p2 : p1;
+        for (int o2 = 0; o2 < (q1 == q2 ? 1 : 2); o2++) {
+            const int s2 = o2 ? q2 : q1, l = o2 ? q1 : q2;
+            if (s2 == s) z = cadd(z, ldcp(h1 + l * 16 + k));
+        }
+    }
+    return z;
+}
+
+template <int M>
+struct PairMulLds {
+    static constexpr int NP = pair_count(M), KS = (NP + 3) / 4, NG = (NP + 15) / 16;
+    static constexpr size_t bytes = (sizeof(double2) + sizeof(double)) * NG * KS * 64;
+};
+
+template <int M>
+__global__ __launch_bounds__(64 * PAIR_MUL_WAVES) void k_pair_mul(PairArgs a, const cplx *X)
+{
+    using L = PairMulLds<M>;
+    constexpr int NP = L::NP, KS = L::KS, NG = L::NG, PWS = pair_stride(M);
+    extern __shared__ __align__(16) unsigned char lds[];
+    double2 *wa = (double2 *)lds;                 // [KS][NG][64]
+    double *wb = (double *)(wa + NG * KS * 64);   // [KS][NG][64]
+    for (int x = threadIdx.x; x < NG * KS * 64; x += blockDim.x) {
+        const int s = x / (NG * 64), g = (x / 64) % NG, ln = x % 64;
+        const int P = 16 * g + (ln & 15), Q = 4 * s + (ln >> 4);
+        double2 v = {0, 0};
+        double vb = 0;
+        if (P < NP && Q < NP) {
+            cplx w = ldcp(a.W + (int64_t)Q * PWS + P);
+            if (a.h1s != 0.0) {
+                const cplx h = h1_pair(a.H1, P, Q);
+                w.re = fma(a.h1s, h.re, w.re);
+                w.im = fma(a.h1s, h.im, w.im);
+            }
+            v.x = w.re;
+            v.y = w.im - w.re;
+            vb = w.re + w.im;
+        }
+        wa[x] = v;
+        wb[x] = vb;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int jl = lane & 15, kl = lane >> 4;
+    const int64_t nrb = (a.nu + 15) / 16, stride = (int64_t)gridDim.x * PAIR_MUL_WAVES;
+    // (the launch gives ld >= 16 nrb)
+    // A fragments: lane (j, k) of step s of row block rb reads X[4s + k][16
+    // rb + j].  X has 4 KS rows of ld >= 16 nrb entries, zero past NP rows
+    // and nu columns, and Y has 16 NG rows of ld entries, so that neither
+    // loads nor stores need a bound; a block past the last is read as the
+    // last.
+    const int64_t rowstep = 4 * a.ld;
+    auto lanep = [&](int64_t rb) { return X + (int64_t)kl * a.ld + (rb < nrb ? rb : nrb - 1) * 16 + jl; };
+    // They are loaded four steps before their use, across row blocks: the
+    // steps of a block are counted up to KS4 = KS rounded up to four (the
+    // steps past KS load step KS - 1 again and skip their MFMAs), so that
+    // step t of the ring always sits in register t % 4.
+    constexpr int KS4 = (KS + 3) & ~3;
+    auto ldx = [&](const cplx *p, int s) { return ldcp(p + (int64_t)(s < KS ? s : KS - 1) * rowstep); };
+    int64_t rb = (int64_t)blockIdx.x * PAIR_MUL_WAVES + wave;
+    const cplx *pc = lanep(rb);
+    cplx x0 = ldx(pc, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    cplx x1 = ldx(pc, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    cplx x2 = ldx(pc, 2);
+    __builtin_amdgcn_sched_barrier(0);
+    cplx x3 = ldx(pc, 3);
+    __builtin_amdgcn_sched_barrier(0);
+    // one row block: KS4 steps in straight-line code, then the stores
+    auto block = [&](int64_t rb, const cplx *pn) {
+        auto ldnext = [&](int t) { return t < KS4 ? ldx(pc, t) : ldx(pn, t - KS4); };
+        mcpi_v4d acc[3 * NG];
+#pragma unroll
+        for (int g = 0; g < 3 * NG; g++) acc[g] = mcpi_v4d{0, 0, 0, 0};
+        auto step = [&](int s, const cplx xc) {
+            if (s >= KS) return;
+            const double xs = xc.re + xc.im;
+#pragma unroll
+            for (int g = 0; g < NG; g++) {
+                const double2 w = wa[(s * NG + g) * 64 + lane];
+                const double w3 = wb[(s * NG + g) * 64 + lane];
+                acc[3 * g] = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, w.x, acc[3 * g], 0, 0, 0);
+                acc[3 * g + 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(xc.re, w.y, acc[3 * g + 1], 0, 0, 0);
+                acc[3 * g + 2] = __builtin_amdgcn_mfma_f64_16x16x4f64(xc.im, w3, acc[3 * g + 2], 0, 0, 0);
+            }
+            // LDS reads of one group ahead of its three MFMAs, in turn
+#pragma unroll
+            for (int g = 0; g < NG; g++) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+            }
+        };
+#pragma unroll
+        for (int s = 0; s < KS4; s += 4) {
+            step(s, x0);
+            __builtin_amdgcn_sched_barrier(0);
+            x0 = ldnext(s + 4);
+            step(s + 1, x1);
+            __builtin_amdgcn_sched_barrier(0);
+            x1 = ldnext(s + 5);
+            step(s + 2, x2);
+            __builtin_amdgcn_sched_barrier(0);
+            x2 = ldnext(s + 6);
+            step(s + 3, x3);
+            __builtin_amdgcn_sched_barrier(0);
+            x3 = ldnext(s + 7);
+        }
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+            cplx *y = a.Y + (int64_t)(16 * g + jl) * a.ld + rb * 16 + kl;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                double2 o;
+                o.x = acc[3 * g][r] - acc[3 * g + 2][r];
+                o.y = acc[3 * g][r] + acc[3 * g + 1][r];
+                *reinterpret_cast<double2 *>(y + 4 * r) = o;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // The first block is peeled, so that the loop is entered with the
+    // stores of a block in flight as on every later pass: the first steps of
+    // a block then wait only for their own fragments (loaded before those
+    // stores), not for the stores to complete.
+    if (rb < nrb) {
+        const cplx *pn = lanep(rb + stride);
+        block(rb, pn);
+        pc = pn;
+        for (rb += stride; rb < nrb; rb += stride) {
+            pn = lanep(rb + stride);
+            block(rb, pn);
+            pc = pn;
+        }
+    }
+}
+
+// out[v] = sum_k sqrt(v_k) Y1[k][rank'(v - e_k)] + sum_P f_P(v) Y2[P][rank''(v - e_P)];
+// FAC (factorized pair form, Y2 = Z with one row per block):
+// out[v] = (sum_k h1[k][k] v_k) C[v] + sum_P f_P(v) za[P] Z[zblk[P]][rank''(v - e_P)]
+// RC (FAC only): za is real.  MV > 1 (FAC only): MV members that share the
+// basis, zb and the blocks (a group of Lieb-Liniger couplings): the row's
+// occupations, prefix sums, pair offsets and factors serve every member;
+// member m reads its C, Z, za and h1 at C + m mC, Z + m mZ and (bytes) za + m
+// mK, h1 + m mK, and writes out + m mC; grid row y serves members y MV .. y MV
+// + MV - 1.
+//
+// One thread per row.  The lanes of a wavefront are consecutive rows, which
+// share the occupations of all but the first few orbitals, so an orbital that
+// is empty in one of them is mostly empty in all: the pairs of a higher orbital
+// c2 are passed over by the wavefront as a whole where no row has c2 (a load
+// takes the vector memory pipeline the same time whether one lane or 64 take
+// part; at N = 16, M = 12 about 50 of 78 loads remain).  Testing c1 too (42
+// loads) costs as much in branches as it saves.  Where an orbital is empty in
+// some lanes only, their offset lies past the column, which the buffer's range
+// check turns into a zero without a memory access: no branch between the
+// loads of a batch.  Occupations stay packed, a byte each, and the roots in
+// LDS: registers are wavefronts, which hide the gathers.  Measured (before: all
+// pairs, in batches of 13): N = 12, M = 12 88 -> 71 us, N = 16, M = 12 970 -> 830
+// us (then bound by the 5.9 GB that the L2s miss), 24 members of N = 10, M = 13,
+// four at a time, 918 -> 705 us.
+struct PairOutArgs {
+    int N;
+    int64_t nc;
+    const int32_t *IF, *B;
+    int64_t nu1, nu2, ld2;
+    const cplx *Y1, *Y2, *za;
+    const int32_t *zblk;
+    const cplx *h1, *C;
+    cplx *out;
+    int64_t mC, mZ, mK;
+};
+
+template <int M, bool FAC, bool RC, int MV>
+__global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
+{
+    static_assert(FAC || (MV == 1 && !RC), "several members: factorized form only");
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int N = a.N;
+    double *sq = (double *)lds;                      // [N + 3]
+    int32_t *Bt = (int32_t *)(sq + N + 3);          // [M][N + 1]
+    const int NB = N + 1;
+    for (int x = threadIdx.x; x < N + 3; x += PT) sq[x] = sqrt((double)x);
+    for (int x = threadIdx.x; x < M * NB; x += PT) Bt[x] = a.B[x];
+    __syncthreads();
+    const int64_t i = (int64_t)blockIdx.x * PT + threadIdx.x;
+    if (i >= a.nc) return;
+    const int64_t m0 = MV > 1 ? (int64_t)blockIdx.y * MV : 0;   // this grid row's first member
+    const cplx *C = a.C + m0 * a.mC, *Z = a.Y2 + m0 * a.mZ;
+    // the coefficients' uniform indices give scalar loads
+    typedef const __attribute__((address_space(4))) char *kchar;
+    typedef const __attribute__((address_space(4))) cplx *kcplx;
+    const kchar za = (kchar)((const char *)a.za + m0 * a.mK), h1 = (kchar)((const char *)a.h1 + m0 * a.mK);
+    const auto zblk = kptr(a.zblk);
+    // occupations, a byte each (v(k)): the registers go to the gathers
+    uint64_t pk[(M + 7) / 8];
+#pragma unroll
+    for (int k = 0; k < (M + 7) / 8; k++) pk[k] = 0;
+#pragma unroll
+    for (int k = 0; k < M; k++) pk[k / 8] |= (uint64_t)a.IF[i * M + k] << (8 * (k % 8));
+    auto v = [&](int k) { return (int)((uint32_t)(pk[k / 8] >> (8 * (k % 8))) & 255u); };
+    // D1[o] = S_0(o) - S_1(o), D2[o] = S_1(o) - S_2(o) of S_d(x) = sum_{j=1..x}
+    // B[j][P_j - d] (P_j: particles below orbital j), modulo 2^32 (every rank
+    // is below 2^31)
+    uint32_t D1[M], D2[M], s1 = 0, s2 = 0;
+    {
+        int pj = 0;
+        uint32_t d1 = 0, d2 = 0;
+        D1[0] = D2[0] = 0;
+#pragma unroll
+        for (int j = 1; j < M; j++) {
+            pj += v(j - 1);
+            const int b = j * NB + pj;
+            const uint32_t b0 = (uint32_t)Bt[b], b1 = (uint32_t)Bt[pj >= 1 ? b - 1 : b];
+            const uint32_t b2 = (uint32_t)Bt[pj >= 2 ? b - 2 : b];
+            s1 += b1;
+            s2 += b2;
+            D1[j] = d1 += b0 - b1;
+            D2[j] = d2 += b1 - b2;
+        }
+    }
+    // orbitals occupied in any row of the wavefront
+    uint32_t any = 0;
+#pragma unroll
+    for (int k = 0; k < M; k++) any |= __ballot(v(k) > 0) ? 1u << k : 0u;
+    any = __builtin_amdgcn_readfirstlane(any);
+    constexpr uint32_t OUT = 0x80000000u;   // beyond every column (< 2 GiB)
+    cplx acc[MV];
+#pragma unroll
+    for (int m = 0; m < MV; m++) {
+        acc[m] = cmake(0, 0);
+        if (FAC) {   // the diagonal one-body part
+            const kcplx h = (kcplx)(h1 + m * a.mK);
+            cplx d = cmake(0, 0);
+#pragma unroll
+            for (int k = 0; k < M; k++) {
+                const int x = k * (pair_h1_stride(M) + 1);
+                d.re = fma(h[x].re, (double)v(k), d.re);
+                if (!RC) d.im = fma(h[x].im, (double)v(k), d.im);
+            }
+            const cplx c = ldcp(C + m * a.mC + i);
+            acc[m] = RC ? cscale(c, d.re) : cfma(d, c, acc[m]);
+        }
+    }
+    if (!FAC && a.nu1 > 0) {
+        const uint32_t top1 = (uint32_t)(a.nu1 - 1) - s1;
+        const int bytes1 = (int)(a.nu1 * (int64_t)sizeof(cplx));
+        cplx y[M];
+#pragma unroll
+        for (int k = 0; k < M; k++) {
+            const uint32_t off = v(k) >= 1 ? (top1 - D1[k]) * (uint32_t)sizeof(cplx) : OUT;
+            y[k] = ldbuf(a.Y1 + (int64_t)k * a.nu1, bytes1, off);
+        }
+#pragma unroll
+        for (int k = 0; k < M; k++) {
+            const double f = sq[v(k)];
+            acc[0].re = fma(f, y[k].re, acc[0].re);
+            acc[0].im = fma(f, y[k].im, acc[0].im);
+        }
+    }
+    if (a.nu2 > 0) {
+        const uint32_t top2 = (uint32_t)(a.nu2 - 1) - s2;
+        const int bytes2 = (int)(a.nu2 * (int64_t)sizeof(cplx));
+        // pairs c1 <= c2, c2 by c2 in batches of BT: every index below is a
+        // constant (full unroll), the loads of a batch are in flight together
+        constexpr int BT = MV == 1 ? 12 : (MV == 2 ? 6 : 4);
+#pragma clang loop unroll(full)
+        for (int c2 = 0; c2 < M; c2++) {
+            if (!(any >> c2 & 1)) continue;
+            const uint32_t t2 = v(c2) >= 1 ? (top2 - D2[c2]) * (uint32_t)sizeof(cplx) : OUT;
+            cplx sum[MV];   // over c1, without the root of v_c2
+#pragma unroll
+            for (int m = 0; m < MV; m++) sum[m] = cmake(0, 0);
+#pragma clang loop unroll(full)
+            for (int b0 = 0; b0 <= c2; b0 += BT) {
+                cplx y[MV][BT];
+#pragma unroll
+                for (int k = 0; k < BT; k++) {
+                    const int c1 = b0 + k;
+                    if (c1 > c2) break;
+                    const int P = c2 * (c2 + 1) / 2 + c1, blk = FAC ? zblk[P] : P;
+                    const bool occ = v(c1) >= (c1 < c2 ? 1 : 2) && v(c2) >= 1 && blk >= 0;
+                    const uint32_t off = occ ? t2 - D1[c1] * (uint32_t)sizeof(cplx) : OUT;
+#pragma unroll
+                    for (int m = 0; m < MV; m++) y[m][k] = ldbuf(Z + m * a.mZ + (int64_t)(blk >= 0 ? blk : 0) * a.ld2, bytes2, off);
+                }
+#pragma unroll
+                for (int k = 0; k < BT; k++) {
+                    const int c1 = b0 + k;
+                    if (c1 > c2) break;
+                    const int P = c2 * (c2 + 1) / 2 + c1;
+                    const double f = sq[c1 < c2 ? v(c1) : (v(c1) >= 1 ? v(c1) - 1 : 0)];
+#pragma unroll
+                    for (int m = 0; m < MV; m++) {
+                        if (!FAC) {
+                            sum[m].re = fma(f, y[m][k].re, sum[m].re);
+                            sum[m].im = fma(f, y[m][k].im, sum[m].im);
+                            continue;
+                        }
+                        const kcplx zp = (kcplx)(za + m * a.mK) + P;
+                        const cplx z = cmake(zp->re, RC ? 0.0 : zp->im);
+                        if (RC) {
+                            sum[m].re = fma(z.re * f, y[m][k].re, sum[m].re);
+                            sum[m].im = fma(z.re * f, y[m][k].im, sum[m].im);
+                        } else {
+                            sum[m] = cfma(cscale(z, f), y[m][k], sum[m]);
+                        }
+                    }
+                }
+            }
+            const double g2 = sq[v(c2)];
+#pragma unroll
+            for (int m = 0; m < MV; m++) {
+                acc[m].re = fma(g2, sum[m].re, acc[m].re);
+                acc[m].im = fma(g2, sum[m].im, acc[m].im);
+            }
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < MV; m++) {
+        double2 o;
+        o.x = acc[m].re;
+        o.y = acc[m].im;
+        *reinterpret_cast<double2 *>(a.out + (m0 + m) * a.mC + i) = o;
+    }
+}
+
+template <int M, int U>
+mcpi_status launch_y1(const PairArgs &a, int ncu, hipStream_t st)
+{
+    const size_t sm = PairLds<M, U>::bytes(a.N);
+    MCPI_ARG(sm <= 160 * 1024, "pair-space tile exceeds LDS");
+    const int per_cu = std::max(1, (int)(160 * 1024 / sm));
+    const int64_t nb = std::max<int64_t>(1, std::min<int64_t>(a.nut, (int64_t)ncu * per_cu));
+    (void)hipFuncSetAttribute((const void *)k_pair_y1<M, U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
+    hipLaunchKernelGGL((k_pair_y1<M, U>), dim3((unsigned)nb), dim3(PT), sm, st, a);
+    MCPI_HIP(hipGetLastError());
+    return MCPI_OK;
+}
+
+template <int M>
+mcpi_status launch_pair_m(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
+                          hipStream_t st)
+{
+    int dev = 0, ncu = 0;
+    MCPI_HIP(hipGetDevice(&dev));
+    MCPI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    const int N = b.N;
+    const int64_t nu1 = N >= 1 ? nc_of(N - 1, M) : 0, nu2 = N >= 2 ? nc_of(N - 2, M) : 0;
+    const int64_t ld2 = pair_ld(nu2);
+    static_assert(pair_h1_stride(M) == 16, "the pair product reads h1 with row stride 16");
+    // with N >= 2 the one-body part rides in the pair product (h1 folded
+    // into W); the pass over N - 1 particles runs only for N = 1
+    const int64_t nu1p = N == 1 ? nu1 : 0;
+    cplx *Y1 = ws, *Y2 = ws + (size_t)M * nu1p;
+    if (nu1p > 0) {
+        PairArgs a{};
+        a.N = N;
+        a.nc = b.nc;
+        a.nu = a.ld = nu1;
+        a.nut = (nu1 + 127) / 128;
+        a.B = b.B;
+        a.C = C;
+        a.W = c.ph1;
+        a.Y = Y1;
+        MCPI_CHECK((launch_y1<M, 128>(a, ncu, st)));
+    }
+    if (nu2 > 0) {
+        // amplitudes X into the workspace after Y2, then Y2 = W X (rows of
+        // ld2 entries; Y2 has pair_stride(M) rows, X pair_x_rows(M))
+        constexpr int U = PAIR_U;
+        static_assert(16 * PairMulLds<M>::NG == pair_stride(M) && 4 * PairMulLds<M>::KS == pair_x_rows(M),
+                      "pair workspace rows");
+        cplx *X = Y2 + (size_t)pair_stride(M) * ld2;
+        PairArgs a{};
+        a.N = N;
+        a.nc = b.nc;
+        a.nu = nu2;
+        a.nut = (nu2 + U - 1) / U;
+        a.B = b.B;
+        a.C = C;
+        a.W = c.pw;
+        a.Y = X;
+        a.ld = ld2;
+        a.H1 = c.ph1;
+        a.h1s = 1.0 / (N - 1);
+        a.occ = b.occ2;
+        a.ql = c.pql;
+        const size_t sm = pair_amp_lds(N, M);
+        int per_cu = 0;
+        MCPI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_pair_amp<M>, PT, sm));
+        int64_t nb = std::max<int64_t>(1, std::min<int64_t>(a.nut, (int64_t)ncu * std::max(per_cu, 1)));
+        hipLaunchKernelGGL((k_pair_amp<M>), dim3((unsigned)nb), dim3(PT), sm, st, a);
+        MCPI_HIP(hipGetLastError());
+        a.Y = Y2;
+        const size_t smw = PairMulLds<M>::bytes;
+        MCPI_ARG(smw <= 160 * 1024, "pair matrix exceeds LDS");
+        (void)hipFuncSetAttribute((const void *)k_pair_mul<M>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)smw);
+        const int nt = 64 * PAIR_MUL_WAVES;
+        MCPI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_pair_mul<M>, nt, smw));
+        const int64_t nrb = (nu2 + 15) / 16;
+        nb = std::max<int64_t>(1, std::min<int64_t>((nrb + PAIR_MUL_WAVES - 1) / PAIR_MUL_WAVES,
+                                                    (int64_t)ncu * std::max(per_cu, 1)));
+        hipLaunchKernelGGL(k_pair_mul<M>, dim3((unsigned)nb), dim3(nt), smw, st, a, (const cplx *)X);
+        MCPI_HIP(hipGetLastError());
+    }
+    PairOutArgs o{};
+    o.N = N;
+    o.nc = b.nc;
+    o.IF = b.IF;
+    o.B = b.B;
+    o.nu1 = nu1p;
+    o.nu2 = nu2;
+    o.ld2 = ld2;
+    o.Y1 = Y1;
+    o.Y2 = Y2;
+    o.C = C;
+    o.out = out;
+    const size_t sm = sizeof(double) * (N + 3) + sizeof(int32_t) * M * (N + 1);
+    hipLaunchKernelGGL((k_pair_out<M, false, false, 1>), dim3((unsigned)((b.nc + PT - 1) / PT)), dim3(PT), sm, st, o);
+    MCPI_HIP(hipGetLastError());
+    return MCPI_OK;
+}
+
+// Z of the factorized form for chunks x MV members: the rows' tiles, the runs
+// of pairs (as many as give about eight blocks a CU where there are few tiles)
+// and the chunks; tiles dealt to the XCDs in equal chunks of at most G
+template <int NW, int MV, bool RC>
+mcpi_status launch_pairz_amp(PairArgs a, int M, int chunks, int ncu, hipStream_t st)
+{
+    const size_t sm = pair_amp_lds(a.N, M);
+    MCPI_ARG(sm <= 160 * 1024, "pair-space tile exceeds LDS");
+    (void)hipFuncSetAttribute((const void *)k_pairz_amp<NW, MV, RC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)sm);
+    const int64_t want = (8 * ncu + a.nut * chunks - 1) / (a.nut * chunks);
+    const int runs = (int)std::max<int64_t>(1, std::min<int64_t>({want, (a.zR + 3) / 4, PAIR_RUNS}));
+    a.run += pair_run(runs);
+    const int64_t G = MV == 1 ? 128 : 32, rounds = (a.nut + 8 * G - 1) / (8 * G);
+    a.G = (unsigned)std::max<int64_t>(1, a.nut / (8 * rounds));
+    hipLaunchKernelGGL((k_pairz_amp<NW, MV, RC>), dim3((unsigned)a.nut, (unsigned)runs, (unsigned)chunks), dim3(PT), sm,
+                       st, a, M);
+    MCPI_HIP(hipGetLastError());
+    return MCPI_OK;
+}
+
+// the factorized pair form (schedule 7) for chunks x MV members: Z (pzR rows
+// of ld2 a member) at the start of the workspace, then the output pass.
+// Vectors mC entries and coefficient blocks mK bytes apart, member 0's tables
+// in c
+template <int M, int MV, bool RC>
+mcpi_status launch_pairz_m(const BasisDev &b, const HamCoefDev &c, int chunks, const cplx *C, cplx *out, int64_t mC,
+                           int64_t mK, cplx *ws, hipStream_t st)
+{
+    int dev = 0, ncu = 0;
+    MCPI_HIP(hipGetDevice(&dev));
+    MCPI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    const int N = b.N;
+    const int64_t nu2 = nc_of(N - 2, M), ld2 = pair_ld(nu2), mZ = (int64_t)c.pzR * ld2;
+    constexpr int U = PAIR_U;
+    PairArgs a{};
+    a.N = N;
+    a.nc = b.nc;
+    a.nu = nu2;
+    a.nut = (nu2 + U - 1) / U;
+    a.B = b.B;
+    a.C = C;
+    a.Y = ws;
+    a.ld = ld2;
+    a.occ = b.occ2;
+    a.rec = c.pzrec;
+    a.run = c.pzrun;
+    a.zR = c.pzR;
+    a.mC = mC;
+    a.mY = mZ;
+    MCPI_CHECK((launch_pairz_amp<M <= 16 ? 4 : 8, MV, RC>(a, M, chunks, ncu, st)));
+    PairOutArgs o{};
+    o.N = N;
+    o.nc = b.nc;
+    o.IF = b.IF;
+    o.B = b.B;
+    o.nu2 = nu2;
+    o.ld2 = ld2;
+    o.Y2 = ws;
+    o.za = c.pza;
+    o.zblk = c.pzblk;
+    o.h1 = c.ph1;
+    o.C = C;
+    o.out = out;
+    o.mC = mC;
+    o.mZ = mZ;
+    o.mK = mK;
+    const size_t so = sizeof(double) * (N + 3) + sizeof(int32_t) * M * (N + 1);
+    hipLaunchKernelGGL((k_pair_out<M, true, RC, MV>), dim3((unsigned)((b.nc + PT - 1) / PT), (unsigned)chunks), dim3(PT),
+                       so, st, o);
+    MCPI_HIP(hipGetLastError());
+    return MCPI_OK;
+}
+
+template <int M, int MV>
+mcpi_status launch_pairz_r(const BasisDev &b, const HamCoefDev &c, int chunks, const cplx *C, cplx *out, int64_t mC,
+                           int64_t mK, cplx *ws, hipStream_t st)
+{
+    return c.real ? launch_pairz_m<M, MV, true>(b, c, chunks, C, out, mC, mK, ws, st)
+                  : launch_pairz_m<M, MV, false>(b, c, chunks, C, out, mC, mK, ws, st);
+}
+
+}  // namespace
+
+#define MCPI_PAIR_CASE(MM) case MM: return launch_pair_m<MM>(b, c, C, out, ws, st);
+// members: one, or chunks of mv
+#define MCPI_PAIRZ_CASE(MM) case MM: return launch_pairz_r<MM, 1>(b, c, 1, C, out, 0, 0, ws, st);
+#define MCPI_PAIRZ_MV_CASE(MM) \
+    case MM: \
+        if (mv == 1) return launch_pairz_r<MM, 1>(b, c, 1, C, out, 0, 0, ws, st); \
+        return mv == 4 ? launch_pairz_r<MM, 4>(b, c, chunks, C, out, mC, mK, ws, st) \
+                       : launch_pairz_r<MM, 2>(b, c, chunks, C, out, mC, mK, ws, st);
+
+}  // namespace mcpi

@@ -197,6 +197,27 @@ struct mcpi_basis_s {
     bool sectored() const { return d.perm != nullptr; }
 };
 
+// Row tables of the pair amplitudes: tiles of PAIR_U rows, three slots of 8
+// bytes per orbital and row, [orbital][slot][row] (acth_pair.hip)
+constexpr int PAIR_U = 64, PAIR_SLOT = 8 * PAIR_U, PAIR_ORB = 3 * PAIR_SLOT;
+// byte offsets into them for a pair q <= l: q's and l's entries, and the step
+// from l's first root to the one the pair takes (the second for q = l)
+struct PairOff {
+    int32_t oq, ol, e, pad;
+};
+// one pair of a block of the factorized pair form, its factor b, and whether
+// it is the block's last
+struct PairRec {
+    double br, bi;
+    int32_t oq, ol, e, last;
+};
+
+struct PairRun {
+    int32_t r, j;
+};
+constexpr int PAIR_RUNS = 12;
+__host__ __device__ constexpr int pair_run(int g) { return (g - 1) * (2 * g + 1); }   // 4 g + 1 entries for each g
+
 // Folded coefficient tables of a Hamiltonian (device memory), produced on
 // the host from Ho and Hint by the rule folding of hamiltonianMatrix.h:
 // 1494-1963.  For a row with occupations v (r1[q] = sqrt(v_q+1),
@@ -241,7 +262,12 @@ struct HamCoefDev {
     int32_t *pzblk;
     int32_t *pzord;
     int32_t *pzoff;
+    PairRec *pzrec;  // the pairs of pzord with their factors pzb
+    PairRun *pzrun;  // the blocks cut into 4 g runs, g = 1 .. PAIR_RUNS, at
+                     // pair_run(g): run w is blocks [w].r .. [w + 1].r, which
+                     // start at pairs [w].j
     int pzR;
+    PairOff *pql;    // pairs P (with pw; null otherwise)
     int real;        // 1 if every coefficient above has a zero imaginary part
     int dense;       // 1 if at least half of the double-jump terms are non-zero:
                      // walking the lists would cost more than it skips
@@ -279,7 +305,10 @@ __host__ __device__ inline HamCoefDev shift_coef(HamCoefDev c, ptrdiff_t d)
         c.pzblk = sh(c.pzblk);
         c.pzord = sh(c.pzord);
         c.pzoff = sh(c.pzoff);
+        c.pzrec = sh(c.pzrec);
+        c.pzrun = sh(c.pzrun);
     }
+    if (c.pql) c.pql = sh(c.pql);
     return c;
 }
 
@@ -330,6 +359,20 @@ __host__ __device__ inline int pair_index(int k, int s, int M)
 {
     // lexicographic index of k<s among M(M-1)/2 pairs
     return k * (2 * M - k - 1) / 2 + (s - k - 1);
+}
+
+// Hardware block b runs on XCD b % 8 as that XCD's (b / 8)-th block.  Chunks
+// of G consecutive row blocks dealt round-robin to the XCDs: each XCD gets
+// rows from the whole basis (the H.v work per row differs between regions
+// of the basis, so contiguous eighths leave XCDs idle at the end) while
+// neighbouring blocks still share an L2.  Blocks past the last full round
+// of chunks keep their index.
+__device__ inline unsigned chunk_xcd(unsigned b, unsigned n, unsigned G)
+{
+    const unsigned full = n / (8 * G) * (8 * G);
+    if (b >= full) return b;
+    const unsigned x = b % 8, k = b / 8;
+    return ((k / G) * 8 + x) * G + k % G;
 }
 
 // kernels launched from host code of other translation units
