@@ -288,7 +288,7 @@ mcpi_status mcpi_hip_ham_set_skip_zero(mcpi_ham h, int on);
  * a*_k a_l = sum_s a*_k a*_s a_s a_l / (N-1)), and each row gathers its
  * M(M+1)/2 products back (any storage mode, reads no
  * map; 3 <= M <= 12, bases in the reference order; a workspace of about
- * 2 M(M+1)/2 NC(N-2, M) complex entries per stream that runs
+ * M(M+1)/2 NC(N-2, M) complex entries per stream that runs
  * the schedule, allocated on that stream's first use outside stream capture,
  * is kept with the basis; falls back to 2 otherwise or when device memory
  * is short), 7 = 6 in the factorized pair form, for Hamiltonians whose

@@ -30,7 +30,7 @@ namespace mcpi {
 // --------------------------------------------------------- coefficients --
 
 mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefDev *c, void **block,
-                               size_t *block_bytes)
+                               size_t *block_bytes, int N)
 {
     const int64_t M2 = (int64_t)M * M, M3 = M2 * M;
     const int P = M * (M - 1) / 2;
@@ -188,6 +188,24 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
                     }
             }
     }
+    // the pair product's copy of W (HamCoefDev::pwf): h1[k][l] / (N - 1) added
+    // to W[{k, s}][{s, l}] for every s
+    std::vector<cplx> pwf;
+    if (pair && M <= MCPI_PAIR_MAXM && N >= 2) {
+        std::vector<cplx> W = pw;
+        for (int k = 0; k < M; k++)
+            for (int l = 0; l < M; l++)
+                for (int s = 0; s < M; s++) {
+                    cplx &w = W[(size_t)pair_of2(s, l) * PWS + pair_of2(k, s)];
+                    w = cadd(w, cscale(ph1[(size_t)l * HS + k], 1.0 / (N - 1)));
+                }
+        const int NP = pair_count(M), KS = pair_x_rows(M) / 4, NG = PWS / 16;
+        pwf.assign((size_t)KS * NG * 64, cmake(0, 0));
+        for (size_t x = 0; x < pwf.size(); x++) {
+            const int ln = (int)(x % 64), P = 16 * (int)(x / 64 % NG) + ln % 16, Q = 4 * (int)(x / 64 / NG) + ln / 16;
+            if (P < NP && Q < NP) pwf[x] = W[(size_t)Q * PWS + P];
+        }
+    }
     // the factorized pair form of schedule 7 (pair_factor.h)
     std::vector<cplx> za, zb;
     std::vector<int32_t> zblk, zord, zoff;
@@ -225,7 +243,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
         for (int x = 0; x < pair_count(M); x++) pql.push_back(offsets(x));
     // one device block: complex tables first (16-byte aligned), then integers
     size_t nC = dk.size() + d1.size() + d2.size() + A0.size() + A.size() + ot.size() + tt.size() + nz_c.size() +
-                otc.size() + ttc.size() + pw.size() + ph1.size() + za.size() + zb.size();
+                otc.size() + ttc.size() + pw.size() + ph1.size() + pwf.size() + za.size() + zb.size();
     size_t nB = nz1.size() + nzo.size() + nzt.size() + 4 * (m1j.size() + ot_off.size() + tt_off.size() +
                                                            nz_e.size() + zblk.size() + zord.size() + zoff.size()) +
                 zrec.size() * sizeof(PairRec) + zrun.size() * sizeof(PairRun) + pql.size() * sizeof(PairOff) + 64;
@@ -247,6 +265,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     size_t o_ttc = put(ttc.data(), ttc.size() * sizeof(cplx));
     const size_t o_pw = pw.empty() ? 0 : put(pw.data(), pw.size() * sizeof(cplx));
     const size_t o_ph1 = ph1.empty() ? 0 : put(ph1.data(), ph1.size() * sizeof(cplx));
+    const size_t o_pwf = pwf.empty() ? 0 : put(pwf.data(), pwf.size() * sizeof(cplx));
     const size_t o_za = za.empty() ? 0 : put(za.data(), za.size() * sizeof(cplx));
     const size_t o_zb = zb.empty() ? 0 : put(zb.data(), zb.size() * sizeof(cplx));
     const size_t o_zrec = zblk.empty() ? 0 : put(zrec.data(), zrec.size() * sizeof(PairRec));
@@ -278,6 +297,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     c->ttc = (cplx *)(dev + o_ttc);
     c->pw = pair ? (cplx *)(dev + o_pw) : nullptr;
     c->ph1 = pair ? (cplx *)(dev + o_ph1) : nullptr;
+    c->pwf = pwf.empty() ? nullptr : (cplx *)(dev + o_pwf);
     const bool fac = !zblk.empty();
     c->pza = fac ? (cplx *)(dev + o_za) : nullptr;
     c->pzb = fac ? (cplx *)(dev + o_zb) : nullptr;
@@ -627,13 +647,6 @@ static cplx *pair_workspace(mcpi_basis b, hipStream_t st, bool may_alloc, size_t
     void *p = nullptr;
     if (hipMalloc(&p, need) != hipSuccess) {
         (void)hipGetLastError();
-        return nullptr;
-    }
-    // zero once: the rows of the pair amplitudes past the pairs are read
-    // (against zero rows of the pair matrix) and never written
-    if (hipMemset(p, 0, need) != hipSuccess) {
-        (void)hipGetLastError();
-        (void)hipFree(p);
         return nullptr;
     }
     b->pair_ws.push_back({st, p});

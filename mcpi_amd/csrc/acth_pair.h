@@ -20,7 +20,7 @@
 // Y2_u(P) = a[P] Z[r(P)][u] with Z[r][u] = sum_{Q in r} b[Q] X[Q][u]: one
 // sum per block and no product (schedule 7).
 //
-// k_pair_amp<M>: X, gathered.  k_pair_mul<M>: Y2 = W X on the MFMA.
+// k_pair_mul<M>: Y2 = W X on the MFMA, X gathered.
 // k_pairz_amp<>: Z, gathered and summed per block.
 // k_pair_out<M, FAC>: one thread per row v of the basis ranks the v - e_P
 // in the smaller basis from its prefix-count tables and sums the factors
@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "mcpi_internal.h"
+#include "pair_rows.h"
 
 namespace mcpi {
 
@@ -51,11 +52,9 @@ struct PairArgs {
     int64_t nut;          // tiles of U rows
     const int32_t *B;     // rank table B[j*(N+1) + p]
     const cplx *C;
-    const cplx *W;        // pair matrix pw[Q * PWS + P], or h1 as ph1[l * 16 + k] (M <= 12)
+    const cplx *W;        // pair matrix in fragment order (c.pwf), or h1 as ph1[l * 16 + k] (M <= 12)
     cplx *Y;              // Y[col * ld + u]
     int64_t ld;           // row stride of Y (and of the pair amplitudes X), >= nu
-    const cplx *H1;       // pair product: h1 (ph1[l * 16 + k]) folded into W with weight h1s
-    double h1s;           // 1 / (N - 1), or 0
     const uint8_t *occ;   // occupations of the N - 2 particle states (BasisDev::occ2)
     const PairOff *ql;    // pairs: their places in the row tables
     const PairRec *rec;   // factorized form: pairs block by block
@@ -394,221 +393,152 @@ __global__ __launch_bounds__(PT) void k_pairz_amp(PairArgs a, int M)
     }
 }
 
-// The pair amplitudes X[Q][u] = <u|a_{Q1} a_{Q2}|C> of the basis with N-2
-// particles, column-major (X[Q * ld + u]): the row tables as above, lanes over
-// the rows of one column at a time (neighbouring targets, coalesced stores),
-// GBP loads in flight per thread.
-template <int M>
-__global__ __launch_bounds__(PT) void k_pair_amp(PairArgs a)
-{
-    constexpr int NP = pair_count(M), U = PAIR_U;
-    static_assert(M <= 16, "16-byte rows");
-    extern __shared__ __align__(16) unsigned char lds[];
-    double *sq = (double *)(lds + PAIR_ORB * M);               // [N + 3]
-    int32_t *tt = (int32_t *)(sq + a.N + 3);                   // [U]
-    int32_t *Bt = tt + U;                                      // [M][N + 1]
-    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int N = a.N, NB1 = N + 1;
-    const auto ql = kptr(a.ql);
-    for (int x = t; x < M * NB1; x += PT) Bt[x] = a.B[x];
-    for (int x = t; x < N + 3; x += PT) sq[x] = sqrt((double)x);
-    unsigned char *tab = lds + 8 * lane;
-    for (int64_t tile = blockIdx.x; tile < a.nut; tile += gridDim.x) {
-        __syncthreads();
-        const int64_t u = tile * U + lane;
-        if (wave == 0) {
-            const uint4 x = *reinterpret_cast<const uint4 *>(a.occ + (u < a.nu ? u : a.nu - 1) * 16);
-            const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-            tt[lane] = pair_rows<4>(w, M, NB1, (int32_t)(a.nc - 1), Bt, sq, tab);
-        }
-        __syncthreads();
-        const int32_t base = tt[lane];
-        constexpr int GBP = 5;
-#pragma clang loop unroll(disable)
-        for (int p0 = wave; p0 < NP; p0 += 4 * GBP) {
-            double f[GBP];
-            cplx v[GBP];
-#pragma unroll
-            for (int k = 0; k < GBP; k++) {
-                const auto &x = ql[p0 + 4 * k < NP ? p0 + 4 * k : NP - 1];
-                v[k] = ldcp(a.C + pair_target(tab, x.oq, x.ol, x.e, base, f[k]));
-            }
-#pragma unroll
-            for (int k = 0; k < GBP; k++) {
-                const int p = p0 + 4 * k;
-                if (p >= NP || u >= a.nu) continue;
-                const cplx z = cscale(v[k], f[k]);
-                double2 o;
-                o.x = z.re;
-                o.y = z.im;
-                *reinterpret_cast<double2 *>(a.Y + (int64_t)p * a.ld + u) = o;
-            }
-        }
-    }
-}
-
-// Y2 = W X through FP64 MFMA (v_mfma_f64_16x16x4f64: lane i + 16k holds
-// A[i][k] and B[k][i]; the result D[g + 4r][j] sits in register r of lane
-// j + 16g), three real products per complex one (Gauss): T1 = (Xr + Xi)
-// Wr, T2 = Xr (Wi - Wr), T3 = Xi (Wr + Wi), then Re = T1 - T3 and Im = T1 +
-// T2.  The block stages W once in LDS as B fragments in the order the lanes
-// read them: Wa[s][g][lane] = (Wr, Wi - Wr) and Wb[s][g][lane] = Wr + Wi of
-// W[4s + k][16g + j], KS = ceil(NP/4) steps of four Q times NG groups of
-// 16 pair columns P, zero past NP; conflict-free reads.
-// Each wavefront takes 16-row blocks of X on its own and keeps the 16 x NP
-// result block in accumulators: per step one A fragment (four Q rows of 16
-// consecutive u, coalesced; loaded four steps ahead, across row blocks)
-// meets the NG fragments of W, three MFMAs each.
+// Y2 = W X, X[Q][u] = <u|a_{Q1} a_{Q2}|C> gathered on the fly, through FP64 MFMA
+// (v_mfma_f64_16x16x4f64: lane i + 16k holds A[i][k] and B[k][i]; the result
+// D[g + 4r][j] sits in register r of lane j + 16g), three real products per
+// complex one (Gauss): T1 = (Xr + Xi) Wr, T2 = Xr (Wi - Wr), T3 = Xi (Wr + Wi),
+// then Re = T1 - T3 and Im = T1 + T2.  A = W: the block keeps it in LDS as
+// fragments in the order the lanes read them, [s][g][lane] = W[16g + i][4s +
+// k], KS = ceil(NP/4) steps of four Q times NG groups of 16 pair rows P, zero
+// past NP (c.pwf, laid out with the Hamiltonian, its one-body part folded in:
+// folding it in every block took 25 us of the kernel's 82 at N = 10, M = 12).
+// B = X: each wavefront takes 16 rows u on its own, tabulates them (the tables
+// of pair_rows, 16 rows wide) and keeps the NP x 16 result in accumulators;
+// lane (j, k) of step s gathers X[4s + k][u_j], four steps ahead of its use, so
+// X is never written.  Wavefronts share nothing but W: while one starts a row
+// block, the other one of its SIMD has the matrix core.
+// Each XCD takes a contiguous eighth of the row blocks (neighbouring rows
+// gather from neighbouring parts of C).
+// Measured (before: X written by a kernel of its own, W folded and staged by
+// every block): N = 10, M = 12 amplitudes and product 30 + 82 -> 66 us; N = 12,
+// M = 12 0.13 + 0.28 -> 0.27 ms; 51 TFLOP/s issued of the 64 that this loop
+// reaches without memory; the workspace halves.
 typedef double mcpi_v4d __attribute__((ext_vector_type(4)));
 
 constexpr int PAIR_MUL_WAVES = 8;
 
-// The one-body operator in pair form: on states of N >= 2 particles
-//   a*_k a_l = (1 / (N - 1)) sum_s a*_k a*_s a_s a_l
-// (the number operator is N - 1 on a_l |v>), so h1 adds
-// h1[k][l] / (N - 1) to W[{k, s}][{s, l}] for every s.  This is the sum of
-// h1[k][l] over the orderings (k, s) of the pair P and (s, l) of the pair Q
-// that share s.
-__device__ inline cplx h1_pair(const cplx *h1, int P, int Q)
-{
-    const int p2 = pair_hi(P), p1 = P - p2 * (p2 + 1) / 2;
-    const int q2 = pair_hi(Q), q1 = Q - q2 * (q2 + 1) / 2;
-    cplx z = cmake(0, 0);
-    for (int o = 0; o < (p1 == p2 ? 1 : 2); o++) {
-        const int k = o ? p1 : p2, s = o ? p2 : p1;
-        for (int o2 = 0; o2 < (q1 == q2 ? 1 : 2); o2++) {
-            const int s2 = o2 ? q2 : q1, l = o2 ? q1 : q2;
-            if (s2 == s) z = cadd(z, ldcp(h1 + l * 16 + k));
-        }
-    }
-    return z;
-}
-
 template <int M>
 struct PairMulLds {
-    static constexpr int NP = pair_count(M), KS = (NP + 3) / 4, NG = (NP + 15) / 16;
-    static constexpr size_t bytes = (sizeof(double2) + sizeof(double)) * NG * KS * 64;
+    static constexpr int NP = pair_count(M), KS = pair_x_rows(M) / 4, NG = pair_stride(M) / 16;
+    static constexpr int ORB = PAIR_ORB / 4, SLOT = PAIR_SLOT / 4;   // tables of 16 rows
+    static size_t bytes(int N)
+    {
+        const size_t o = sizeof(cplx) * NG * KS * 64 + (size_t)PAIR_MUL_WAVES * ORB * M + sizeof(double) * (N + 3) +
+                         sizeof(int4) * 4 * KS + sizeof(int32_t) * M * (N + 1);
+        return (o + 31) / 16 * 16;
+    }
 };
 
 template <int M>
-__global__ __launch_bounds__(64 * PAIR_MUL_WAVES) void k_pair_mul(PairArgs a, const cplx *X)
+__global__ __launch_bounds__(64 * PAIR_MUL_WAVES) void k_pair_mul(PairArgs a)
 {
     using L = PairMulLds<M>;
-    constexpr int NP = L::NP, KS = L::KS, NG = L::NG, PWS = pair_stride(M);
+    constexpr int NP = L::NP, KS = L::KS, NG = L::NG, ORB = L::ORB, SLOT = L::SLOT;
+    static_assert(M <= 16, "16-byte occupation rows");
     extern __shared__ __align__(16) unsigned char lds[];
-    double2 *wa = (double2 *)lds;                 // [KS][NG][64]
-    double *wb = (double *)(wa + NG * KS * 64);   // [KS][NG][64]
-    for (int x = threadIdx.x; x < NG * KS * 64; x += blockDim.x) {
-        const int s = x / (NG * 64), g = (x / 64) % NG, ln = x % 64;
-        const int P = 16 * g + (ln & 15), Q = 4 * s + (ln >> 4);
-        double2 v = {0, 0};
-        double vb = 0;
-        if (P < NP && Q < NP) {
-            cplx w = ldcp(a.W + (int64_t)Q * PWS + P);
-            if (a.h1s != 0.0) {
-                const cplx h = h1_pair(a.H1, P, Q);
-                w.re = fma(a.h1s, h.re, w.re);
-                w.im = fma(a.h1s, h.im, w.im);
-            }
-            v.x = w.re;
-            v.y = w.im - w.re;
-            vb = w.re + w.im;
-        }
-        wa[x] = v;
-        wb[x] = vb;
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    cplx *wl = (cplx *)lds;                                            // [KS][NG][64]
+    int4 *off = (int4 *)(wl + NG * KS * 64);                           // [4 KS]
+    unsigned char *tabs = (unsigned char *)(off + 4 * KS);             // [wave][M][3][16] of 8 bytes
+    double *sq = (double *)(tabs + PAIR_MUL_WAVES * ORB * M);          // [N + 3]
+    int32_t *Bt = (int32_t *)(sq + a.N + 3);                           // [M][N + 1]
+    const int N = a.N, NB1 = N + 1, nt = 64 * PAIR_MUL_WAVES, t = threadIdx.x;
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int jl = lane & 15, kl = lane >> 4;
-    const int64_t nrb = (a.nu + 15) / 16, stride = (int64_t)gridDim.x * PAIR_MUL_WAVES;
-    // (the launch gives ld >= 16 nrb)
-    // A fragments: lane (j, k) of step s of row block rb reads X[4s + k][16
-    // rb + j].  X has 4 KS rows of ld >= 16 nrb entries, zero past NP rows
-    // and nu columns, and Y has 16 NG rows of ld entries, so that neither
-    // loads nor stores need a bound; a block past the last is read as the
-    // last.
-    const int64_t rowstep = 4 * a.ld;
-    auto lanep = [&](int64_t rb) { return X + (int64_t)kl * a.ld + (rb < nrb ? rb : nrb - 1) * 16 + jl; };
-    // They are loaded four steps before their use, across row blocks: the
-    // steps of a block are counted up to KS4 = KS rounded up to four (the
-    // steps past KS load step KS - 1 again and skip their MFMAs), so that
-    // step t of the ring always sits in register t % 4.
-    constexpr int KS4 = (KS + 3) & ~3;
-    auto ldx = [&](const cplx *p, int s) { return ldcp(p + (int64_t)(s < KS ? s : KS - 1) * rowstep); };
-    int64_t rb = (int64_t)blockIdx.x * PAIR_MUL_WAVES + wave;
-    const cplx *pc = lanep(rb);
-    cplx x0 = ldx(pc, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    cplx x1 = ldx(pc, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    cplx x2 = ldx(pc, 2);
-    __builtin_amdgcn_sched_barrier(0);
-    cplx x3 = ldx(pc, 3);
-    __builtin_amdgcn_sched_barrier(0);
-    // one row block: KS4 steps in straight-line code, then the stores
-    auto block = [&](int64_t rb, const cplx *pn) {
-        auto ldnext = [&](int t) { return t < KS4 ? ldx(pc, t) : ldx(pn, t - KS4); };
+
+    // this wavefront's row blocks: the XCD's eighth, dealt to its blocks, then
+    // to their wavefronts
+    const int64_t nrb = (a.nu + 15) / 16;
+    const int nx = gridDim.x >= 8 ? 8 : 1, x = blockIdx.x % nx, bx = blockIdx.x / nx;
+    const int nbx = ((int)gridDim.x - x + nx - 1) / nx;   // blocks of this XCD
+    const int64_t end = nrb * (x + 1) / nx, step = (int64_t)nbx * PAIR_MUL_WAVES;
+    int64_t rb = nrb * x / nx + bx + (int64_t)nbx * wave;
+
+    // occupations of a row block: lanes 0..15 and 16..31 hold the same rows
+    // (one half of the tables each)
+    uint32_t ow[4] = {0, 0, 0, 0};
+    auto occ_row = [&](int64_t r) {
+        if (lane >= 32) return;
+        int64_t u = r * 16 + jl;
+        u = u < a.nu ? u : a.nu - 1;
+        const uint4 w = *reinterpret_cast<const uint4 *>(a.occ + u * 16);
+        ow[0] = w.x;
+        ow[1] = w.y;
+        ow[2] = w.z;
+        ow[3] = w.w;
+    };
+    if (rb < end) occ_row(rb);
+    for (int k = t; k < NG * KS * 64; k += nt) wl[k] = ldcp(a.W + k);
+    for (int k = t; k < 4 * KS; k += nt) {
+        const PairOff o = a.ql[k < NP ? k : NP - 1];
+        off[k] = make_int4(o.oq / 4, o.ol / 4, o.e / 4, 0);
+    }
+    for (int k = t; k < M * NB1; k += nt) Bt[k] = a.B[k];
+    for (int k = t; k < N + 3; k += nt) sq[k] = sqrt((double)k);
+    __syncthreads();
+    unsigned char *tab = tabs + wave * (ORB * M);
+    int32_t base = 0;
+    // targets and factors of step s, and the gather
+    auto get = [&](int s, cplx &v, double &f) {
+        const int4 o = off[4 * (s < KS ? s : KS - 1) + kl];
+        const unsigned char *p = tab + 8 * jl;
+        f = *(const double *)(p + o.x + SLOT) * *(const double *)(p + o.y + o.z + SLOT);
+        v = ldcp(a.C + (uint32_t)(base - *(const int32_t *)(p + o.x) - *(const int32_t *)(p + o.y + PAIR_DL)));
+    };
+    for (; rb < end; rb += step) {
+        if (lane < 32) {
+            const int d = lane >> 4;
+            const int32_t s = pair_row_tables<4>(ow, M, NB1, Bt, sq, d, (int32_t *)(tab + 8 * jl + 4 * d), ORB / 4,
+                                                 (double *)(tab + 8 * jl + SLOT * (1 + d)), ORB / 8);
+            base = (int32_t)(a.nc - 1) - s;   // of lanes 16..31: rank(u + 2 e_0)
+        }
+        base = __shfl(base, 16 + jl, 64);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (rb + step < end) occ_row(rb + step);
+        cplx x0, x1, x2, x3;
+        double f0, f1, f2, f3;
+        get(0, x0, f0);
+        get(1, x1, f1);
+        get(2, x2, f2);
+        get(3, x3, f3);
         mcpi_v4d acc[3 * NG];
 #pragma unroll
         for (int g = 0; g < 3 * NG; g++) acc[g] = mcpi_v4d{0, 0, 0, 0};
-        auto step = [&](int s, const cplx xc) {
-            if (s >= KS) return;
-            const double xs = xc.re + xc.im;
+        auto mul = [&](int s, const cplx v, double f) {
+            const double xr = v.re * f, xi = v.im * f, xs = xr + xi;
 #pragma unroll
             for (int g = 0; g < NG; g++) {
-                const double2 w = wa[(s * NG + g) * 64 + lane];
-                const double w3 = wb[(s * NG + g) * 64 + lane];
-                acc[3 * g] = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, w.x, acc[3 * g], 0, 0, 0);
-                acc[3 * g + 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(xc.re, w.y, acc[3 * g + 1], 0, 0, 0);
-                acc[3 * g + 2] = __builtin_amdgcn_mfma_f64_16x16x4f64(xc.im, w3, acc[3 * g + 2], 0, 0, 0);
-            }
-            // LDS reads of one group ahead of its three MFMAs, in turn
-#pragma unroll
-            for (int g = 0; g < NG; g++) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+                const cplx w = wl[(s * NG + g) * 64 + lane];
+                acc[3 * g] = __builtin_amdgcn_mfma_f64_16x16x4f64(w.re, xs, acc[3 * g], 0, 0, 0);
+                acc[3 * g + 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(w.im - w.re, xr, acc[3 * g + 1], 0, 0, 0);
+                acc[3 * g + 2] = __builtin_amdgcn_mfma_f64_16x16x4f64(w.re + w.im, xi, acc[3 * g + 2], 0, 0, 0);
             }
         };
 #pragma unroll
-        for (int s = 0; s < KS4; s += 4) {
-            step(s, x0);
+        for (int s = 0; s < KS; s += 4) {
+            mul(s, x0, f0);
+            if (s + 4 < KS) get(s + 4, x0, f0);
             __builtin_amdgcn_sched_barrier(0);
-            x0 = ldnext(s + 4);
-            step(s + 1, x1);
+            if (s + 1 < KS) mul(s + 1, x1, f1);
+            if (s + 5 < KS) get(s + 5, x1, f1);
             __builtin_amdgcn_sched_barrier(0);
-            x1 = ldnext(s + 5);
-            step(s + 2, x2);
+            if (s + 2 < KS) mul(s + 2, x2, f2);
+            if (s + 6 < KS) get(s + 6, x2, f2);
             __builtin_amdgcn_sched_barrier(0);
-            x2 = ldnext(s + 6);
-            step(s + 3, x3);
+            if (s + 3 < KS) mul(s + 3, x3, f3);
+            if (s + 7 < KS) get(s + 7, x3, f3);
             __builtin_amdgcn_sched_barrier(0);
-            x3 = ldnext(s + 7);
         }
+        // (Y has 16 NG rows of ld >= 16 nrb entries: no bounds)
 #pragma unroll
         for (int g = 0; g < NG; g++) {
-            cplx *y = a.Y + (int64_t)(16 * g + jl) * a.ld + rb * 16 + kl;
+            cplx *y = a.Y + (int64_t)(16 * g + kl) * a.ld + rb * 16 + jl;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 double2 o;
                 o.x = acc[3 * g][r] - acc[3 * g + 2][r];
                 o.y = acc[3 * g][r] + acc[3 * g + 1][r];
-                *reinterpret_cast<double2 *>(y + 4 * r) = o;
+                *reinterpret_cast<double2 *>(y + 4 * r * a.ld) = o;
             }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // The first block is peeled, so that the loop is entered with the
-    // stores of a block in flight as on every later pass: the first steps of
-    // a block then wait only for their own fragments (loaded before those
-    // stores), not for the stores to complete.
-    if (rb < nrb) {
-        const cplx *pn = lanep(rb + stride);
-        block(rb, pn);
-        pc = pn;
-        for (rb += stride; rb < nrb; rb += stride) {
-            pn = lanep(rb + stride);
-            block(rb, pn);
-            pc = pn;
         }
     }
 }
@@ -844,43 +774,27 @@ mcpi_status launch_pair_m(const BasisDev &b, const HamCoefDev &c, const cplx *C,
         MCPI_CHECK((launch_y1<M, 128>(a, ncu, st)));
     }
     if (nu2 > 0) {
-        // amplitudes X into the workspace after Y2, then Y2 = W X (rows of
-        // ld2 entries; Y2 has pair_stride(M) rows, X pair_x_rows(M))
-        constexpr int U = PAIR_U;
-        static_assert(16 * PairMulLds<M>::NG == pair_stride(M) && 4 * PairMulLds<M>::KS == pair_x_rows(M),
-                      "pair workspace rows");
-        cplx *X = Y2 + (size_t)pair_stride(M) * ld2;
         PairArgs a{};
         a.N = N;
         a.nc = b.nc;
         a.nu = nu2;
-        a.nut = (nu2 + U - 1) / U;
         a.B = b.B;
         a.C = C;
-        a.W = c.pw;
-        a.Y = X;
+        a.W = c.pwf;
+        a.Y = Y2;
         a.ld = ld2;
-        a.H1 = c.ph1;
-        a.h1s = 1.0 / (N - 1);
         a.occ = b.occ2;
         a.ql = c.pql;
-        const size_t sm = pair_amp_lds(N, M);
-        int per_cu = 0;
-        MCPI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_pair_amp<M>, PT, sm));
-        int64_t nb = std::max<int64_t>(1, std::min<int64_t>(a.nut, (int64_t)ncu * std::max(per_cu, 1)));
-        hipLaunchKernelGGL((k_pair_amp<M>), dim3((unsigned)nb), dim3(PT), sm, st, a);
-        MCPI_HIP(hipGetLastError());
-        a.Y = Y2;
-        const size_t smw = PairMulLds<M>::bytes;
+        const size_t smw = PairMulLds<M>::bytes(N);
         MCPI_ARG(smw <= 160 * 1024, "pair matrix exceeds LDS");
         (void)hipFuncSetAttribute((const void *)k_pair_mul<M>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)smw);
         const int nt = 64 * PAIR_MUL_WAVES;
+        int per_cu = 0;
         MCPI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_pair_mul<M>, nt, smw));
         const int64_t nrb = (nu2 + 15) / 16;
-        nb = std::max<int64_t>(1, std::min<int64_t>((nrb + PAIR_MUL_WAVES - 1) / PAIR_MUL_WAVES,
-                                                    (int64_t)ncu * std::max(per_cu, 1)));
-        hipLaunchKernelGGL(k_pair_mul<M>, dim3((unsigned)nb), dim3(nt), smw, st, a, (const cplx *)X);
+        const int64_t nb = std::max<int64_t>(1, std::min<int64_t>(nrb, (int64_t)ncu * std::max(per_cu, 1)));
+        hipLaunchKernelGGL(k_pair_mul<M>, dim3((unsigned)nb), dim3(nt), smw, st, a);
         MCPI_HIP(hipGetLastError());
     }
     PairOutArgs o{};

@@ -18,21 +18,19 @@ mcpi_status launch_pairz_c(MCPI_PAIRZ_ARGS);
 mcpi_status launch_pairz_d(MCPI_PAIRZ_ARGS);
 
 // complex entries of the pair-space workspace of a basis: Y1 (M rows of
-// NC(N-1, M), for N = 1 only), then Y2 (pair_stride(M) rows) and the pair
-// amplitudes X (pair_x_rows(M) rows) with rows of pair_ld(NC(N-2, M))
-// entries; the caller zeroes it once (the pad rows and columns of X are
-// read, never written)
+// NC(N-1, M), for N = 1 only), then Y2 (pair_stride(M) rows of
+// pair_ld(NC(N-2, M)) entries)
 size_t pair_workspace_entries(int N, int M)
 {
     const int64_t nu1 = N == 1 ? nc_of(N - 1, M) : 0, nu2 = N >= 2 ? nc_of(N - 2, M) : 0;
-    return (size_t)M * nu1 + (size_t)(pair_stride(M) + pair_x_rows(M)) * pair_ld(nu2);
+    return (size_t)M * nu1 + (size_t)pair_stride(M) * pair_ld(nu2);
 }
 
 bool pair_applicable(const BasisDev &b, const HamCoefDev &c)
 {
     // (the output pass reads Y1 and Y2 columns as buffers of < 2 GiB:
     // NC(N-1, M) >= NC(N-2, M) entries of 16 bytes)
-    return c.pw && c.ph1 && (b.occ2 || b.N < 2) && b.M >= 3 && b.M <= MCPI_PAIR_MAXM && !b.perm && b.IF && b.nc <= INT32_MAX &&
+    return c.ph1 && (b.N < 2 || (c.pwf && b.occ2)) && b.M >= 3 && b.M <= MCPI_PAIR_MAXM && !b.perm && b.IF && b.nc <= INT32_MAX &&
            b.N <= MCPI_MAXN && (b.N < 1 || nc_of(b.N - 1, b.M) < ((int64_t)1 << 27));
 }
 

@@ -151,7 +151,7 @@ mcpi_status mcpi_hip_ham_create(mcpi_basis b, const mcpi_cplx *Ho, const mcpi_cp
         }
     }
     mcpi_status st = build_coefficients(M, (const cplx *)Ho, (const cplx *)Hint, &h->c, &h->coef_block,
-                                        &h->coef_bytes);
+                                        &h->coef_bytes, b->d.N);
     // sector order: the zero-skipping kernel on the pattern tables is the one
     // H.v, so its term lists are walked even when most terms are non-zero
     if (st == MCPI_OK && b->sectored()) h->c.dense = 0;

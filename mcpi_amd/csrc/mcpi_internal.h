@@ -170,12 +170,11 @@ struct mcpi_basis_s {
     void *rho_ws = nullptr;
     size_t rho_ws_bytes = 0;
     std::mutex rho_mu;
-    // pair-space H.v workspaces (schedule 6: the pair amplitudes and the Y
-    // tables of the bases with N-1 and N-2 particles; schedule 7: the Z
-    // rows), per stream that ran a pair-space schedule (so that H.v calls
-    // on different streams never share one), allocated on first use, a
-    // larger one beside a smaller one when the schedule needs it, and kept
-    // until the basis is freed
+    // pair-space H.v workspaces (schedule 6: the Y table of the basis with
+    // N - 2 particles, or N - 1 = 0; schedule 7: the Z rows), per stream that
+    // ran a pair-space schedule (so that H.v calls on different streams never
+    // share one), allocated on first use, a larger one beside a smaller one
+    // when the schedule needs it, and kept until the basis is freed
     struct PairWs {
         hipStream_t st;
         void *p;
@@ -253,6 +252,11 @@ struct HamCoefDev {
     // orbital contiguous, PWS = M(M+1)/2 rounded up to 16, zero padded)
     cplx *pw;
     cplx *ph1;
+    // pw with the one-body part folded in for N >= 2 particles (a*_k a_l =
+    // sum_s a*_k a*_s a_s a_l / (N - 1)), as the fragments of the pair product:
+    // [s][g][lane] = W[16 g + lane % 16][4 s + lane / 16], zero past the pairs
+    // (M <= MCPI_PAIR_MAXM and N given to build_coefficients; null otherwise)
+    cplx *pwf;
     // factorized pair form (schedule 7; null / 0 unless h1 is diagonal and
     // pw is block diagonal with rank-one blocks): pw[P][Q] = pza[P] pzb[Q]
     // for P, Q in one block; pzblk[P] = block of P (-1: none); pzord lists
@@ -299,6 +303,7 @@ __host__ __device__ inline HamCoefDev shift_coef(HamCoefDev c, ptrdiff_t d)
     c.nz_c = sh(c.nz_c);
     if (c.pw) c.pw = sh(c.pw);
     if (c.ph1) c.ph1 = sh(c.ph1);
+    if (c.pwf) c.pwf = sh(c.pwf);
     if (c.pza) {
         c.pza = sh(c.pza);
         c.pzb = sh(c.pzb);
@@ -325,8 +330,7 @@ __host__ __device__ constexpr int pair_hi(int P)
     while ((c2 + 1) * (c2 + 2) / 2 <= P) c2++;
     return c2;
 }
-// rows of the pair-amplitude matrix X of the pair-space H.v: the pairs,
-// rounded up to four (the rows past the pairs stay zero)
+// columns of the pair matrix in the pair product: the pairs, rounded up to four
 __host__ __device__ constexpr int pair_x_rows(int M) { return (pair_count(M) + 3) / 4 * 4; }
 // row stride of the pair-space matrices over nu states: nu rounded up to 16
 __host__ __device__ constexpr int64_t pair_ld(int64_t nu) { return (nu + 15) / 16 * 16; }
@@ -394,8 +398,9 @@ mcpi_status launch_comp(const BasisDev &b, const HamCoefDev &c, const cplx *C, c
 // wavefronts (Map and packed tables; 2 when the basis has no packed tables)
 mcpi_status launch_apply_raw(const BasisDev &b, int maps, const HamCoefDev &c, int skip_zero,
                              int schedule, const cplx *C, cplx *out, hipStream_t st);
+// N: particles, for the tables of the pair product (0: without them)
 mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefDev *c, void **block,
-                               size_t *block_bytes = nullptr);
+                               size_t *block_bytes = nullptr, int N = 0);
 mcpi_status basis_upload_raw(int N, int M, const int32_t *IF, const int32_t *NCmat,
                              const int32_t *Map, const int32_t *MapOT, const int32_t *MapTT,
                              const int *strideOT, const int *strideTT, int64_t ot_len,

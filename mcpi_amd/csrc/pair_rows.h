@@ -14,14 +14,14 @@
 namespace mcpi {
 
 // One half of the tables of a row with occupations w (bytes, orbital 0
-// first): D[o * stride] = S_d(o) - S_{d+1}(o) and G[o * stride] = sqrt(v_o + 1
-// + d) for every orbital o < M; returns S_{d+1}(M - 1).  NW words of w cover M
+// first): D[o * sd] = S_d(o) - S_{d+1}(o) and G[o * sg] = sqrt(v_o + 1 + d) for
+// every orbital o < M; returns S_{d+1}(M - 1).  NW words of w cover M
 // orbitals.  d = 0: the tables of q (and of l > q for the roots), d = 1: of l.
 // Four orbitals' entries are in flight together (all of them took more
 // registers than the products beside leave).
 template <int NW>
 __device__ inline int32_t pair_row_tables(const uint32_t (&w)[NW], int M, int NB1, const int32_t *Bt, const double *sq,
-                                          int d, int32_t *D, double *G, int stride)
+                                          int d, int32_t *D, int sd, double *G, int sg)
 {
     // (an empty statement that takes the sizes: without it what depends on
     // them alone moves out of the caller's loop, and every scalar register
@@ -54,8 +54,8 @@ __device__ inline int32_t pair_row_tables(const uint32_t (&w)[NW], int M, int NB
                 s += lo[j] - hi[j];
                 s1 += hi[j];
             }
-            D[o * stride] = s;
-            G[o * stride] = r[j];
+            D[o * sd] = s;
+            G[o * sg] = r[j];
         }
     }
     return s1;

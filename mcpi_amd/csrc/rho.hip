@@ -295,7 +295,8 @@ k_gram(GramArgs a)
         }
     };
     auto occ_tables = [&](int64_t tile) {
-        const int32_t s = pair_row_tables<NW>(ow, M, NB1, Bt, sq, dh, dd + dh * M * GU + dr, g + dh * M * GU + dr, GU);
+        const int32_t s = pair_row_tables<NW>(ow, M, NB1, Bt, sq, dh, dd + dh * M * GU + dr, GU,
+                                              g + dh * M * GU + dr, GU);
         if (dh == 1) tt[dr] = tile * GU + dr < a.nu ? (int32_t)(a.nc - 1) - s : -1;
     };
 
