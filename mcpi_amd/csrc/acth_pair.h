@@ -577,10 +577,12 @@ struct PairOutArgs {
     const cplx *h1, *C;
     cplx *out;
     int64_t mC, mZ, mK;
+    int S;   // wavefronts that share a row's pairs: 1, 2 or 4
 };
 
 template <int M, bool FAC, bool RC, int MV>
-__global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
+__global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(MV == 1 && M <= 16 ? 4 : 3))) void
+k_pair_out(PairOutArgs a)
 {
     static_assert(FAC || (MV == 1 && !RC), "several members: factorized form only");
     extern __shared__ __align__(16) unsigned char lds[];
@@ -591,8 +593,10 @@ __global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
     for (int x = threadIdx.x; x < N + 3; x += PT) sq[x] = sqrt((double)x);
     for (int x = threadIdx.x; x < M * NB; x += PT) Bt[x] = a.B[x];
     __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * PT + threadIdx.x;
-    if (i >= a.nc) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = wave % a.S;   // this wavefront's share of its rows
+    const int64_t i0 = ((int64_t)blockIdx.x * (PT / 64 / a.S) + wave / a.S) * 64 + lane;
+    const int64_t i = i0 < a.nc ? i0 : a.nc - 1;
     const int64_t m0 = MV > 1 ? (int64_t)blockIdx.y * MV : 0;   // this grid row's first member
     const cplx *C = a.C + m0 * a.mC, *Z = a.Y2 + m0 * a.mZ;
     // the coefficients' uniform indices give scalar loads
@@ -632,12 +636,23 @@ __global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
 #pragma unroll
     for (int k = 0; k < M; k++) any |= __ballot(v(k) > 0) ? 1u << k : 0u;
     any = __builtin_amdgcn_readfirstlane(any);
+    // with S wavefronts a row, the orbitals c2 this one takes: dealt from the
+    // highest (most pairs) to and fro
+    uint32_t mine = any;
+    if (a.S > 1) {
+        mine = 0;
+#pragma unroll
+        for (int k = 0; k < M; k++) {
+            const int x = (M - 1 - k) & (2 * a.S - 1);
+            if ((x < a.S ? x : 2 * a.S - 1 - x) == sub) mine |= any & 1u << k;
+        }
+    }
     constexpr uint32_t OUT = 0x80000000u;   // beyond every column (< 2 GiB)
     cplx acc[MV];
 #pragma unroll
     for (int m = 0; m < MV; m++) {
         acc[m] = cmake(0, 0);
-        if (FAC) {   // the diagonal one-body part
+        if (FAC && sub == 0) {   // the diagonal one-body part
             const kcplx h = (kcplx)(h1 + m * a.mK);
             cplx d = cmake(0, 0);
 #pragma unroll
@@ -650,7 +665,7 @@ __global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
             acc[m] = RC ? cscale(c, d.re) : cfma(d, c, acc[m]);
         }
     }
-    if (!FAC && a.nu1 > 0) {
+    if (!FAC && a.nu1 > 0 && sub == 0) {
         const uint32_t top1 = (uint32_t)(a.nu1 - 1) - s1;
         const int bytes1 = (int)(a.nu1 * (int64_t)sizeof(cplx));
         cplx y[M];
@@ -674,7 +689,7 @@ __global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
         constexpr int BT = MV == 1 ? 12 : (MV == 2 ? 6 : 4);
 #pragma clang loop unroll(full)
         for (int c2 = 0; c2 < M; c2++) {
-            if (!(any >> c2 & 1)) continue;
+            if (!(mine >> c2 & 1)) continue;
             const uint32_t t2 = v(c2) >= 1 ? (top2 - D2[c2]) * (uint32_t)sizeof(cplx) : OUT;
             cplx sum[MV];   // over c1, without the root of v_c2
 #pragma unroll
@@ -724,6 +739,20 @@ __global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
             }
         }
     }
+    if (a.S > 1) {   // the shares' sums, in order (over the tables, which are done with)
+        cplx *red = (cplx *)lds;   // [member][wave][64]
+        __syncthreads();
+        if (sub > 0) {
+#pragma unroll
+            for (int m = 0; m < MV; m++) red[(m * (PT / 64) + wave) * 64 + lane] = acc[m];
+        }
+        __syncthreads();
+        if (sub > 0) return;
+        for (int w = 1; w < a.S; w++)
+#pragma unroll
+            for (int m = 0; m < MV; m++) acc[m] = cadd(acc[m], red[(m * (PT / 64) + wave + w) * 64 + lane]);
+    }
+    if (i0 >= a.nc) return;
 #pragma unroll
     for (int m = 0; m < MV; m++) {
         double2 o;
@@ -731,6 +760,26 @@ __global__ __launch_bounds__(PT) void k_pair_out(PairOutArgs a)
         o.y = acc[m].im;
         *reinterpret_cast<double2 *>(a.out + (m0 + m) * a.mC + i) = o;
     }
+}
+
+// launch of the output pass for `chunks` grid rows.  A row's pairs are a serial
+// chain of batches, which few rows leave exposed: up to four wavefronts share
+// a row's pairs until there are two blocks a CU.  Lanczos steps, us, without
+// and with: N = 5, M = 21 (208 blocks of whole rows) 118, 110; N = 6, M = 9 (12)
+// 43.0, 40.5; N = 7, M = 13 (197) 66.3, 63.2; with eight blocks a CU N = 10, M =
+// 11 (722) slows from 125 to 129.
+template <int M, bool FAC, bool RC, int MV>
+mcpi_status launch_pair_out(PairOutArgs o, int chunks, int ncu, hipStream_t st)
+{
+    const int64_t rows = (o.nc + 63) / 64;   // wavefronts of whole rows
+    o.S = 1;
+    while (o.S < 4 && rows * chunks * o.S < (int64_t)2 * 4 * ncu) o.S *= 2;
+    const int64_t nb = (rows * o.S + PT / 64 - 1) / (PT / 64);
+    size_t sm = sizeof(double) * (o.N + 3) + sizeof(int32_t) * M * (o.N + 1);
+    if (o.S > 1) sm = std::max(sm, sizeof(cplx) * PT * MV);
+    hipLaunchKernelGGL((k_pair_out<M, FAC, RC, MV>), dim3((unsigned)nb, (unsigned)chunks), dim3(PT), sm, st, o);
+    MCPI_HIP(hipGetLastError());
+    return MCPI_OK;
 }
 
 template <int M, int U>
@@ -809,10 +858,7 @@ mcpi_status launch_pair_m(const BasisDev &b, const HamCoefDev &c, const cplx *C,
     o.Y2 = Y2;
     o.C = C;
     o.out = out;
-    const size_t sm = sizeof(double) * (N + 3) + sizeof(int32_t) * M * (N + 1);
-    hipLaunchKernelGGL((k_pair_out<M, false, false, 1>), dim3((unsigned)((b.nc + PT - 1) / PT)), dim3(PT), sm, st, o);
-    MCPI_HIP(hipGetLastError());
-    return MCPI_OK;
+    return launch_pair_out<M, false, false, 1>(o, 1, ncu, st);
 }
 
 // Z of the factorized form for chunks x MV members: the rows' tiles, the runs
@@ -882,11 +928,7 @@ mcpi_status launch_pairz_m(const BasisDev &b, const HamCoefDev &c, int chunks, c
     o.mC = mC;
     o.mZ = mZ;
     o.mK = mK;
-    const size_t so = sizeof(double) * (N + 3) + sizeof(int32_t) * M * (N + 1);
-    hipLaunchKernelGGL((k_pair_out<M, true, RC, MV>), dim3((unsigned)((b.nc + PT - 1) / PT), (unsigned)chunks), dim3(PT),
-                       so, st, o);
-    MCPI_HIP(hipGetLastError());
-    return MCPI_OK;
+    return launch_pair_out<M, true, RC, MV>(o, chunks, ncu, st);
 }
 
 template <int M, int MV>

@@ -21,7 +21,9 @@
 //     gemv_dots     partial o_t = <v_t, HC>, t <= i+1
 //   7 fin_ortho     o_t
 //   8 reorth_norm   HC -= sum_t v_t o_t;  partial ||HC||^2 for the next step
-//   9 advance       i += 1
+// With few partials the kernel that needs a sum forms it itself, every block
+// the same one in the same order, and 1, 5 and 7 are no launches of their own;
+// on short vectors 6 is one launch too (LzChain).
 // Every scalar lives in device memory and the pointers never change, so the
 // chain is captured once in a hipGraph and replayed lm-1 times with no host
 // round trip.  An instance that breaks down stops updating (its kernels
@@ -44,6 +46,8 @@ namespace mcpi {
 
 struct LanczosState {
     int it;        // current iteration index i
+    int it_next;   // the next one: read by the first kernel of an iteration
+                   // only, written by the last only
     int broke;     // 1 once a breakdown was detected
     int steps;     // size of the tridiagonal built so far
     int lm;
@@ -68,6 +72,7 @@ struct LzInst {
     cplx *rpart;          // small bases: per-vector-group partial updates of
                           // the Gram-Schmidt pass (ceil(lm / LZ_TG) x n), null
                           // for the single-pass update
+    cplx *HC2;            // short vectors: H.v output less its alpha part
     const int32_t *iperm; // sector-ordered basis: reference index of each row
                           // (the start vector is gathered through it and the
                           // Ritz vector scattered); null otherwise
@@ -100,6 +105,27 @@ __device__ inline void block_sum2(double a, double b, double *partial2)
     }
 }
 
+// sums of nb block partials, the same in every thread and block (fixed order)
+__device__ inline double2 sum_partials(const double *partial, int nb)
+{
+    __shared__ double red[2][LZ_T / 64];
+    double a = 0, b = 0;
+    for (int x = threadIdx.x; x < nb; x += LZ_T) {
+        const double2 p = *reinterpret_cast<const double2 *>(partial + 2 * x);
+        a += p.x;
+        b += p.y;
+    }
+    a = lz_wave_sum(a);
+    b = lz_wave_sum(b);
+    const int w = threadIdx.x >> 6;
+    __syncthreads();   // (an earlier call's sums are read)
+    if ((threadIdx.x & 63) == 0) { red[0][w] = a; red[1][w] = b; }
+    __syncthreads();
+    double2 s = {0, 0};
+    for (int x = 0; x < LZ_T / 64; x++) { s.x += red[0][x]; s.y += red[1][x]; }
+    return s;
+}
+
 // The descriptors hold generic pointers; vector accesses go through global
 // (address space 1) pointers and the per-step coefficients through constant
 // (address space 4) ones, so that the compiler emits global and scalar loads
@@ -130,6 +156,11 @@ __device__ inline cplx ldv_nt(const LZ_GLOBAL cplx *p)
     const lz_d2 t = __builtin_nontemporal_load((const LZ_GLOBAL lz_d2 *)p);
     return cmake(t.x, t.y);
 }
+template <bool NT>
+__device__ inline cplx ldv_as(const LZ_GLOBAL cplx *p)
+{
+    return NT ? ldv_nt(p) : ldv(p);
+}
 __device__ inline void stv(LZ_GLOBAL cplx *p, cplx z)
 {
     lz_d2 t;
@@ -156,6 +187,7 @@ __global__ void lz_init(LanczosState *sts, const LzInst *in, int lm, double tol)
     }
     if (threadIdx.x == 0) {
         st->it = 0;
+        st->it_next = 0;
         st->broke = 0;
         st->steps = lm;
         st->lm = lm;
@@ -196,22 +228,15 @@ __global__ __launch_bounds__(LZ_T) void lz_dot(const LzInst *in)
 
 // alpha from the block partials, into diag[0] (first) or diag[it + 1]
 // (grid (1, K))
-__global__ void lz_fin_alpha(LanczosState *sts, const LzInst *in, int first)
+__global__ __launch_bounds__(LZ_T) void lz_fin_alpha(LanczosState *sts, const LzInst *in, int first)
 {
-    __shared__ double red[2][LZ_T];
     LanczosState *st = sts + blockIdx.y;
     const LzInst &I = in[blockIdx.y];
     if (st->broke) return;
-    double re = 0, im = 0;
-    for (int x = threadIdx.x; x < I.nb; x += LZ_T) { re += I.partial[2 * x]; im += I.partial[2 * x + 1]; }
-    red[0][threadIdx.x] = re;
-    red[1][threadIdx.x] = im;
-    __syncthreads();
+    const double2 s = sum_partials(I.partial, I.nb);
     if (threadIdx.x == 0) {
-        double a = 0, b = 0;
-        for (int x = 0; x < LZ_T; x++) { a += red[0][x]; b += red[1][x]; }
-        st->alpha = cmake(a, b);
-        I.diag[first ? 0 : st->it + 1] = cmake(a, b);
+        st->alpha = cmake(s.x, s.y);
+        I.diag[first ? 0 : st->it + 1] = cmake(s.x, s.y);
     }
 }
 
@@ -236,41 +261,59 @@ __global__ __launch_bounds__(LZ_T) void lz_sub_alpha_norm(const LanczosState *st
 
 // ---- iteration kernels --
 
-// 1: beta_i and the breakdown test (groundStateLieb.c:287-292); grid (1, K)
-__global__ void lz_fin_beta(LanczosState *sts, const LzInst *in)
+// 1: beta_i and the breakdown test (groundStateLieb.c:287-292): every thread
+// of a block; one writes the state.  False on a breakdown (now or before).
+// Other blocks of the launch may see the state before or after that write:
+// max(maxb, beta) is the same either way, and a block that already sees a
+// breakdown has nothing left to do.
+__device__ inline bool begin_step(LanczosState *st, const LzInst &I, bool writer, double &beta)
 {
-    __shared__ double red[LZ_T];
-    LanczosState *st = sts + blockIdx.y;
-    const LzInst &I = in[blockIdx.y];
-    if (st->broke) return;
-    double s = 0;
-    for (int x = threadIdx.x; x < I.nb; x += LZ_T) s += I.partial[2 * x];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0;
-        for (int x = 0; x < LZ_T; x++) t += red[x];
-        double b = sqrt(t);
-        const int i = st->it;
+    const double b = sqrt(sum_partials(I.partial, I.nb).x);   // (barriers: before the state is read)
+    if (st->broke) return false;
+    const double mb = st->maxb;
+    const double maxb = b > mb ? b : mb;
+    const bool broke = b == 0.0 || b / maxb < st->tol;
+    beta = b;
+    if (writer) {
+        const int i = st->it_next;
+        st->it = i;
         I.offd[i] = cmake(b, 0);
-        if (b > st->maxb) st->maxb = b;
+        st->maxb = maxb;
         st->beta = b;
-        if (b == 0.0 || b / st->maxb < st->tol) {
+        if (broke) {
             // invariant Krylov space of dimension i+1: keep alpha_0..alpha_i
             st->broke = 1;
             st->steps = i + 1;
         }
     }
+    return !broke;
 }
 
-// 2: v_{i+1} = HC / beta_i, stored in lvec[i+1] and in the H.v input buffer
-__global__ __launch_bounds__(LZ_T) void lz_scale(const LanczosState *sts, const LzInst *in)
+// grid (1, K)
+__global__ __launch_bounds__(LZ_T) void lz_fin_beta(LanczosState *sts, const LzInst *in)
 {
-    const LanczosState *st = sts + blockIdx.y;
+    double beta;
+    begin_step(sts + blockIdx.y, in[blockIdx.y], threadIdx.x == 0, beta);
+}
+
+// 2: v_{i+1} = HC / beta_i, stored in lvec[i+1] and in the H.v input buffer;
+// INL: beta_i formed here (1 is no launch of its own)
+template <bool INL>
+__global__ __launch_bounds__(LZ_T) void lz_scale(LanczosState *sts, const LzInst *in)
+{
+    LanczosState *st = sts + blockIdx.y;
     const LzInst &I = in[blockIdx.y];
-    if ((int)blockIdx.x >= I.nb || st->broke) return;
-    const double inv = 1.0 / st->beta;
-    LZ_GLOBAL cplx *dst = gp(I.lvec) + (int64_t)(st->it + 1) * I.n;
+    if ((int)blockIdx.x >= I.nb) return;
+    double beta = 0;
+    const int i = INL ? st->it_next : st->it;
+    if (INL) {
+        if (!begin_step(st, I, blockIdx.x == 0 && threadIdx.x == 0, beta)) return;
+    } else {
+        if (st->broke) return;
+        beta = st->beta;
+    }
+    const double inv = 1.0 / beta;
+    LZ_GLOBAL cplx *dst = gp(I.lvec) + (int64_t)(i + 1) * I.n;
     LZ_ROWS(I, j)
     {
         cplx h = ldv(gp(I.HC) + j);
@@ -302,13 +345,19 @@ __global__ __launch_bounds__(LZ_T) void lz_sub_dot(const LanczosState *sts, cons
     block_sum2(re, im, I.partial);
 }
 
-// 6a: HC -= alpha v_{i+1}
-__global__ __launch_bounds__(LZ_T) void lz_sub_alpha(const LanczosState *sts, const LzInst *in)
+// 6a: HC -= alpha v_{i+1}; INL: alpha formed here (5 is no launch)
+template <bool INL>
+__global__ __launch_bounds__(LZ_T) void lz_sub_alpha(LanczosState *sts, const LzInst *in)
 {
-    const LanczosState *st = sts + blockIdx.y;
+    LanczosState *st = sts + blockIdx.y;
     const LzInst &I = in[blockIdx.y];
     if ((int)blockIdx.x >= I.nb || st->broke) return;
-    const cplx a = st->alpha;
+    cplx a = st->alpha;
+    if (INL) {
+        const double2 p = sum_partials(I.partial, I.nb);
+        a = cmake(p.x, p.y);
+        if (blockIdx.x == 0 && threadIdx.x == 0) I.diag[st->it + 1] = a;
+    }
     LZ_ROWS(I, j)
     {
         cplx x = ldv(gp(I.HC) + j), y = ldv(gp(I.vin) + j);
@@ -328,12 +377,20 @@ __global__ __launch_bounds__(LZ_T) void lz_sub_alpha(const LanczosState *sts, co
 // 5.6 / 5.1 / 4.7, 13.0 M rows 6.3 / 6.4 / 6.4; 352,716 rows 4.8 / 4.3
 // with 8 / 16.
 #define LZ_R 8
+// rows of a thread in the short-vector (FUSE) dots and update: smaller
+// segments give those chains blocks enough
+#define LZ_RF 4
+#define LZ_RP 2
 #define LZ_SEG ((int64_t)LZ_T * LZ_R)
 // vector groups of the split Gram-Schmidt update (small bases)
 #define LZ_TG 32
-template <int TG>
+// FUSE (short vectors): 5 and 6a here too, HC - alpha v_{i+1} formed in
+// registers by every block of a segment and stored, to HC2, by those of the
+// first vectors.
+template <int TG, bool FUSE, bool NT>
 __global__ __launch_bounds__(LZ_T) void lz_gemv_dots(const LanczosState *sts, const LzInst *in)
 {
+    constexpr int R = FUSE ? LZ_RF : LZ_R;   // rows of a thread
     __shared__ double red[TG][LZ_T / 64][2];
     const LanczosState *st = sts + blockIdx.z;
     const LzInst &I = in[blockIdx.z];
@@ -343,12 +400,30 @@ __global__ __launch_bounds__(LZ_T) void lz_gemv_dots(const LanczosState *sts, co
     if (t0 >= nt) return;
     const int t1 = min(nt, t0 + TG);
     const int64_t n = I.n;
-    const int64_t base = (int64_t)blockIdx.x * LZ_SEG + threadIdx.x;
-    cplx h[LZ_R];
+    const int64_t base = (int64_t)blockIdx.x * LZ_T * R + threadIdx.x;
+    cplx h[R];
 #pragma unroll
-    for (int r = 0; r < LZ_R; r++) {
+    for (int r = 0; r < R; r++) {
         int64_t j = base + (int64_t)r * LZ_T;
         h[r] = (j < n) ? ldv(gp(I.HC) + j) : cmake(0, 0);
+    }
+    if (FUSE) {
+        cplx y[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int64_t j = base + (int64_t)r * LZ_T;
+            y[r] = (j < n) ? ldv(gp(I.vin) + j) : cmake(0, 0);
+        }
+        const double2 a = sum_partials(I.partial, I.nb);
+        const bool first = blockIdx.y == 0;
+        if (first && blockIdx.x == 0 && threadIdx.x == 0) I.diag[st->it + 1] = cmake(a.x, a.y);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int64_t j = base + (int64_t)r * LZ_T;
+            h[r].re -= a.x * y[r].re - a.y * y[r].im;
+            h[r].im -= a.x * y[r].im + a.y * y[r].re;
+            if (first && j < n) stv(gp(I.HC2) + j, h[r]);
+        }
     }
     const int w = threadIdx.x >> 6;
     for (int tt = t0; tt < t1; tt++) {
@@ -359,10 +434,10 @@ __global__ __launch_bounds__(LZ_T) void lz_gemv_dots(const LanczosState *sts, co
         // ones keep the branch (the loads then wait one by one, which with
         // many resident waves measured faster: 13.0 M rows, 200 steps)
 #pragma unroll
-        for (int r = 0; r < LZ_R; r++) {
+        for (int r = 0; r < R; r++) {
             const int64_t j = base + (int64_t)r * LZ_T;
             if (TG == 8 || j < n) {
-                const cplx x = ldv_nt(vt + (j < n ? j : n - 1));
+                const cplx x = ldv_as<NT>(vt + (j < n ? j : n - 1));
                 re += x.re * h[r].re + x.im * h[r].im;
                 im += x.re * h[r].im - x.im * h[r].re;
             }
@@ -425,11 +500,12 @@ __global__ __launch_bounds__(LZ_T) void lz_fin_ortho(const LanczosState *sts, co
 // is 4, or 2 when the chain's instances have too few rows for 4 to fill
 // the device (update_rows).
 template <int RR>
-__global__ __launch_bounds__(LZ_T) void lz_reorth_norm(const LanczosState *sts, const LzInst *in)
+__global__ __launch_bounds__(LZ_T) void lz_reorth_norm(LanczosState *sts, const LzInst *in)
 {
-    const LanczosState *st = sts + blockIdx.y;
+    LanczosState *st = sts + blockIdx.y;
     const LzInst &I = in[blockIdx.y];
     if ((int)blockIdx.x >= I.nb || st->broke || I.rpart) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->it_next = st->it + 1;   // the step's last kernel
     const int nt = st->it + 2;
     const int64_t n = I.n;
     const LZ_CONST cplx *o = kp(I.ortho);
@@ -479,51 +555,80 @@ __global__ __launch_bounds__(LZ_T) void lz_reorth_norm(const LanczosState *sts, 
 // like the dots: block (s, g, instance) sums v_t o_t over the vector group g
 // for the rows of segment s into rpart[g] (8a), then one pass subtracts the
 // groups' partial sums from HC and forms the norm partials (8b).
+// FUSE (short vectors): 7 here too, each block forming the o_t of its group
+// (eight lanes a vector).
+template <bool FUSE, bool NT>
 __global__ __launch_bounds__(LZ_T) void lz_reorth_part(const LanczosState *sts, const LzInst *in)
 {
+    constexpr int R = FUSE ? LZ_RP : LZ_R;   // rows of a thread
+    __shared__ cplx so[LZ_TG];
     const LanczosState *st = sts + blockIdx.z;
     const LzInst &I = in[blockIdx.z];
-    if (!I.rpart || (int)blockIdx.x >= I.nbg || st->broke) return;
+    if (!I.rpart || (int)blockIdx.x >= (FUSE ? I.nb : I.nbg) || st->broke) return;
     const int nt = st->it + 2;
     const int t0 = blockIdx.y * LZ_TG;
     if (t0 >= nt) return;
     const int t1 = min(nt, t0 + LZ_TG);
     const int64_t n = I.n;
-    const int64_t base = (int64_t)blockIdx.x * LZ_SEG + threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * LZ_T * R + threadIdx.x;
     const LZ_CONST cplx *o = kp(I.ortho);
-    cplx p[LZ_R];
+    if (FUSE) {
+        const int t = threadIdx.x / 8, l = threadIdx.x % 8;
+        static_assert(LZ_T / 8 == LZ_TG, "eight lanes a vector");
+        double re = 0, im = 0;
+        if (t0 + t < t1) {
+            const double2 *q = reinterpret_cast<const double2 *>(I.partial_o) + (int64_t)(t0 + t) * I.nbg;
+            for (int x = l; x < I.nbg; x += 8) {
+                const double2 z = q[x];
+                re += z.x;
+                im += z.y;
+            }
+        }
+        for (int k = 4; k > 0; k >>= 1) {
+            re += __shfl_xor(re, k, 64);
+            im += __shfl_xor(im, k, 64);
+        }
+        if (l == 0) so[t] = cmake(re, im);
+        __syncthreads();
+    }
+    cplx p[R];
 #pragma unroll
-    for (int r = 0; r < LZ_R; r++) p[r] = cmake(0, 0);
+    for (int r = 0; r < R; r++) p[r] = cmake(0, 0);
+    constexpr int UN = FUSE ? 4 : 1;
+#pragma unroll UN
     for (int tt = t0; tt < t1; tt++) {
-        const cplx ot = cmake(o[tt].re, o[tt].im);
+        const cplx ot = FUSE ? so[tt - t0] : cmake(o[tt].re, o[tt].im);
         const LZ_GLOBAL cplx *vt = gp(I.lvec) + (int64_t)tt * n;
 #pragma unroll
-        for (int r = 0; r < LZ_R; r++) {   // rows past n: row n - 1, never stored
+        for (int r = 0; r < R; r++) {   // rows past n: row n - 1, never stored
             const int64_t j = base + (int64_t)r * LZ_T;
-            const cplx x = ldv_nt(vt + (j < n ? j : n - 1));
+            const cplx x = ldv_as<NT>(vt + (j < n ? j : n - 1));
             p[r].re += x.re * ot.re - x.im * ot.im;
             p[r].im += x.re * ot.im + x.im * ot.re;
         }
     }
     LZ_GLOBAL cplx *dst = gp(I.rpart) + (int64_t)blockIdx.y * n;
 #pragma unroll
-    for (int r = 0; r < LZ_R; r++) {
+    for (int r = 0; r < R; r++) {
         const int64_t j = base + (int64_t)r * LZ_T;
         if (j < n) stv(dst + j, p[r]);
     }
 }
 
-__global__ __launch_bounds__(LZ_T) void lz_reorth_sum(const LanczosState *sts, const LzInst *in)
+// FUSE: from HC2
+template <bool FUSE>
+__global__ __launch_bounds__(LZ_T) void lz_reorth_sum(LanczosState *sts, const LzInst *in)
 {
-    const LanczosState *st = sts + blockIdx.y;
+    LanczosState *st = sts + blockIdx.y;
     const LzInst &I = in[blockIdx.y];
     if (!I.rpart || (int)blockIdx.x >= I.nb || st->broke) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->it_next = st->it + 1;   // the step's last kernel
     const int ng = (st->it + 2 + LZ_TG - 1) / LZ_TG;
     const int64_t n = I.n;
     double s = 0;
     LZ_ROWS(I, j)
     {
-        cplx h = ldv(gp(I.HC) + j);
+        cplx h = ldv(gp(FUSE ? I.HC2 : I.HC) + j);
         for (int g = 0; g < ng; g++) {
             const cplx x = ldv(gp(I.rpart) + (int64_t)g * n + j);
             h.re -= x.re;
@@ -533,13 +638,6 @@ __global__ __launch_bounds__(LZ_T) void lz_reorth_sum(const LanczosState *sts, c
         s += h.re * h.re + h.im * h.im;
     }
     block_sum2(s, 0, I.partial);
-}
-
-// 9: one thread per instance
-__global__ void lz_advance(LanczosState *sts, int K)
-{
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x < K && !sts[x].broke) sts[x].it += 1;
 }
 
 // Ritz vector C = sum_k lvec[k] z[k]  (groundStateLieb.c:454-458); z read
@@ -703,8 +801,8 @@ static int64_t row_blocks(int64_t n, int rr)
 
 // the Gram-Schmidt update of an instance with fewer than 256 blocks of 4
 // rows per thread is split over vector groups (lz_reorth_part /
-// lz_reorth_sum) when there are more vectors than one group
-static bool split_update(int64_t n, int lm) { return row_blocks(n, 4) < 256 && lm > LZ_TG; }
+// lz_reorth_sum)
+static bool split_update(int64_t n) { return row_blocks(n, 4) < 256; }
 
 // rows per thread of the single-pass update for a chain of instances: 2
 // when 4 leave fewer than 1024 blocks in all (4 per CU), else 4.  Measured
@@ -727,6 +825,26 @@ static int dot_group(const std::vector<int64_t> &ns)
     for (int64_t n : ns) sg += (n + LZ_SEG - 1) / LZ_SEG;
     return sg < 4096 ? 8 : 16;
 }
+
+// What the kernels of a chain do beside their own work.  Forming the sums of
+// block partials in every block that needs them takes less than a launch of
+// its own (about 4.5 us a step each) up to 2^20 partials in all (1024 blocks of
+// one instance, 16 MB from the L2s); the 64-instance call, with ten times as
+// many, loses 15 us a step to them.  Where every instance has the split update
+// (vectors of up to 262,144 entries, at most 128 segments), the alpha part and
+// the o_t are formed where they are used too.  Basis vectors that the Infinity
+// Cache can hold for the most part (512 MB at the last step) are read with
+// plain loads, larger ones pass it by.  Measured, us a step (before; with inl
+// only; now): N = 6, M = 9, 120 steps 68, 52, 43; N = 8, M = 11 100, 80, 63; N =
+// 5, M = 21, 400 steps 192, 126, 116; N = 10, M = 11 154, 130, 125; N = 5, M =
+// 21, 1500 steps 352, 282, 288.
+struct LzChain {
+    bool inl = true;     // 1 and 5 inside 2 and 6
+    bool fuse = true;    // 5, 6a inside 6b and 7 inside 8
+    bool cached = true;  // (fuse) basis vectors read with plain loads
+    bool split = false;  // an instance has the split update
+    bool whole = false;  // an instance has the single-pass update
+};
 
 // One device allocation carved into aligned pieces.
 struct Arena {
@@ -1113,12 +1231,26 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
     std::vector<int64_t> ns(K);
     for (int x = 0; x < K; x++) ns[x] = hams[x]->basis->d.nc;
     const int rr = update_rows(ns), dtg = dot_group(ns);
+    LzChain ch;
+    int64_t vbytes = 0, reads = 0;   // partials read by all blocks of a kernel
+    for (int64_t n : ns) {
+        const bool sp = split_update(n);
+        ch.split = ch.split || sp;
+        ch.whole = ch.whole || !sp;
+        reads += row_blocks(n, rr) * row_blocks(n, rr);
+        ch.fuse = ch.fuse && sp;
+        vbytes += (int64_t)sizeof(cplx) * n * lm;
+    }
+    ch.inl = reads <= (int64_t)1 << 20;
+    ch.fuse = ch.fuse && ch.inl && dtg == 8;
+    ch.cached = vbytes <= (int64_t)512 << 20;
     for (int x = 0; x < K; x++) {
         const int64_t n = ns[x];
         LzInst &I = hin[x];
         I.n = n;
         I.nb = (int)row_blocks(n, rr);
-        I.nbg = (int)((n + LZ_SEG - 1) / LZ_SEG);
+        const int64_t seg = ch.fuse ? LZ_T * LZ_RF : LZ_SEG;
+        I.nbg = (int)((n + seg - 1) / seg);
         nbmax = std::max(nbmax, I.nb);
         nbgmax = std::max(nbgmax, I.nbg);
         if (!(lvec_ext && lvec_ext[x])) A.reserve(sizeof(cplx) * n * (size_t)lm);
@@ -1128,7 +1260,8 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
         A.reserve(sizeof(double) * 2 * I.nb);
         A.reserve(sizeof(double) * 2 * (size_t)I.nbg * lm);
         A.reserve(sizeof(double) * lm);
-        if (split_update(n, lm)) A.reserve(sizeof(cplx) * n * (size_t)((lm + LZ_TG - 1) / LZ_TG));
+        if (split_update(n)) A.reserve(sizeof(cplx) * n * (size_t)((lm + LZ_TG - 1) / LZ_TG));
+        if (ch.fuse) A.reserve(sizeof(cplx) * n);
     }
     for (HvGroup &g : groups) {
         if (!g.batched) continue;
@@ -1138,7 +1271,6 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
         if (g.pzmv_ok) A.reserve(pairz_multi_bytes(g, hams));
     }
     MCPI_CHECK(A.allocate());
-    bool any_split = false;
     LanczosState *sts = A.take<LanczosState>(K);
     LzInst *din = A.take<LzInst>(K);
     for (HvGroup &g : groups) {
@@ -1174,8 +1306,8 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
         I.partial_o = A.take<double>(2 * (size_t)I.nbg * lm);
         double *z = A.take<double>(lm);
         I.z = z;
-        I.rpart = split_update(n, lm) ? A.take<cplx>(n * (size_t)((lm + LZ_TG - 1) / LZ_TG)) : nullptr;
-        any_split = any_split || I.rpart != nullptr;
+        I.rpart = split_update(n) ? A.take<cplx>(n * (size_t)((lm + LZ_TG - 1) / LZ_TG)) : nullptr;
+        I.HC2 = ch.fuse ? A.take<cplx>(n) : nullptr;
         I.Cout = (Cout && Cout[x]) ? Cout[x] : nullptr;
         I.iperm = hams[x]->basis->iperm;
         I.steps = 0;
@@ -1203,9 +1335,8 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
     MCPI_HIP(hipMemcpyAsync(din, hin.data(), sizeof(LzInst) * K, hipMemcpyHostToDevice, s));
 
     const dim3 blk(LZ_T), gv(nbmax, K), g1(1, K);
-    const dim3 gd(nbgmax, (lm + dtg - 1) / dtg, K), gpart(nbgmax, (lm + LZ_TG - 1) / LZ_TG, K);
+    const dim3 gd(nbgmax, (lm + dtg - 1) / dtg, K), gpart(ch.fuse ? nbmax : nbgmax, (lm + LZ_TG - 1) / LZ_TG, K);
     const dim3 go(lm, K);
-    const int ga = (K + 63) / 64;
 
     // ---- set-up: v_0, schedules, HC = H v_0, alpha_0, HC -= alpha_0 v_0
     hipLaunchKernelGGL(lz_init, g1, dim3(64), 0, s, sts, (const LzInst *)din, lm, 1e-15);
@@ -1226,26 +1357,47 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
         const LanczosState *cst = sts;
         const LzInst *cin = din;
         auto enqueue = [&]() -> mcpi_status {
-            hipLaunchKernelGGL(lz_fin_beta, g1, blk, 0, s, sts, cin);
-            hipLaunchKernelGGL(lz_scale, gv, blk, 0, s, cst, cin);
+            if (ch.inl) {
+                hipLaunchKernelGGL(lz_scale<true>, gv, blk, 0, s, sts, cin);
+            } else {
+                hipLaunchKernelGGL(lz_fin_beta, g1, blk, 0, s, sts, cin);
+                hipLaunchKernelGGL(lz_scale<false>, gv, blk, 0, s, sts, cin);
+            }
             for (const HvGroup &g : groups) MCPI_CHECK(launch_group(g, hams, hin, s));
             hipLaunchKernelGGL(lz_sub_dot, gv, blk, 0, s, cst, cin);
-            hipLaunchKernelGGL(lz_fin_alpha, g1, blk, 0, s, sts, cin, 0);
-            hipLaunchKernelGGL(lz_sub_alpha, gv, blk, 0, s, cst, cin);
-            if (dtg == 8)
-                hipLaunchKernelGGL(lz_gemv_dots<8>, gd, blk, 0, s, cst, cin);
-            else
-                hipLaunchKernelGGL(lz_gemv_dots<16>, gd, blk, 0, s, cst, cin);
-            hipLaunchKernelGGL(lz_fin_ortho, go, blk, 0, s, cst, cin);
-            if (rr == 2)
-                hipLaunchKernelGGL(lz_reorth_norm<2>, gv, blk, 0, s, cst, cin);
-            else
-                hipLaunchKernelGGL(lz_reorth_norm<4>, gv, blk, 0, s, cst, cin);
-            if (any_split) {
-                hipLaunchKernelGGL(lz_reorth_part, gpart, blk, 0, s, cst, cin);
-                hipLaunchKernelGGL(lz_reorth_sum, gv, blk, 0, s, cst, cin);
+            if (ch.fuse) {
+                if (ch.cached) {
+                    hipLaunchKernelGGL((lz_gemv_dots<8, true, false>), gd, blk, 0, s, cst, cin);
+                    hipLaunchKernelGGL((lz_reorth_part<true, false>), gpart, blk, 0, s, cst, cin);
+                } else {
+                    hipLaunchKernelGGL((lz_gemv_dots<8, true, true>), gd, blk, 0, s, cst, cin);
+                    hipLaunchKernelGGL((lz_reorth_part<true, true>), gpart, blk, 0, s, cst, cin);
+                }
+                hipLaunchKernelGGL(lz_reorth_sum<true>, gv, blk, 0, s, sts, cin);
+                MCPI_HIP(hipGetLastError());
+                return MCPI_OK;
             }
-            hipLaunchKernelGGL(lz_advance, dim3(ga), dim3(64), 0, s, sts, K);
+            if (ch.inl) {
+                hipLaunchKernelGGL(lz_sub_alpha<true>, gv, blk, 0, s, sts, cin);
+            } else {
+                hipLaunchKernelGGL(lz_fin_alpha, g1, blk, 0, s, sts, cin, 0);
+                hipLaunchKernelGGL(lz_sub_alpha<false>, gv, blk, 0, s, sts, cin);
+            }
+            if (dtg == 8)
+                hipLaunchKernelGGL((lz_gemv_dots<8, false, true>), gd, blk, 0, s, cst, cin);
+            else
+                hipLaunchKernelGGL((lz_gemv_dots<16, false, true>), gd, blk, 0, s, cst, cin);
+            hipLaunchKernelGGL(lz_fin_ortho, go, blk, 0, s, cst, cin);
+            if (ch.whole) {
+                if (rr == 2)
+                    hipLaunchKernelGGL(lz_reorth_norm<2>, gv, blk, 0, s, sts, cin);
+                else
+                    hipLaunchKernelGGL(lz_reorth_norm<4>, gv, blk, 0, s, sts, cin);
+            }
+            if (ch.split) {
+                hipLaunchKernelGGL((lz_reorth_part<false, true>), gpart, blk, 0, s, cst, cin);
+                hipLaunchKernelGGL(lz_reorth_sum<false>, gv, blk, 0, s, sts, cin);
+            }
             MCPI_HIP(hipGetLastError());
             return MCPI_OK;
         };
