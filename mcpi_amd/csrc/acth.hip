@@ -219,6 +219,35 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
             zoff = std::move(pf.zoff);
         }
     }
+    // blocks of one pair: a*_q a*_l a_q a_l is diagonal, so they need neither
+    // of the two passes (Lieb-Liniger: the two lowest and the two highest
+    // total momenta)
+    std::vector<PairDiag> zdiag;
+    if (zoff.size() > 1) {
+        const int R = (int)zoff.size() - 1;
+        int many = 0;
+        for (int r = 0; r < R; r++) many += zoff[r + 1] - zoff[r] > 1;
+        if (many > 0 && many < R) {
+            std::vector<int32_t> ord, off(1, 0);
+            for (int r = 0; r < R; r++) {
+                if (zoff[r + 1] - zoff[r] > 1) {
+                    for (int j = zoff[r]; j < zoff[r + 1]; j++) {
+                        ord.push_back(zord[j]);
+                        zblk[zord[j]] = (int32_t)off.size() - 1;
+                    }
+                    off.push_back((int32_t)ord.size());
+                } else {
+                    const int P = zord[zoff[r]], l = pair_hi(P);
+                    cplx w = cmake(0, 0);
+                    w = cfma(za[P], zb[P], w);
+                    zdiag.push_back({w.re, w.im, P - l * (l + 1) / 2, l});
+                    zblk[P] = -1;
+                }
+            }
+            zord = std::move(ord);
+            zoff = std::move(off);
+        }
+    }
     auto offsets = [](int x) {
         const int l = pair_hi(x), q = x - l * (l + 1) / 2;
         return PairOff{q * PAIR_ORB, l * PAIR_ORB, q == l ? PAIR_SLOT : 0, 0};
@@ -246,7 +275,8 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
                 otc.size() + ttc.size() + pw.size() + ph1.size() + pwf.size() + za.size() + zb.size();
     size_t nB = nz1.size() + nzo.size() + nzt.size() + 4 * (m1j.size() + ot_off.size() + tt_off.size() +
                                                            nz_e.size() + zblk.size() + zord.size() + zoff.size()) +
-                zrec.size() * sizeof(PairRec) + zrun.size() * sizeof(PairRun) + pql.size() * sizeof(PairOff) + 64;
+                zrec.size() * sizeof(PairRec) + zrun.size() * sizeof(PairRun) +
+                zdiag.size() * sizeof(PairDiag) + pql.size() * sizeof(PairOff) + 64;
     size_t bytes = (nC * sizeof(cplx) + nB + 64 + 255) & ~(size_t)255;
     char *dev = nullptr;
     MCPI_HIP(hipMalloc(&dev, bytes));
@@ -269,6 +299,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     const size_t o_za = za.empty() ? 0 : put(za.data(), za.size() * sizeof(cplx));
     const size_t o_zb = zb.empty() ? 0 : put(zb.data(), zb.size() * sizeof(cplx));
     const size_t o_zrec = zblk.empty() ? 0 : put(zrec.data(), zrec.size() * sizeof(PairRec));
+    const size_t o_zdiag = put(zdiag.data(), zdiag.size() * sizeof(PairDiag));
     const size_t o_zrun = zblk.empty() ? 0 : put(zrun.data(), zrun.size() * sizeof(PairRun));
     const size_t o_pql = pql.empty() ? 0 : put(pql.data(), pql.size() * sizeof(PairOff));
     size_t o_m1 = put(m1j.data(), m1j.size() * 4);
@@ -306,6 +337,8 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     c->pzoff = fac ? (int32_t *)(dev + o_zoff) : nullptr;
     c->pzrec = fac ? (PairRec *)(dev + o_zrec) : nullptr;
     c->pzrun = fac ? (PairRun *)(dev + o_zrun) : nullptr;
+    c->pzdiag = (PairDiag *)(dev + o_zdiag);
+    c->pznd = (int)zdiag.size();
     c->pzR = fac ? (int)zoff.size() - 1 : 0;
     c->pql = pair ? (PairOff *)(dev + o_pql) : nullptr;
     c->nz_1j = (uint8_t *)(dev + o_n1);

@@ -545,7 +545,8 @@ __global__ __launch_bounds__(64 * PAIR_MUL_WAVES) void k_pair_mul(PairArgs a)
 
 // out[v] = sum_k sqrt(v_k) Y1[k][rank'(v - e_k)] + sum_P f_P(v) Y2[P][rank''(v - e_P)];
 // FAC (factorized pair form, Y2 = Z with one row per block):
-// out[v] = (sum_k h1[k][k] v_k) C[v] + sum_P f_P(v) za[P] Z[zblk[P]][rank''(v - e_P)]
+// out[v] = (sum_k h1[k][k] v_k + sum_diag w v_q (v_l - [q = l])) C[v]
+//          + sum_P f_P(v) za[P] Z[zblk[P]][rank''(v - e_P)]
 // RC (FAC only): za is real.  MV > 1 (FAC only): MV members that share the
 // basis, zb and the blocks (a group of Lieb-Liniger couplings): the row's
 // occupations, prefix sums, pair offsets and factors serve every member;
@@ -575,6 +576,8 @@ struct PairOutArgs {
     const cplx *Y1, *Y2, *za;
     const int32_t *zblk;
     const cplx *h1, *C;
+    const PairDiag *diag;   // pairs that are a block by themselves
+    int nd;
     cplx *out;
     int64_t mC, mZ, mK;
     int S;   // wavefronts that share a row's pairs: 1, 2 or 4
@@ -604,6 +607,8 @@ k_pair_out(PairOutArgs a)
     typedef const __attribute__((address_space(4))) cplx *kcplx;
     const kchar za = (kchar)((const char *)a.za + m0 * a.mK), h1 = (kchar)((const char *)a.h1 + m0 * a.mK);
     const auto zblk = kptr(a.zblk);
+    typedef const __attribute__((address_space(4))) PairDiag *kdiag;
+    const kchar dgp = (kchar)((const char *)a.diag + m0 * a.mK);
     // occupations, a byte each (v(k)): the registers go to the gathers
     uint64_t pk[(M + 7) / 8];
 #pragma unroll
@@ -611,6 +616,13 @@ k_pair_out(PairOutArgs a)
 #pragma unroll
     for (int k = 0; k < M; k++) pk[k / 8] |= (uint64_t)a.IF[i * M + k] << (8 * (k % 8));
     auto v = [&](int k) { return (int)((uint32_t)(pk[k / 8] >> (8 * (k % 8))) & 255u); };
+    // the same for a run-time (uniform) orbital
+    auto vrt = [&](int k) {
+        uint64_t w = pk[0];
+#pragma unroll
+        for (int x = 1; x < (M + 7) / 8; x++) w = k >= 8 * x ? pk[x] : w;
+        return (int)((uint32_t)(w >> (8 * (k & 7))) & 255u);
+    };
     // D1[o] = S_0(o) - S_1(o), D2[o] = S_1(o) - S_2(o) of S_d(x) = sum_{j=1..x}
     // B[j][P_j - d] (P_j: particles below orbital j), modulo 2^32 (every rank
     // is below 2^31)
@@ -660,6 +672,13 @@ k_pair_out(PairOutArgs a)
                 const int x = k * (pair_h1_stride(M) + 1);
                 d.re = fma(h[x].re, (double)v(k), d.re);
                 if (!RC) d.im = fma(h[x].im, (double)v(k), d.im);
+            }
+            const kdiag dg = (kdiag)(dgp + m * a.mK);
+            for (int x = 0; x < a.nd; x++) {
+                const int q = dg[x].q, l = dg[x].l;
+                const double w = (double)(vrt(q) * (vrt(l) - (q == l)));
+                d.re = fma(dg[x].wr, w, d.re);
+                if (!RC) d.im = fma(dg[x].wi, w, d.im);
             }
             const cplx c = ldcp(C + m * a.mC + i);
             acc[m] = RC ? cscale(c, d.re) : cfma(d, c, acc[m]);
@@ -923,6 +942,8 @@ mcpi_status launch_pairz_m(const BasisDev &b, const HamCoefDev &c, int chunks, c
     o.za = c.pza;
     o.zblk = c.pzblk;
     o.h1 = c.ph1;
+    o.diag = c.pzdiag;
+    o.nd = c.pznd;
     o.C = C;
     o.out = out;
     o.mC = mC;

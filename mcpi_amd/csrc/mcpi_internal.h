@@ -211,6 +211,11 @@ struct PairRec {
     int32_t oq, ol, e, last;
 };
 
+// a pair q <= l that is a block by itself: the diagonal term w v_q (v_l - [q = l])
+struct PairDiag {
+    double wr, wi;
+    int32_t q, l;
+};
 struct PairRun {
     int32_t r, j;
 };
@@ -260,7 +265,9 @@ struct HamCoefDev {
     // factorized pair form (schedule 7; null / 0 unless h1 is diagonal and
     // pw is block diagonal with rank-one blocks): pw[P][Q] = pza[P] pzb[Q]
     // for P, Q in one block; pzblk[P] = block of P (-1: none); pzord lists
-    // the pairs of block r at pzoff[r] .. pzoff[r+1]; pzR blocks
+    // the pairs of block r at pzoff[r] .. pzoff[r+1]; pzR blocks.  Blocks of
+    // one pair are diagonal terms and listed apart (pznd in pzdiag), unless
+    // there is no other block
     cplx *pza;
     cplx *pzb;
     int32_t *pzblk;
@@ -270,6 +277,8 @@ struct HamCoefDev {
     PairRun *pzrun;  // the blocks cut into 4 g runs, g = 1 .. PAIR_RUNS, at
                      // pair_run(g): run w is blocks [w].r .. [w + 1].r, which
                      // start at pairs [w].j
+    PairDiag *pzdiag;
+    int pznd;
     int pzR;
     PairOff *pql;    // pairs P (with pw; null otherwise)
     int real;        // 1 if every coefficient above has a zero imaginary part
@@ -312,6 +321,7 @@ __host__ __device__ inline HamCoefDev shift_coef(HamCoefDev c, ptrdiff_t d)
         c.pzoff = sh(c.pzoff);
         c.pzrec = sh(c.pzrec);
         c.pzrun = sh(c.pzrun);
+        c.pzdiag = sh(c.pzdiag);
     }
     if (c.pql) c.pql = sh(c.pql);
     return c;
