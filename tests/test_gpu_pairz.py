@@ -67,3 +67,34 @@ def test_disguised_members(oracle_lib, N, M):
         # twelve steps of a start in every sector: rounding of 1e-16 grows with
         # the norm of H (about 1e4) only
         assert abs(E[x] - E_o) <= 1e-11 * max(1.0, np.abs(Ho).max() * N), (x, E[x], E_o)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (1, 2), (1, 1, 1, 3), (1, 9), (1, 1, 6, 1)])
+@pytest.mark.parametrize("N,M", [(2, 3), (5, 5), (3, 11), (4, 18)])
+def test_single_pair_blocks(oracle_lib, N, M, sizes):
+    """Blocks of one pair beside larger ones, only blocks of one pair, and
+    pairs in no block: Hermitian rank-one blocks over a random order of the
+    pairs, zero on the rest."""
+    note(f"pairz single pairs N={N} M={M} sizes={sizes}")
+    rng = np.random.default_rng(100 * N + M + len(sizes))
+    pairs = [(q, l) for l in range(M) for q in range(l + 1)]
+    order = list(rng.permutation(len(pairs)))
+    Hint = np.zeros((M,) * 4, complex)
+    while order:
+        for s in sizes:
+            blk, order = [pairs[x] for x in order[:s]], order[s:]
+            if rng.random() < 0.2:
+                continue
+            a = rng.standard_normal(len(blk)) + 1j * rng.standard_normal(len(blk))
+            w = rng.choice([-1.0, 1.0])
+            for x, (k, s2) in enumerate(blk):
+                for y, (q, l) in enumerate(blk):
+                    for kk, ss in {(k, s2), (s2, k)}:
+                        for qq, ll in {(q, l), (l, q)}:
+                            Hint[kk, ss, qq, ll] = w * a[x] * np.conj(a[y])
+    Ho = np.diag(rng.standard_normal(M)).astype(complex)
+    o = oracle.Basis(N, M)
+    C, _, _ = oracle.random_inputs(N, M, seed=3)
+    b = mcpi_amd.Basis(N, M, "single")
+    H = mcpi_amd.Hamiltonian(b, Ho, Hint, schedule=7)
+    assert_close(H(C), o.acth(C, Ho, Hint), 1e-12, "schedule 7")
