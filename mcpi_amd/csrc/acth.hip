@@ -272,7 +272,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
         for (int x = 0; x < pair_count(M); x++) pql.push_back(offsets(x));
     // one device block: complex tables first (16-byte aligned), then integers
     size_t nC = dk.size() + d1.size() + d2.size() + A0.size() + A.size() + ot.size() + tt.size() + nz_c.size() +
-                otc.size() + ttc.size() + pw.size() + ph1.size() + pwf.size() + za.size() + zb.size();
+                otc.size() + ttc.size() + ph1.size() + pwf.size() + za.size() + zb.size();
     size_t nB = nz1.size() + nzo.size() + nzt.size() + 4 * (m1j.size() + ot_off.size() + tt_off.size() +
                                                            nz_e.size() + zblk.size() + zord.size() + zoff.size()) +
                 zrec.size() * sizeof(PairRec) + zrun.size() * sizeof(PairRun) +
@@ -293,7 +293,6 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     size_t o_nc = put(nz_c.data(), nz_c.size() * sizeof(cplx));
     size_t o_otc = put(otc.data(), otc.size() * sizeof(cplx));
     size_t o_ttc = put(ttc.data(), ttc.size() * sizeof(cplx));
-    const size_t o_pw = pw.empty() ? 0 : put(pw.data(), pw.size() * sizeof(cplx));
     const size_t o_ph1 = ph1.empty() ? 0 : put(ph1.data(), ph1.size() * sizeof(cplx));
     const size_t o_pwf = pwf.empty() ? 0 : put(pwf.data(), pwf.size() * sizeof(cplx));
     const size_t o_za = za.empty() ? 0 : put(za.data(), za.size() * sizeof(cplx));
@@ -326,7 +325,6 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     c->tt = (cplx *)(dev + o_tt);
     c->otc = (cplx *)(dev + o_otc);
     c->ttc = (cplx *)(dev + o_ttc);
-    c->pw = pair ? (cplx *)(dev + o_pw) : nullptr;
     c->ph1 = pair ? (cplx *)(dev + o_ph1) : nullptr;
     c->pwf = pwf.empty() ? nullptr : (cplx *)(dev + o_pwf);
     const bool fac = !zblk.empty();

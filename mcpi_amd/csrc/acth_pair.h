@@ -298,11 +298,11 @@ __device__ inline uint32_t pair_target(const unsigned char *tab, int oq, int ol,
 // gather.  What bounds it is the L2: neighbouring tiles gather from
 // neighbouring parts of C, so chunks of them go to one XCD each.
 // Measured (before: rows unranked in the kernel, two pairs in flight, tiles
-// dealt out one by one): N = 12, M = 12 88 -> 44 us; N = 16, M = 12 1220 -> 730
-// us (chunks of 128 tiles; single tiles 820); 24 members of N = 10, M = 13, four
-// at a time, 688 -> 567 us (chunks of 32 tiles, whose part of four C vectors an
-// L2 holds; 128: 770 with batches of four); N = 5, M = 21 60 -> 6 us (eleven
-// runs of 28 tiles).
+// dealt out one by one; blocks of one pair included): N = 12, M = 12 88 -> 38
+// us, 11 TB/s of gathered entries; N = 16, M = 12 1220 -> 630 us (chunks of 128
+// tiles; single tiles 14 % more); 24 members of N = 10, M = 13, four at a time,
+// 688 -> 530 us (chunks of 32 tiles, whose part of four C vectors an L2 holds;
+// 128 tiles 36 % more); N = 5, M = 21 60 -> 6 us (eleven runs of 28 tiles).
 template <int NW, int MV, bool RC>
 __global__ __launch_bounds__(PT) void k_pairz_amp(PairArgs a, int M)
 {
@@ -565,9 +565,11 @@ __global__ __launch_bounds__(64 * PAIR_MUL_WAVES) void k_pair_mul(PairArgs a)
 // check turns into a zero without a memory access: no branch between the
 // loads of a batch.  Occupations stay packed, a byte each, and the roots in
 // LDS: registers are wavefronts, which hide the gathers.  Measured (before: all
-// pairs, in batches of 13): N = 12, M = 12 88 -> 71 us, N = 16, M = 12 970 -> 830
-// us (then bound by the 5.9 GB that the L2s miss), 24 members of N = 10, M = 13,
-// four at a time, 918 -> 705 us.
+// pairs, in batches of 13): N = 12, M = 12 88 -> 68 us, N = 16, M = 12 970 -> 780
+// us (then bound by the nearly 6 GB that the L2s miss: the rows that read one
+// entry of Z lie far apart), 24 members of N = 10, M = 13, four at a time, 918 ->
+// 675 us.  Slower: each lane walking the pairs its own row has, through tables
+// in LDS (N = 12 110 us, N = 16 1310 us, N = 5, M = 21 18 us as here).
 struct PairOutArgs {
     int N;
     int64_t nc;

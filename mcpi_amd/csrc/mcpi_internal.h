@@ -249,21 +249,19 @@ struct HamCoefDev {
     int32_t *tt_off; // P+1: same for TT chunk p
     int32_t *nz_e;   // entry index q + l*M of each listed term
     cplx *nz_c;      // its folded coefficient
-    // The same operator through the pair space (schedule 6, 3 <= M <= 12;
-    // null otherwise): H = sum_{k,l} h1[k][l] a*_k a_l
-    //                    + sum_{P,Q} pw[P][Q] a*_{P1} a*_{P2} a_{Q1} a_{Q2}
-    // over unordered orbital pairs P, Q (index p = hi(hi+1)/2 + lo), stored
-    // pw[Q * PWS + P] and ph1[l * HS + k], HS = pair_h1_stride(M) (column of an annihilated pair or
-    // orbital contiguous, PWS = M(M+1)/2 rounded up to 16, zero padded)
-    cplx *pw;
+    // The same operator through the pair space (null where it does not
+    // apply): H = sum_{k,l} h1[k][l] a*_k a_l
+    //             + sum_{P,Q} w[P][Q] a*_{P1} a*_{P2} a_{Q1} a_{Q2}
+    // over unordered orbital pairs P, Q (index p = hi(hi+1)/2 + lo); h1 is
+    // stored ph1[l * HS + k], HS = pair_h1_stride(M)
     cplx *ph1;
-    // pw with the one-body part folded in for N >= 2 particles (a*_k a_l =
+    // w with the one-body part folded in for N >= 2 particles (a*_k a_l =
     // sum_s a*_k a*_s a_s a_l / (N - 1)), as the fragments of the pair product:
-    // [s][g][lane] = W[16 g + lane % 16][4 s + lane / 16], zero past the pairs
+    // [s][g][lane] = w[16 g + lane % 16][4 s + lane / 16], zero past the pairs
     // (M <= MCPI_PAIR_MAXM and N given to build_coefficients; null otherwise)
     cplx *pwf;
     // factorized pair form (schedule 7; null / 0 unless h1 is diagonal and
-    // pw is block diagonal with rank-one blocks): pw[P][Q] = pza[P] pzb[Q]
+    // w is block diagonal with rank-one blocks): w[P][Q] = pza[P] pzb[Q]
     // for P, Q in one block; pzblk[P] = block of P (-1: none); pzord lists
     // the pairs of block r at pzoff[r] .. pzoff[r+1]; pzR blocks.  Blocks of
     // one pair are diagonal terms and listed apart (pznd in pzdiag), unless
@@ -280,7 +278,7 @@ struct HamCoefDev {
     PairDiag *pzdiag;
     int pznd;
     int pzR;
-    PairOff *pql;    // pairs P (with pw; null otherwise)
+    PairOff *pql;    // pairs P (with ph1; null otherwise)
     int real;        // 1 if every coefficient above has a zero imaginary part
     int dense;       // 1 if at least half of the double-jump terms are non-zero:
                      // walking the lists would cost more than it skips
@@ -310,7 +308,6 @@ __host__ __device__ inline HamCoefDev shift_coef(HamCoefDev c, ptrdiff_t d)
     c.tt_off = sh(c.tt_off);
     c.nz_e = sh(c.nz_e);
     c.nz_c = sh(c.nz_c);
-    if (c.pw) c.pw = sh(c.pw);
     if (c.ph1) c.ph1 = sh(c.ph1);
     if (c.pwf) c.pwf = sh(c.pwf);
     if (c.pza) {
