@@ -785,7 +785,10 @@ k_pair_out(PairOutArgs a)
 
 // launch of the output pass for `chunks` grid rows.  A row's pairs are a serial
 // chain of batches, which few rows leave exposed: up to four wavefronts share
-// a row's pairs until there are two blocks a CU.  Lanczos steps, us, without
+// a row's pairs until there are two blocks a CU, two where four would be more
+// wavefronts than the registers of all CUs hold (three a SIMD beyond M = 16:
+// N = 5, M = 21 H.v 20.9 us with two, 22.1 with four; N = 5, M = 20, whose four
+// fit, 19.2 and 17.3).  Lanczos steps, us, without
 // and with: N = 5, M = 21 (208 blocks of whole rows) 118, 110; N = 6, M = 9 (12)
 // 43.0, 40.5; N = 7, M = 13 (197) 66.3, 63.2; with eight blocks a CU N = 10, M =
 // 11 (722) slows from 125 to 129.
@@ -794,7 +797,8 @@ mcpi_status launch_pair_out(PairOutArgs o, int chunks, int ncu, hipStream_t st)
 {
     const int64_t rows = (o.nc + 63) / 64;   // wavefronts of whole rows
     o.S = 1;
-    while (o.S < 4 && rows * chunks * o.S < (int64_t)2 * 4 * ncu) o.S *= 2;
+    const int64_t resident = (int64_t)(M > 16 ? 3 : 4) * 4 * ncu;
+    if (rows * chunks < (int64_t)2 * 4 * ncu) o.S = rows * chunks * 4 <= resident ? 4 : 2;
     const int64_t nb = (rows * o.S + PT / 64 - 1) / (PT / 64);
     size_t sm = sizeof(double) * (o.N + 3) + sizeof(int32_t) * M * (o.N + 1);
     if (o.S > 1) sm = std::max(sm, sizeof(cplx) * PT * MV);
