@@ -219,6 +219,20 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
             zoff = std::move(pf.zoff);
         }
     }
+    // the same term by term, for bases of few rows
+    std::vector<PairTerm> zterm;
+    for (size_t r = 0; r + 1 < zoff.size() && zterm.size() <= (size_t)PAIR_TERMS; r++)
+        for (int x = zoff[r]; x < zoff[r + 1] && zterm.size() <= (size_t)PAIR_TERMS; x++)
+            for (int y = zoff[r]; y < zoff[r + 1]; y++) {
+                const int P = zord[x], Q = zord[y], c2 = pair_hi(P), q2 = pair_hi(Q);
+                const cplx w = pw[(size_t)Q * PWS + P];
+                zterm.push_back({w.re, w.im,
+                                 (uint32_t)(P - c2 * (c2 + 1) / 2) | (uint32_t)c2 << 8 |
+                                     (uint32_t)(Q - q2 * (q2 + 1) / 2) << 16 | (uint32_t)q2 << 24,
+                                 0});
+            }
+    const int nterm = zterm.size() <= (size_t)PAIR_TERMS ? (int)zterm.size() : 0;
+    if (!zoff.empty()) zterm.resize(PAIR_TERMS);
     // blocks of one pair: a*_q a*_l a_q a_l is diagonal, so they need neither
     // of the two passes (Lieb-Liniger: the two lowest and the two highest
     // total momenta)
@@ -276,7 +290,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     size_t nB = nz1.size() + nzo.size() + nzt.size() + 4 * (m1j.size() + ot_off.size() + tt_off.size() +
                                                            nz_e.size() + zblk.size() + zord.size() + zoff.size()) +
                 zrec.size() * sizeof(PairRec) + zrun.size() * sizeof(PairRun) +
-                zdiag.size() * sizeof(PairDiag) + pql.size() * sizeof(PairOff) + 64;
+                zdiag.size() * sizeof(PairDiag) + zterm.size() * sizeof(PairTerm) + pql.size() * sizeof(PairOff) + 64;
     size_t bytes = (nC * sizeof(cplx) + nB + 64 + 255) & ~(size_t)255;
     char *dev = nullptr;
     MCPI_HIP(hipMalloc(&dev, bytes));
@@ -299,6 +313,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     const size_t o_zb = zb.empty() ? 0 : put(zb.data(), zb.size() * sizeof(cplx));
     const size_t o_zrec = zblk.empty() ? 0 : put(zrec.data(), zrec.size() * sizeof(PairRec));
     const size_t o_zdiag = put(zdiag.data(), zdiag.size() * sizeof(PairDiag));
+    const size_t o_zterm = put(zterm.data(), zterm.size() * sizeof(PairTerm));
     const size_t o_zrun = zblk.empty() ? 0 : put(zrun.data(), zrun.size() * sizeof(PairRun));
     const size_t o_pql = pql.empty() ? 0 : put(pql.data(), pql.size() * sizeof(PairOff));
     size_t o_m1 = put(m1j.data(), m1j.size() * 4);
@@ -337,6 +352,8 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     c->pzrun = fac ? (PairRun *)(dev + o_zrun) : nullptr;
     c->pzdiag = (PairDiag *)(dev + o_zdiag);
     c->pznd = (int)zdiag.size();
+    c->pzterm = (PairTerm *)(dev + o_zterm);
+    c->pznt = nterm;
     c->pzR = fac ? (int)zoff.size() - 1 : 0;
     c->pql = pair ? (PairOff *)(dev + o_pql) : nullptr;
     c->nz_1j = (uint8_t *)(dev + o_n1);

@@ -943,7 +943,7 @@ static bool pairz_multi_ok(const HvGroup &g, const mcpi_ham *hams)
             off(h, c.pzblk) != off(h0, c0.pzblk) || off(h, c.pzord) != off(h0, c0.pzord) ||
             off(h, c.pzoff) != off(h0, c0.pzoff) || off(h, c.pzrec) != off(h0, c0.pzrec) ||
             off(h, c.pzrun) != off(h0, c0.pzrun) || off(h, c.pzdiag) != off(h0, c0.pzdiag) ||
-            c.pznd != c0.pznd || off(h, c.ph1) != off(h0, c0.ph1))
+            c.pznd != c0.pznd || off(h, c.pzterm) != off(h0, c0.pzterm) || c.pznt != c0.pznt || off(h, c.ph1) != off(h0, c0.ph1))
             return false;
         if (x == g.members[0]) continue;
         if (!tables(c, t)) {

@@ -216,6 +216,13 @@ struct PairDiag {
     double wr, wi;
     int32_t q, l;
 };
+// a term w a*_{c1} a*_{c2} a_{q1} a_{q2} of the pair form (c1 <= c2, q1 <= q2),
+// an orbital a byte: c1, c2, q1, q2 from the lowest
+struct PairTerm {
+    double wr, wi;
+    uint32_t orb, pad;
+};
+constexpr int PAIR_TERMS = 512;   // records kept with a Hamiltonian in the factorized form
 struct PairRun {
     int32_t r, j;
 };
@@ -277,6 +284,8 @@ struct HamCoefDev {
                      // start at pairs [w].j
     PairDiag *pzdiag;
     int pznd;
+    PairTerm *pzterm;   // w term by term, single pairs included, if there are
+    int pznt;           // at most PAIR_TERMS terms (else pznt is 0)
     int pzR;
     PairOff *pql;    // pairs P (with ph1; null otherwise)
     int real;        // 1 if every coefficient above has a zero imaginary part
@@ -319,6 +328,7 @@ __host__ __device__ inline HamCoefDev shift_coef(HamCoefDev c, ptrdiff_t d)
         c.pzrec = sh(c.pzrec);
         c.pzrun = sh(c.pzrun);
         c.pzdiag = sh(c.pzdiag);
+        c.pzterm = sh(c.pzterm);
     }
     if (c.pql) c.pql = sh(c.pql);
     return c;
