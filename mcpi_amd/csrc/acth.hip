@@ -706,7 +706,7 @@ static bool pair_schedule_ok(mcpi_ham h) { return pair_applicable(h->basis->d, h
 // one H.v with schedule `sched`; 4 = specialised kernel reading the pattern
 // tables of the Hamiltonian's zero pattern (built on first use unless the
 // stream is capturing or memory is short; schedule 2 otherwise)
-static mcpi_status launch_sched(mcpi_ham h, int sched, const cplx *C, cplx *out, hipStream_t st)
+static mcpi_status launch_sched(mcpi_ham h, int sched, const cplx *C, cplx *out, hipStream_t st, PairEpi *e = nullptr)
 {
     const BasisDev &b = h->basis->d;
     if (h->basis->sectored()) {
@@ -734,7 +734,7 @@ static mcpi_status launch_sched(mcpi_ham h, int sched, const cplx *C, cplx *out,
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
             MCPI_HIP(hipStreamIsCapturing(st, &cs));
             cplx *ws = pair_workspace(h->basis, st, cs == hipStreamCaptureStatusNone, pair_need(h, sched));
-            if (ws) return sched == 7 ? launch_pairz(b, h->c, C, out, ws, st) : launch_pair(b, h->c, C, out, ws, st);
+            if (ws) return sched == 7 ? launch_pairz(b, h->c, C, out, ws, st, e) : launch_pair(b, h->c, C, out, ws, st, e);
         }
         sched = 2;
     }
@@ -809,7 +809,7 @@ static mcpi_status autotune(mcpi_ham h, const cplx *C, cplx *out, hipStream_t st
     return MCPI_OK;
 }
 
-mcpi_status launch_apply(mcpi_ham h, const cplx *C, cplx *out, hipStream_t st)
+mcpi_status launch_apply(mcpi_ham h, const cplx *C, cplx *out, hipStream_t st, PairEpi *e)
 {
     int sched = h->schedule;
     if (sched == 0) {
@@ -821,7 +821,7 @@ mcpi_status launch_apply(mcpi_ham h, const cplx *C, cplx *out, hipStream_t st)
         }
         sched = t ? t : (has_fast_kernel(h->basis->d.N, h->basis->d.M) ? 2 : 1);
     }
-    return launch_sched(h, sched, C, out, st);
+    return launch_sched(h, sched, C, out, st, e);
 }
 
 int ham_schedule(mcpi_ham h) { return h->schedule ? h->schedule : h->tuned[h->skip_zero ? 1 : 0]; }

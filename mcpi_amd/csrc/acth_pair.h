@@ -583,6 +583,7 @@ struct PairOutArgs {
     cplx *out;
     int64_t mC, mZ, mK;
     int S;   // wavefronts that share a row's pairs: 1, 2 or 4
+    PairEpi ep;   // (one member) a Lanczos step's next vector operation, if ep.partial
 };
 
 template <int M, bool FAC, bool RC, int MV>
@@ -768,12 +769,40 @@ k_pair_out(PairOutArgs a)
             for (int m = 0; m < MV; m++) red[(m * (PT / 64) + wave) * 64 + lane] = acc[m];
         }
         __syncthreads();
-        if (sub > 0) return;
-        for (int w = 1; w < a.S; w++)
+        for (int w = 1; w < a.S && sub == 0; w++)
 #pragma unroll
             for (int m = 0; m < MV; m++) acc[m] = cadd(acc[m], red[(m * (PT / 64) + wave + w) * 64 + lane]);
     }
-    if (i0 >= a.nc) return;
+    const bool own = sub == 0 && i0 < a.nc;
+    if (MV == 1 && a.ep.partial) {
+        double re = 0, im = 0;
+        if (own) {
+            const cplx x = ldcp(a.ep.lvec + (int64_t)*a.ep.it * a.nc + i), y = ldcp(C + i);
+            const double beta = *a.ep.beta;
+            acc[0].re -= beta * x.re;
+            acc[0].im -= beta * x.im;
+            re = y.re * acc[0].re + y.im * acc[0].im;
+            im = y.re * acc[0].im - y.im * acc[0].re;
+        }
+#pragma unroll
+        for (int k = 32; k > 0; k >>= 1) {
+            re += __shfl_xor(re, k, 64);
+            im += __shfl_xor(im, k, 64);
+        }
+        double *red = (double *)lds;   // [wave][2]
+        __syncthreads();
+        if (lane == 0) {
+            red[2 * wave] = re;
+            red[2 * wave + 1] = im;
+        }
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            double s = 0;
+            for (int w = 0; w < PT / 64; w++) s += red[2 * w + threadIdx.x];
+            a.ep.partial[2 * blockIdx.x + threadIdx.x] = s;
+        }
+    }
+    if (!own) return;
 #pragma unroll
     for (int m = 0; m < MV; m++) {
         double2 o;
@@ -793,7 +822,7 @@ k_pair_out(PairOutArgs a)
 // 43.0, 40.5; N = 7, M = 13 (197) 66.3, 63.2; with eight blocks a CU N = 10, M =
 // 11 (722) slows from 125 to 129.
 template <int M, bool FAC, bool RC, int MV>
-mcpi_status launch_pair_out(PairOutArgs o, int chunks, int ncu, hipStream_t st)
+mcpi_status launch_pair_out(PairOutArgs o, int chunks, int ncu, hipStream_t st, PairEpi *e)
 {
     const int64_t rows = (o.nc + 63) / 64;   // wavefronts of whole rows
     o.S = 1;
@@ -801,7 +830,11 @@ mcpi_status launch_pair_out(PairOutArgs o, int chunks, int ncu, hipStream_t st)
     if (rows * chunks < (int64_t)2 * 4 * ncu) o.S = rows * chunks * 4 <= resident ? 4 : 2;
     const int64_t nb = (rows * o.S + PT / 64 - 1) / (PT / 64);
     size_t sm = sizeof(double) * (o.N + 3) + sizeof(int32_t) * M * (o.N + 1);
-    if (o.S > 1) sm = std::max(sm, sizeof(cplx) * PT * MV);
+    sm = std::max(sm, o.S > 1 ? sizeof(cplx) * PT * MV : 2 * sizeof(double) * (PT / 64));
+    if (MV == 1 && e && nb <= e->cap) {
+        e->blocks = (int)nb;
+        o.ep = *e;
+    }
     hipLaunchKernelGGL((k_pair_out<M, FAC, RC, MV>), dim3((unsigned)nb, (unsigned)chunks), dim3(PT), sm, st, o);
     MCPI_HIP(hipGetLastError());
     return MCPI_OK;
@@ -822,7 +855,7 @@ mcpi_status launch_y1(const PairArgs &a, int ncu, hipStream_t st)
 
 template <int M>
 mcpi_status launch_pair_m(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
-                          hipStream_t st)
+                          hipStream_t st, PairEpi *e)
 {
     int dev = 0, ncu = 0;
     MCPI_HIP(hipGetDevice(&dev));
@@ -883,7 +916,7 @@ mcpi_status launch_pair_m(const BasisDev &b, const HamCoefDev &c, const cplx *C,
     o.Y2 = Y2;
     o.C = C;
     o.out = out;
-    return launch_pair_out<M, false, false, 1>(o, 1, ncu, st);
+    return launch_pair_out<M, false, false, 1>(o, 1, ncu, st, e);
 }
 
 // Z of the factorized form for chunks x MV members: the rows' tiles, the runs
@@ -913,7 +946,7 @@ mcpi_status launch_pairz_amp(PairArgs a, int M, int chunks, int ncu, hipStream_t
 // in c
 template <int M, int MV, bool RC>
 mcpi_status launch_pairz_m(const BasisDev &b, const HamCoefDev &c, int chunks, const cplx *C, cplx *out, int64_t mC,
-                           int64_t mK, cplx *ws, hipStream_t st)
+                           int64_t mK, cplx *ws, hipStream_t st, PairEpi *e)
 {
     int dev = 0, ncu = 0;
     MCPI_HIP(hipGetDevice(&dev));
@@ -955,26 +988,26 @@ mcpi_status launch_pairz_m(const BasisDev &b, const HamCoefDev &c, int chunks, c
     o.mC = mC;
     o.mZ = mZ;
     o.mK = mK;
-    return launch_pair_out<M, true, RC, MV>(o, chunks, ncu, st);
+    return launch_pair_out<M, true, RC, MV>(o, chunks, ncu, st, e);
 }
 
 template <int M, int MV>
 mcpi_status launch_pairz_r(const BasisDev &b, const HamCoefDev &c, int chunks, const cplx *C, cplx *out, int64_t mC,
-                           int64_t mK, cplx *ws, hipStream_t st)
+                           int64_t mK, cplx *ws, hipStream_t st, PairEpi *e)
 {
-    return c.real ? launch_pairz_m<M, MV, true>(b, c, chunks, C, out, mC, mK, ws, st)
-                  : launch_pairz_m<M, MV, false>(b, c, chunks, C, out, mC, mK, ws, st);
+    return c.real ? launch_pairz_m<M, MV, true>(b, c, chunks, C, out, mC, mK, ws, st, e)
+                  : launch_pairz_m<M, MV, false>(b, c, chunks, C, out, mC, mK, ws, st, e);
 }
 
 }  // namespace
 
-#define MCPI_PAIR_CASE(MM) case MM: return launch_pair_m<MM>(b, c, C, out, ws, st);
+#define MCPI_PAIR_CASE(MM) case MM: return launch_pair_m<MM>(b, c, C, out, ws, st, e);
 // members: one, or chunks of mv
-#define MCPI_PAIRZ_CASE(MM) case MM: return launch_pairz_r<MM, 1>(b, c, 1, C, out, 0, 0, ws, st);
+#define MCPI_PAIRZ_CASE(MM) case MM: return launch_pairz_r<MM, 1>(b, c, 1, C, out, 0, 0, ws, st, e);
 #define MCPI_PAIRZ_MV_CASE(MM) \
     case MM: \
-        if (mv == 1) return launch_pairz_r<MM, 1>(b, c, 1, C, out, 0, 0, ws, st); \
-        return mv == 4 ? launch_pairz_r<MM, 4>(b, c, chunks, C, out, mC, mK, ws, st) \
-                       : launch_pairz_r<MM, 2>(b, c, chunks, C, out, mC, mK, ws, st);
+        if (mv == 1) return launch_pairz_r<MM, 1>(b, c, 1, C, out, 0, 0, ws, st, e); \
+        return mv == 4 ? launch_pairz_r<MM, 4>(b, c, chunks, C, out, mC, mK, ws, st, nullptr) \
+                       : launch_pairz_r<MM, 2>(b, c, chunks, C, out, mC, mK, ws, st, nullptr);
 
 }  // namespace mcpi

@@ -10,9 +10,9 @@
 
 namespace mcpi {
 
-#define MCPI_PAIR_ARGS const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws, hipStream_t st
+#define MCPI_PAIR_ARGS const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws, hipStream_t st, PairEpi *e
 #define MCPI_PAIRZ_ARGS const BasisDev &b, const HamCoefDev &c, int mv, int chunks, const cplx *C, cplx *out, \
-                        int64_t mC, int64_t mK, cplx *ws, hipStream_t st
+                        int64_t mC, int64_t mK, cplx *ws, hipStream_t st, PairEpi *e
 mcpi_status launch_pair_a(MCPI_PAIR_ARGS);
 mcpi_status launch_pair_b(MCPI_PAIR_ARGS);
 mcpi_status launch_pairz_a(MCPI_PAIRZ_ARGS);
@@ -40,7 +40,7 @@ constexpr int DW = 4;   // rows (wavefronts) a block
 template <int NW, bool RC>
 __global__ __launch_bounds__(64 * DW) void k_pair_terms(int N, int M, int64_t nc, int nt, const int32_t *IF,
                                                         const int32_t *B, const PairTerm *term, const cplx *h1,
-                                                        const cplx *C, cplx *out)
+                                                        const cplx *C, cplx *out, PairEpi ep)
 {
     constexpr int CW = RC ? 1 : 2;   // doubles of a coefficient
     extern __shared__ __align__(16) unsigned char lds[];
@@ -125,21 +125,49 @@ __global__ __launch_bounds__(64 * DW) void k_pair_terms(int N, int M, int64_t nc
         acc.re += __shfl_xor(acc.re, k, 64);
         acc.im += __shfl_xor(acc.im, k, 64);
     }
+    if (ep.partial) {
+        double re = 0, im = 0;
+        if (i0 < nc) {
+            const cplx x = ep.lvec[(int64_t)*ep.it * nc + i];
+            const double beta = *ep.beta;
+            acc.re -= beta * x.re;
+            acc.im -= beta * x.im;
+            re = c0.re * acc.re + c0.im * acc.im;
+            im = c0.re * acc.im - c0.im * acc.re;
+        }
+        double *red = (double *)lds;   // (over the tables, which are done with)
+        __syncthreads();
+        if (lane == 0) {
+            red[2 * wave] = re;
+            red[2 * wave + 1] = im;
+        }
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            double s = 0;
+            for (int w = 0; w < DW; w++) s += red[2 * w + threadIdx.x];
+            ep.partial[2 * blockIdx.x + threadIdx.x] = s;
+        }
+    }
     if (lane == 0 && i0 < nc) out[i0] = acc;
 }
 
 template <int NW>
-mcpi_status launch_pair_terms(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, hipStream_t st)
+mcpi_status launch_pair_terms(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, hipStream_t st, PairEpi *e)
 {
     const size_t sm = sizeof(double) * (b.N + 3 + (c.real ? 1 : 2) * c.pznt) + 4 * (size_t)(c.pznt + b.M * (b.N + 1)) +
                       2 * (size_t)DW * c.pznt;
     const dim3 grid((unsigned)((b.nc + DW - 1) / DW)), blk(64 * DW);
+    PairEpi ep{};
+    if (e && grid.x <= (unsigned)e->cap) {
+        e->blocks = (int)grid.x;
+        ep = *e;
+    }
     if (c.real)
         hipLaunchKernelGGL((k_pair_terms<NW, true>), grid, blk, sm, st, b.N, b.M, b.nc, c.pznt, b.IF, b.B, c.pzterm,
-                           c.ph1, C, out);
+                           c.ph1, C, out, ep);
     else
         hipLaunchKernelGGL((k_pair_terms<NW, false>), grid, blk, sm, st, b.N, b.M, b.nc, c.pznt, b.IF, b.B, c.pzterm,
-                           c.ph1, C, out);
+                           c.ph1, C, out, ep);
     MCPI_HIP(hipGetLastError());
     return MCPI_OK;
 }
@@ -164,10 +192,10 @@ bool pair_applicable(const BasisDev &b, const HamCoefDev &c)
 }
 
 mcpi_status launch_pair(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
-                        hipStream_t st)
+                        hipStream_t st, PairEpi *e)
 {
     MCPI_ARG(pair_applicable(b, c), "the pair-space H.v does not apply to this basis");
-    return b.M <= 9 ? launch_pair_a(b, c, C, out, ws, st) : launch_pair_b(b, c, C, out, ws, st);
+    return b.M <= 9 ? launch_pair_a(b, c, C, out, ws, st, e) : launch_pair_b(b, c, C, out, ws, st, e);
 }
 
 bool pairz_applicable(const BasisDev &b, const HamCoefDev &c)
@@ -177,16 +205,16 @@ bool pairz_applicable(const BasisDev &b, const HamCoefDev &c)
 }
 
 static mcpi_status launch_pairz_any(const BasisDev &b, const HamCoefDev &c, int mv, int chunks, const cplx *C,
-                                    cplx *out, int64_t mC, int64_t mK, cplx *ws, hipStream_t st)
+                                    cplx *out, int64_t mC, int64_t mK, cplx *ws, hipStream_t st, PairEpi *e)
 {
-    if (b.M <= 9) return launch_pairz_a(b, c, mv, chunks, C, out, mC, mK, ws, st);
-    if (b.M <= 13) return launch_pairz_b(b, c, mv, chunks, C, out, mC, mK, ws, st);
-    if (b.M <= 19) return launch_pairz_c(b, c, mv, chunks, C, out, mC, mK, ws, st);
-    return launch_pairz_d(b, c, mv, chunks, C, out, mC, mK, ws, st);
+    if (b.M <= 9) return launch_pairz_a(b, c, mv, chunks, C, out, mC, mK, ws, st, e);
+    if (b.M <= 13) return launch_pairz_b(b, c, mv, chunks, C, out, mC, mK, ws, st, e);
+    if (b.M <= 19) return launch_pairz_c(b, c, mv, chunks, C, out, mC, mK, ws, st, e);
+    return launch_pairz_d(b, c, mv, chunks, C, out, mC, mK, ws, st, e);
 }
 
 mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
-                        hipStream_t st)
+                        hipStream_t st, PairEpi *e)
 {
     MCPI_ARG(pairz_applicable(b, c), "the factorized pair-space H.v does not apply to this basis and Hamiltonian");
     // by terms while every row's wavefront is resident at once (32 a CU); us a
@@ -196,9 +224,10 @@ mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, 
     MCPI_HIP(hipGetDevice(&dev));
     MCPI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     if (c.pznt > 0 && b.nc <= (int64_t)32 * ncu)
-        return b.M <= 8 ? launch_pair_terms<1>(b, c, C, out, st) : b.M <= 16 ? launch_pair_terms<2>(b, c, C, out, st)
-                                                                             : launch_pair_terms<3>(b, c, C, out, st);
-    return launch_pairz_any(b, c, 1, 1, C, out, 0, 0, ws, st);
+        return b.M <= 8    ? launch_pair_terms<1>(b, c, C, out, st, e)
+               : b.M <= 16 ? launch_pair_terms<2>(b, c, C, out, st, e)
+                           : launch_pair_terms<3>(b, c, C, out, st, e);
+    return launch_pairz_any(b, c, 1, 1, C, out, 0, 0, ws, st, e);
 }
 
 mcpi_status launch_pairz_multi(const BasisDev &b, const HamCoefDev &c, int mv, int chunks, const cplx *C, cplx *out,
@@ -207,7 +236,7 @@ mcpi_status launch_pairz_multi(const BasisDev &b, const HamCoefDev &c, int mv, i
     MCPI_ARG(pairz_applicable(b, c) && b.M <= MCPI_PAIRZ_MULTI_MAXM && (mv == 2 || mv == 4),
              "the factorized pair form for several members does not apply");
     MCPI_ARG(mK % 16 == 0 && mC >= b.nc && chunks >= 1 && chunks <= 65535, "member strides and chunks");
-    return launch_pairz_any(b, c, mv, chunks, C, out, mC, mK, ws, st);
+    return launch_pairz_any(b, c, mv, chunks, C, out, mC, mK, ws, st, nullptr);
 }
 
 }  // namespace mcpi

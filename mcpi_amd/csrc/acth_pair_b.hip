@@ -4,7 +4,7 @@
 namespace mcpi {
 
 mcpi_status launch_pair_b(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
-                          hipStream_t st)
+                          hipStream_t st, PairEpi *e)
 {
     switch (b.M) {
         MCPI_PAIR_CASE(10) MCPI_PAIR_CASE(11) MCPI_PAIR_CASE(12)
@@ -13,7 +13,7 @@ mcpi_status launch_pair_b(const BasisDev &b, const HamCoefDev &c, const cplx *C,
 }
 
 mcpi_status launch_pairz_b(const BasisDev &b, const HamCoefDev &c, int mv, int chunks, const cplx *C, cplx *out,
-                           int64_t mC, int64_t mK, cplx *ws, hipStream_t st)
+                           int64_t mC, int64_t mK, cplx *ws, hipStream_t st, PairEpi *e)
 {
     switch (b.M) {
         MCPI_PAIRZ_MV_CASE(10) MCPI_PAIRZ_MV_CASE(11) MCPI_PAIRZ_MV_CASE(12) MCPI_PAIRZ_MV_CASE(13)

@@ -4,7 +4,7 @@
 namespace mcpi {
 
 mcpi_status launch_pairz_c(const BasisDev &b, const HamCoefDev &c, int mv, int chunks, const cplx *C, cplx *out,
-                           int64_t mC, int64_t mK, cplx *ws, hipStream_t st)
+                           int64_t mC, int64_t mK, cplx *ws, hipStream_t st, PairEpi *e)
 {
     switch (b.M) {
         MCPI_PAIRZ_CASE(14) MCPI_PAIRZ_CASE(15) MCPI_PAIRZ_CASE(16) MCPI_PAIRZ_CASE(17)

@@ -4,7 +4,7 @@
 namespace mcpi {
 
 mcpi_status launch_pairz_d(const BasisDev &b, const HamCoefDev &c, int mv, int chunks, const cplx *C, cplx *out,
-                           int64_t mC, int64_t mK, cplx *ws, hipStream_t st)
+                           int64_t mC, int64_t mK, cplx *ws, hipStream_t st, PairEpi *e)
 {
     switch (b.M) {
         MCPI_PAIRZ_CASE(20) MCPI_PAIRZ_CASE(21) MCPI_PAIRZ_CASE(22) MCPI_PAIRZ_CASE(23)

@@ -228,12 +228,12 @@ __global__ __launch_bounds__(LZ_T) void lz_dot(const LzInst *in)
 
 // alpha from the block partials, into diag[0] (first) or diag[it + 1]
 // (grid (1, K))
-__global__ __launch_bounds__(LZ_T) void lz_fin_alpha(LanczosState *sts, const LzInst *in, int first)
+__global__ __launch_bounds__(LZ_T) void lz_fin_alpha(LanczosState *sts, const LzInst *in, int first, int na)
 {
     LanczosState *st = sts + blockIdx.y;
     const LzInst &I = in[blockIdx.y];
     if (st->broke) return;
-    const double2 s = sum_partials(I.partial, I.nb);
+    const double2 s = sum_partials(I.partial, na ? na : I.nb);
     if (threadIdx.x == 0) {
         st->alpha = cmake(s.x, s.y);
         I.diag[first ? 0 : st->it + 1] = cmake(s.x, s.y);
@@ -347,14 +347,14 @@ __global__ __launch_bounds__(LZ_T) void lz_sub_dot(const LanczosState *sts, cons
 
 // 6a: HC -= alpha v_{i+1}; INL: alpha formed here (5 is no launch)
 template <bool INL>
-__global__ __launch_bounds__(LZ_T) void lz_sub_alpha(LanczosState *sts, const LzInst *in)
+__global__ __launch_bounds__(LZ_T) void lz_sub_alpha(LanczosState *sts, const LzInst *in, int na)
 {
     LanczosState *st = sts + blockIdx.y;
     const LzInst &I = in[blockIdx.y];
     if ((int)blockIdx.x >= I.nb || st->broke) return;
     cplx a = st->alpha;
     if (INL) {
-        const double2 p = sum_partials(I.partial, I.nb);
+        const double2 p = sum_partials(I.partial, na ? na : I.nb);
         a = cmake(p.x, p.y);
         if (blockIdx.x == 0 && threadIdx.x == 0) I.diag[st->it + 1] = a;
     }
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(LZ_T) void lz_sub_alpha(LanczosState *sts, const Lz
 // registers by every block of a segment and stored, to HC2, by those of the
 // first vectors.
 template <int TG, bool FUSE, bool NT>
-__global__ __launch_bounds__(LZ_T) void lz_gemv_dots(const LanczosState *sts, const LzInst *in)
+__global__ __launch_bounds__(LZ_T) void lz_gemv_dots(const LanczosState *sts, const LzInst *in, int na)
 {
     constexpr int R = FUSE ? LZ_RF : LZ_R;   // rows of a thread
     __shared__ double red[TG][LZ_T / 64][2];
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(LZ_T) void lz_gemv_dots(const LanczosState *sts, co
             const int64_t j = base + (int64_t)r * LZ_T;
             y[r] = (j < n) ? ldv(gp(I.vin) + j) : cmake(0, 0);
         }
-        const double2 a = sum_partials(I.partial, I.nb);
+        const double2 a = sum_partials(I.partial, na ? na : I.nb);
         const bool first = blockIdx.y == 0;
         if (first && blockIdx.x == 0 && threadIdx.x == 0) I.diag[st->it + 1] = cmake(a.x, a.y);
 #pragma unroll
@@ -825,6 +825,14 @@ static int dot_group(const std::vector<int64_t> &ns)
     for (int64_t n : ns) sg += (n + LZ_SEG - 1) / LZ_SEG;
     return sg < 4096 ? 8 : 16;
 }
+
+// Most partials of alpha that a pair-space H.v may leave (one a block of 256
+// rows or fewer: vectors of up to 2 M entries); past them their sum, in one
+// block, takes what sparing lz_sub_dot saves.  One instance, us a step with
+// lz_sub_dot and without: N = 6, M = 9 37.3, 35.2; N = 8, M = 11 60.0, 57.8; N = 5,
+// M = 21, 400 steps 108.3, 105.5; N = 10, M = 11 124.5, 121.0; N = 10, M = 12
+// 170.6, 168.1; N = 11, M = 12 300, 297.
+constexpr int LZ_EPI = 8192;
 
 // What the kernels of a chain do beside their own work.  Forming the sums of
 // block partials in every block that needs them takes less than a launch of
@@ -1258,7 +1266,7 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
         if (batched_member[x] < 0)
             for (int k = 0; k < 2; k++) A.reserve(sizeof(cplx) * n);
         for (int k = 0; k < 3; k++) A.reserve(sizeof(cplx) * lm);
-        A.reserve(sizeof(double) * 2 * I.nb);
+        A.reserve(sizeof(double) * 2 * (K == 1 ? std::max(I.nb, LZ_EPI) : I.nb));
         A.reserve(sizeof(double) * 2 * (size_t)I.nbg * lm);
         A.reserve(sizeof(double) * lm);
         if (split_update(n)) A.reserve(sizeof(cplx) * n * (size_t)((lm + LZ_TG - 1) / LZ_TG));
@@ -1303,7 +1311,7 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
         I.diag = A.take<cplx>(lm);
         I.offd = A.take<cplx>(lm);
         I.ortho = A.take<cplx>(lm);
-        I.partial = A.take<double>(2 * I.nb);
+        I.partial = A.take<double>(2 * (K == 1 ? std::max(I.nb, LZ_EPI) : I.nb));
         I.partial_o = A.take<double>(2 * (size_t)I.nbg * lm);
         double *z = A.take<double>(lm);
         I.z = z;
@@ -1350,7 +1358,7 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
     }
     for (const HvGroup &g : groups) MCPI_CHECK(launch_group(g, hams, hin, s));
     hipLaunchKernelGGL(lz_dot, gv, blk, 0, s, (const LzInst *)din);
-    hipLaunchKernelGGL(lz_fin_alpha, g1, blk, 0, s, sts, (const LzInst *)din, 1);
+    hipLaunchKernelGGL(lz_fin_alpha, g1, blk, 0, s, sts, (const LzInst *)din, 1, 0);
     hipLaunchKernelGGL(lz_sub_alpha_norm, gv, blk, 0, s, (const LanczosState *)sts, (const LzInst *)din);
     MCPI_HIP(hipGetLastError());
 
@@ -1364,14 +1372,23 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
                 hipLaunchKernelGGL(lz_fin_beta, g1, blk, 0, s, sts, cin);
                 hipLaunchKernelGGL(lz_scale<false>, gv, blk, 0, s, sts, cin);
             }
-            for (const HvGroup &g : groups) MCPI_CHECK(launch_group(g, hams, hin, s));
-            hipLaunchKernelGGL(lz_sub_dot, gv, blk, 0, s, cst, cin);
+            // one instance: the pair-space H.v does 4 as well and says in how
+            // many partials (0: it did not)
+            int na = 0;
+            if (K == 1 && !groups[0].batched) {
+                PairEpi e{hin[0].lvec, &sts->it, &sts->beta, hin[0].partial, LZ_EPI, 0};
+                MCPI_CHECK(launch_apply(hams[0], hin[0].vin, hin[0].HC, s, &e));
+                na = e.blocks;
+            } else {
+                for (const HvGroup &g : groups) MCPI_CHECK(launch_group(g, hams, hin, s));
+            }
+            if (!na) hipLaunchKernelGGL(lz_sub_dot, gv, blk, 0, s, cst, cin);
             if (ch.fuse) {
                 if (ch.cached) {
-                    hipLaunchKernelGGL((lz_gemv_dots<8, true, false>), gd, blk, 0, s, cst, cin);
+                    hipLaunchKernelGGL((lz_gemv_dots<8, true, false>), gd, blk, 0, s, cst, cin, na);
                     hipLaunchKernelGGL((lz_reorth_part<true, false>), gpart, blk, 0, s, cst, cin);
                 } else {
-                    hipLaunchKernelGGL((lz_gemv_dots<8, true, true>), gd, blk, 0, s, cst, cin);
+                    hipLaunchKernelGGL((lz_gemv_dots<8, true, true>), gd, blk, 0, s, cst, cin, na);
                     hipLaunchKernelGGL((lz_reorth_part<true, true>), gpart, blk, 0, s, cst, cin);
                 }
                 hipLaunchKernelGGL(lz_reorth_sum<true>, gv, blk, 0, s, sts, cin);
@@ -1379,15 +1396,15 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
                 return MCPI_OK;
             }
             if (ch.inl) {
-                hipLaunchKernelGGL(lz_sub_alpha<true>, gv, blk, 0, s, sts, cin);
+                hipLaunchKernelGGL(lz_sub_alpha<true>, gv, blk, 0, s, sts, cin, na);
             } else {
-                hipLaunchKernelGGL(lz_fin_alpha, g1, blk, 0, s, sts, cin, 0);
-                hipLaunchKernelGGL(lz_sub_alpha<false>, gv, blk, 0, s, sts, cin);
+                hipLaunchKernelGGL(lz_fin_alpha, g1, blk, 0, s, sts, cin, 0, na);
+                hipLaunchKernelGGL(lz_sub_alpha<false>, gv, blk, 0, s, sts, cin, na);
             }
             if (dtg == 8)
-                hipLaunchKernelGGL((lz_gemv_dots<8, false, true>), gd, blk, 0, s, cst, cin);
+                hipLaunchKernelGGL((lz_gemv_dots<8, false, true>), gd, blk, 0, s, cst, cin, na);
             else
-                hipLaunchKernelGGL((lz_gemv_dots<16, false, true>), gd, blk, 0, s, cst, cin);
+                hipLaunchKernelGGL((lz_gemv_dots<16, false, true>), gd, blk, 0, s, cst, cin, na);
             hipLaunchKernelGGL(lz_fin_ortho, go, blk, 0, s, cst, cin);
             if (ch.whole) {
                 if (rr == 2)

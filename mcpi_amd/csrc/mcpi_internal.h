@@ -226,6 +226,18 @@ constexpr int PAIR_TERMS = 512;   // records kept with a Hamiltonian in the fact
 struct PairRun {
     int32_t r, j;
 };
+// What the last kernel of a pair-space H.v does beside writing out = H C, in a
+// Lanczos step: out = H C - beta v_it (v_t at lvec + t nc) and, per block, the
+// partial sum of conj(C) out.  The launch sets blocks to the number of
+// partials, or leaves 0 where it does not do this (another schedule, more than
+// cap blocks)
+struct PairEpi {
+    const cplx *lvec;
+    const int *it;
+    const double *beta;
+    double *partial;
+    int cap, blocks;
+};
 constexpr int PAIR_RUNS = 12;
 __host__ __device__ constexpr int pair_run(int g) { return (g - 1) * (2 * g + 1); }   // 4 g + 1 entries for each g
 
@@ -397,7 +409,7 @@ __device__ inline unsigned chunk_xcd(unsigned b, unsigned n, unsigned G)
 }
 
 // kernels launched from host code of other translation units
-mcpi_status launch_apply(mcpi_ham h, const cplx *C, cplx *out, hipStream_t st);
+mcpi_status launch_apply(mcpi_ham h, const cplx *C, cplx *out, hipStream_t st, PairEpi *e = nullptr);
 int ham_schedule(mcpi_ham h);
 bool has_fast_kernel(int N, int M);
 // pattern tables of basis b for the zero pattern of c; built when absent if
@@ -439,13 +451,13 @@ mcpi_status widen_strides(int64_t n, const int32_t *a, int64_t *w, hipStream_t s
 bool pair_applicable(const BasisDev &b, const HamCoefDev &c);
 size_t pair_workspace_entries(int N, int M);
 mcpi_status launch_pair(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
-                        hipStream_t st);
+                        hipStream_t st, PairEpi *e = nullptr);
 // schedule 7 (acth_pair.hip): the factorized pair form applies (as 6, and
 // the Hamiltonian's pair matrix factorizes, N >= 2); launch into a
 // workspace of (blocks) x pair_ld(NC(N-2, M)) complex entries
 bool pairz_applicable(const BasisDev &b, const HamCoefDev &c);
 mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
-                         hipStream_t st);
+                         hipStream_t st, PairEpi *e = nullptr);
 // the same for chunks x mv (mv 2 or 4) Hamiltonians of one basis whose
 // pair matrices share the blocks and b factors (M <=
 // MCPI_PAIRZ_MULTI_MAXM), mv members per thread: member m's vectors at
