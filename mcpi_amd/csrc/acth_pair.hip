@@ -35,7 +35,7 @@ constexpr int DW = 4;   // rows (wavefronts) a block
 // the rank table in LDS; the lanes' sums meet in a fixed order.  What bounds it
 // is latency, then the integer work of the targets, which the two passes share
 // between the rows of a pair state.  Measured (before: the two passes): N = 6, M
-// = 9 8.5 -> 4.9 us, N = 20, M = 4 6.2 -> 3.5, N = 4, M = 13 9.9 -> 5.1 (without
+// = 9 8.5 -> 5.0 us, N = 20, M = 4 6.2 -> 3.7, N = 4, M = 13 9.9 -> 5.2 (without
 // the list 6.0, 3.1 and 8.7).
 template <int NW, bool RC>
 __global__ __launch_bounds__(64 * DW) void k_pair_terms(int N, int M, int64_t nc, int nt, const int32_t *IF,
@@ -88,8 +88,16 @@ __global__ __launch_bounds__(64 * DW) void k_pair_terms(int N, int M, int64_t nc
         for (int w = 1; w < NW; w++) x = k >= 8 * w ? p[w] : x;
         return (int)((uint32_t)(x >> (8 * (k & 7))) & 255u);
     };
-    // the diagonal one-body part, an orbital a lane
-    cplx acc = cfma(cmake(hr * vk, hi * vk), c0, cmake(0, 0));
+    // the diagonal one-body part, an orbital a lane; its sum meets C[v] once, so
+    // that an infinite entry does not meet the zeros of the empty orbitals
+    double dr = hr * vk, di = hi * vk;
+#pragma unroll
+    for (int k = 32; k > 0; k >>= 1) {
+        dr += __shfl_xor(dr, k, 64);
+        if (!RC) di += __shfl_xor(di, k, 64);
+    }
+    cplx acc = cmake(0, 0);
+    if (lane == 0) acc = RC ? cscale(c0, dr) : cfma(cmake(dr, di), c0, acc);
     for (int x = lane; x < n; x += 64) {
         const int id = list[x];
         const uint32_t o = orb[id];
@@ -118,7 +126,13 @@ __global__ __launch_bounds__(64 * DW) void k_pair_terms(int N, int M, int64_t nc
             below = (uint32_t)(p >> 56);
         }
         const double f = sq[c1 < c2 ? v1 : v1 - 1] * sq[v2] * (sq[q1 < q2 ? u1 : u1 - 1] * sq[u2]);
-        acc = cfma(cscale(w, f), C[(uint32_t)(nc - 1) - s], acc);
+        const cplx x0 = C[(uint32_t)(nc - 1) - s];
+        if (RC) {
+            acc.re = fma(w.re * f, x0.re, acc.re);
+            acc.im = fma(w.re * f, x0.im, acc.im);
+        } else {
+            acc = cfma(cscale(w, f), x0, acc);
+        }
     }
 #pragma unroll
     for (int k = 32; k > 0; k >>= 1) {
@@ -218,8 +232,8 @@ mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, 
 {
     MCPI_ARG(pairz_applicable(b, c), "the factorized pair-space H.v does not apply to this basis and Hamiltonian");
     // by terms while every row's wavefront is resident at once (32 a CU); us a
-    // H.v through the pair space and by terms: N = 6, M = 9 (3,003 rows) 8.5, 4.9;
-    // N = 6, M = 11 (8,008) 9.4, 8.5; N = 8, M = 9 (12,870) 8.8, 11.0
+    // H.v through the pair space and by terms: N = 6, M = 9 (3,003 rows) 8.5, 5.0;
+    // N = 6, M = 11 (8,008) 9.4, 9.0; N = 8, M = 9 (12,870) 8.8, 11.0
     int dev = 0, ncu = 0;
     MCPI_HIP(hipGetDevice(&dev));
     MCPI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));

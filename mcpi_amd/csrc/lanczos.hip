@@ -23,7 +23,8 @@
 //   8 reorth_norm   HC -= sum_t v_t o_t;  partial ||HC||^2 for the next step
 // With few partials the kernel that needs a sum forms it itself, every block
 // the same one in the same order, and 1, 5 and 7 are no launches of their own;
-// on short vectors 6 is one launch too (LzChain).
+// on short vectors 6 is one launch too (LzChain).  For one instance a
+// pair-space H.v does 4 itself.
 // Every scalar lives in device memory and the pointers never change, so the
 // chain is captured once in a hipGraph and replayed lm-1 times with no host
 // round trip.  An instance that breaks down stops updating (its kernels

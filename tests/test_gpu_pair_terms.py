@@ -38,6 +38,26 @@ def test_terms_and_passes(oracle_lib, N, M, phases):
     assert_close(H(C), ref, 1e-13, "two passes")
 
 
+@pytest.mark.parametrize("phases", [False, True])
+def test_infinite_entry(phases):
+    """The entries of the result that an infinite entry of C reaches are the
+    same ones by terms and through the two passes."""
+    N, M = 5, 8
+    note(f"pair terms infinite entry phases={phases}")
+    b = mcpi_amd.Basis(N, M, "none")
+    H = mcpi_amd.Hamiltonian(b, *disguised(M, 2.0, 3, phases), schedule=7)
+    rng = np.random.default_rng(2)
+    for j in (0, b.nc // 3, b.nc - 1):
+        C = rng.standard_normal(b.nc) + 1j * rng.standard_normal(b.nc)
+        C[j] = complex(np.inf, 1.0)
+        H2 = mcpi_amd.Hamiltonian(b, *disguised(M, 2.0, 3, phases), schedule=7)
+        drop_terms(H2)
+        x, y = H(C), H2(C)
+        assert np.array_equal(np.isfinite(x.real), np.isfinite(y.real))
+        assert np.array_equal(np.isfinite(x.imag), np.isfinite(y.imag))
+        assert 0 < np.count_nonzero(~np.isfinite(x.real)) < b.nc
+
+
 # two words with terms in the second, three words: one larger block of pairs
 @pytest.mark.parametrize("M", [10, 16, 17, 24])
 def test_one_block_of_pairs(oracle_lib, M):
