@@ -77,7 +77,9 @@ struct LzInst {
     const int32_t *iperm; // sector-ordered basis: reference index of each row
                           // (the start vector is gathered through it and the
                           // Ritz vector scattered); null otherwise
-    int nb, nbg;          // vector and dot blocks used by this instance
+    int nb, nbg, nbp;     // blocks of this instance in the vector passes (which
+                          // stride), the dots and the partial update (which do
+                          // not: dot_rows, part_rows)
     int steps;            // Ritz length (after the host solve)
 };
 
@@ -383,6 +385,11 @@ __global__ __launch_bounds__(LZ_T) void lz_sub_alpha(LanczosState *sts, const Lz
 #define LZ_RF 4
 #define LZ_RP 2
 #define LZ_SEG ((int64_t)LZ_T * LZ_R)
+// rows of a block of the dots and of the partial update: a block covers them
+// once, so each pass has a block count of its own (it is not nb, which goes with
+// the rows of a thread in the single-pass update)
+__host__ __device__ constexpr int dot_rows(bool fuse) { return LZ_T * (fuse ? LZ_RF : LZ_R); }
+__host__ __device__ constexpr int part_rows(bool fuse) { return LZ_T * (fuse ? LZ_RP : LZ_R); }
 // vector groups of the split Gram-Schmidt update (small bases)
 #define LZ_TG 32
 // FUSE (short vectors): 5 and 6a here too, HC - alpha v_{i+1} formed in
@@ -391,7 +398,7 @@ __global__ __launch_bounds__(LZ_T) void lz_sub_alpha(LanczosState *sts, const Lz
 template <int TG, bool FUSE, bool NT>
 __global__ __launch_bounds__(LZ_T) void lz_gemv_dots(const LanczosState *sts, const LzInst *in, int na)
 {
-    constexpr int R = FUSE ? LZ_RF : LZ_R;   // rows of a thread
+    constexpr int R = dot_rows(FUSE) / LZ_T;   // rows of a thread
     __shared__ double red[TG][LZ_T / 64][2];
     const LanczosState *st = sts + blockIdx.z;
     const LzInst &I = in[blockIdx.z];
@@ -561,11 +568,11 @@ __global__ __launch_bounds__(LZ_T) void lz_reorth_norm(LanczosState *sts, const 
 template <bool FUSE, bool NT>
 __global__ __launch_bounds__(LZ_T) void lz_reorth_part(const LanczosState *sts, const LzInst *in)
 {
-    constexpr int R = FUSE ? LZ_RP : LZ_R;   // rows of a thread
+    constexpr int R = part_rows(FUSE) / LZ_T;   // rows of a thread
     __shared__ cplx so[LZ_TG];
     const LanczosState *st = sts + blockIdx.z;
     const LzInst &I = in[blockIdx.z];
-    if (!I.rpart || (int)blockIdx.x >= (FUSE ? I.nb : I.nbg) || st->broke) return;
+    if (!I.rpart || (int)blockIdx.x >= I.nbp || st->broke) return;
     const int nt = st->it + 2;
     const int t0 = blockIdx.y * LZ_TG;
     if (t0 >= nt) return;
@@ -1237,7 +1244,7 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
     A.reserve(sizeof(LanczosState) * K);
     A.reserve(sizeof(LzInst) * K);
     std::vector<LzInst> hin(K);
-    int nbmax = 1, nbgmax = 1;
+    int nbmax = 1, nbgmax = 1, nbpmax = 1;
     std::vector<int64_t> ns(K);
     for (int x = 0; x < K; x++) ns[x] = hams[x]->basis->d.nc;
     const int rr = update_rows(ns), dtg = dot_group(ns);
@@ -1259,10 +1266,11 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
         LzInst &I = hin[x];
         I.n = n;
         I.nb = (int)row_blocks(n, rr);
-        const int64_t seg = ch.fuse ? LZ_T * LZ_RF : LZ_SEG;
-        I.nbg = (int)((n + seg - 1) / seg);
+        I.nbg = (int)((n + dot_rows(ch.fuse) - 1) / dot_rows(ch.fuse));
+        I.nbp = (int)((n + part_rows(ch.fuse) - 1) / part_rows(ch.fuse));
         nbmax = std::max(nbmax, I.nb);
         nbgmax = std::max(nbgmax, I.nbg);
+        nbpmax = std::max(nbpmax, I.nbp);
         if (!(lvec_ext && lvec_ext[x])) A.reserve(sizeof(cplx) * n * (size_t)lm);
         if (batched_member[x] < 0)
             for (int k = 0; k < 2; k++) A.reserve(sizeof(cplx) * n);
@@ -1345,7 +1353,7 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
     MCPI_HIP(hipMemcpyAsync(din, hin.data(), sizeof(LzInst) * K, hipMemcpyHostToDevice, s));
 
     const dim3 blk(LZ_T), gv(nbmax, K), g1(1, K);
-    const dim3 gd(nbgmax, (lm + dtg - 1) / dtg, K), gpart(ch.fuse ? nbmax : nbgmax, (lm + LZ_TG - 1) / LZ_TG, K);
+    const dim3 gd(nbgmax, (lm + dtg - 1) / dtg, K), gpart(nbpmax, (lm + LZ_TG - 1) / LZ_TG, K);
     const dim3 go(lm, K);
 
     // ---- set-up: v_0, schedules, HC = H v_0, alpha_0, HC -= alpha_0 v_0
