@@ -846,14 +846,25 @@ constexpr int LZ_EPI = 8192;
 // block partials in every block that needs them takes less than a launch of
 // its own (about 4.5 us a step each) up to 2^20 partials in all (1024 blocks of
 // one instance, 16 MB from the L2s); the 64-instance call, with ten times as
-// many, loses 15 us a step to them.  Where every instance has the split update
-// (vectors of up to 262,144 entries, at most 128 segments), the alpha part and
-// the o_t are formed where they are used too.  Basis vectors that the Infinity
-// Cache can hold for the most part (512 MB at the last step) are read with
-// plain loads, larger ones pass it by.  Measured, us a step (before; with inl
-// only; now): N = 6, M = 9, 120 steps 68, 52, 43; N = 8, M = 11 100, 80, 63; N =
-// 5, M = 21, 400 steps 192, 126, 116; N = 10, M = 11 154, 130, 125; N = 5, M =
-// 21, 1500 steps 352, 282, 288.
+// many, loses 15 us a step to them.  (Alpha of one instance may have twice as
+// many, one a block of the H.v: N = 6, M = 24, 928 blocks of 1,856 partials,
+// 204.8 us a step here, 207.0 with a kernel of its own for alpha.)
+// Where every instance has the split update (vectors of up to 262,144 entries:
+// at most 256 segments in the fused passes), the alpha part and the o_t are
+// formed where they are used too, unless the basis vectors of an instance are
+// more than 512 MB at the last step: then what every block of eight vectors
+// reads and sums again costs more than the launches.  One instance, us a step
+// fused and not: N = 5, M = 21, 400 steps 106, 116, 1500 277, 270; N = 17, M = 7,
+// 120 steps 79, 93, 400 166, 158, 1000 336, 317; N = 10, M = 11, 120 steps 122,
+// 129, 250 197, 186, 700 437, 404.  (In a call of many instances the two differ
+// by 2 % between 80 and 300 MB an instance; 342 of N = 6, M = 9, 60 steps: 924,
+// 1014.)  Basis vectors that the Infinity Cache can hold for the most part (512
+// MB at the last step, all instances) are read with plain loads, larger ones
+// pass it by.  Measured, us a step (before; with inl only; now): N = 6, M = 9, 120
+// steps 68, 52, 43; N = 8, M = 11 100, 80, 63; N = 5, M = 21, 400 steps 192, 126,
+// 116; N = 10, M = 11 154, 130, 125.
+constexpr int64_t LZ_VBYTES = (int64_t)512 << 20;
+
 struct LzChain {
     bool inl = true;     // 1 and 5 inside 2 and 6
     bool fuse = true;    // 5, 6a inside 6b and 7 inside 8
@@ -1249,18 +1260,21 @@ static mcpi_status lanczos_core(int K, const mcpi_ham *hams, const cplx *const *
     for (int x = 0; x < K; x++) ns[x] = hams[x]->basis->d.nc;
     const int rr = update_rows(ns), dtg = dot_group(ns);
     LzChain ch;
-    int64_t vbytes = 0, reads = 0;   // partials read by all blocks of a kernel
+    int64_t vbytes = 0, vmost = 0;   // basis vectors: all instances, the largest
+    int64_t reads = 0;               // partials read by all blocks of a kernel
     for (int64_t n : ns) {
         const bool sp = split_update(n);
         ch.split = ch.split || sp;
         ch.whole = ch.whole || !sp;
         reads += row_blocks(n, rr) * row_blocks(n, rr);
         ch.fuse = ch.fuse && sp;
-        vbytes += (int64_t)sizeof(cplx) * n * lm;
+        const int64_t v = (int64_t)sizeof(cplx) * n * lm;
+        vbytes += v;
+        vmost = std::max(vmost, v);
     }
     ch.inl = reads <= (int64_t)1 << 20;
-    ch.fuse = ch.fuse && ch.inl && dtg == 8;
-    ch.cached = vbytes <= (int64_t)512 << 20;
+    ch.fuse = ch.fuse && ch.inl && dtg == 8 && vmost <= LZ_VBYTES;
+    ch.cached = vbytes <= LZ_VBYTES;
     for (int x = 0; x < K; x++) {
         const int64_t n = ns[x];
         LzInst &I = hin[x];
