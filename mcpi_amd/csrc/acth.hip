@@ -128,9 +128,8 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
             if (nzt[p * M2 + e]) { nz_e.push_back(e); nz_c.push_back(tt[p * M2 + e]); }
     }
     tt_off[P] = (int32_t)nz_e.size();
-    // the lists are padded to their largest possible length, so that every
-    // Hamiltonian with M orbitals has the same block layout and size (batched
-    // H.v addresses instance x's tables at a fixed stride from instance 0's)
+    // the lists are padded to their largest possible length: batched H.v
+    // addresses instance x's tables at a fixed stride from instance 0's
     nz_e.resize((size_t)(M + std::max(P, 1)) * M2 + 1, 0);
     nz_c.resize(nz_e.size(), cmake(0, 0));
     // The operator in pair form (schedule 6): every folded term is a
@@ -284,7 +283,10 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     std::vector<PairOff> pql;
     if (pair)
         for (int x = 0; x < pair_count(M); x++) pql.push_back(offsets(x));
-    // one device block: complex tables first (16-byte aligned), then integers
+    // One device block, the tables whose sizes M alone gives first (complex
+    // ones, then integers): they have the same offsets in every Hamiltonian
+    // with M orbitals.  Those that depend on N and on the factorized form come
+    // last; blocks of the same size may still differ there.
     size_t nC = dk.size() + d1.size() + d2.size() + A0.size() + A.size() + ot.size() + tt.size() + nz_c.size() +
                 otc.size() + ttc.size() + ph1.size() + pwf.size() + za.size() + zb.size();
     size_t nB = nz1.size() + nzo.size() + nzt.size() + 4 * (m1j.size() + ot_off.size() + tt_off.size() +
@@ -308,6 +310,15 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     size_t o_otc = put(otc.data(), otc.size() * sizeof(cplx));
     size_t o_ttc = put(ttc.data(), ttc.size() * sizeof(cplx));
     const size_t o_ph1 = ph1.empty() ? 0 : put(ph1.data(), ph1.size() * sizeof(cplx));
+    const size_t o_pql = pql.empty() ? 0 : put(pql.data(), pql.size() * sizeof(PairOff));
+    size_t o_m1 = put(m1j.data(), m1j.size() * 4);
+    size_t o_oo = put(ot_off.data(), ot_off.size() * 4);
+    size_t o_to = put(tt_off.data(), tt_off.size() * 4);
+    size_t o_ne = put(nz_e.data(), nz_e.size() * 4);
+    size_t o_n1 = put(nz1.data(), nz1.size());
+    size_t o_no = put(nzo.data(), nzo.size());
+    size_t o_nt = put(nzt.data(), nzt.size());
+    off = (off + 15) & ~(size_t)15;
     const size_t o_pwf = pwf.empty() ? 0 : put(pwf.data(), pwf.size() * sizeof(cplx));
     const size_t o_za = za.empty() ? 0 : put(za.data(), za.size() * sizeof(cplx));
     const size_t o_zb = zb.empty() ? 0 : put(zb.data(), zb.size() * sizeof(cplx));
@@ -315,17 +326,9 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     const size_t o_zdiag = put(zdiag.data(), zdiag.size() * sizeof(PairDiag));
     const size_t o_zterm = put(zterm.data(), zterm.size() * sizeof(PairTerm));
     const size_t o_zrun = zblk.empty() ? 0 : put(zrun.data(), zrun.size() * sizeof(PairRun));
-    const size_t o_pql = pql.empty() ? 0 : put(pql.data(), pql.size() * sizeof(PairOff));
-    size_t o_m1 = put(m1j.data(), m1j.size() * 4);
-    size_t o_oo = put(ot_off.data(), ot_off.size() * 4);
-    size_t o_to = put(tt_off.data(), tt_off.size() * 4);
-    size_t o_ne = put(nz_e.data(), nz_e.size() * 4);
     const size_t o_zblk = zblk.empty() ? 0 : put(zblk.data(), zblk.size() * 4);
     const size_t o_zord = zblk.empty() ? 0 : put(zord.data(), zord.size() * 4);
     const size_t o_zoff = zblk.empty() ? 0 : put(zoff.data(), zoff.size() * 4);
-    size_t o_n1 = put(nz1.data(), nz1.size());
-    size_t o_no = put(nzo.data(), nzo.size());
-    size_t o_nt = put(nzt.data(), nzt.size());
     hipError_t e = hipMemcpy(dev, host.data(), bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(dev);

@@ -378,7 +378,9 @@ struct mcpi_ham_s {
     mcpi_basis basis;
     HamCoefDev c;
     void *coef_block;   // single device allocation holding the tables
-    size_t coef_bytes;  // its size (the same for every Hamiltonian with M orbitals)
+    size_t coef_bytes;  // its size: M's tables, at the same offsets for every
+                        // Hamiltonian with M orbitals, then N's and those of
+                        // the factorized form
     cplx *Ho_dev;       // M*M flat, k + M*l
     cplx *Hint_dev;     // M^4
     int skip_zero;
