@@ -29,8 +29,27 @@ namespace mcpi {
 
 // --------------------------------------------------------- coefficients --
 
+static size_t fragment_entries(int M) { return (size_t)(pair_x_rows(M) / 4) * (pair_stride(M) / 16) * 64; }
+
+// the pair product's copy of the pair matrix (HamCoefDev::pwf) at f, zero
+// before: h1[k][l] / (N - 1) added to w[{k, s}][{s, l}] for every s
+static void pair_fragments(int N, int M, const cplx *pw, const cplx *ph1, cplx *f)
+{
+    const int NP = pair_count(M), PWS = pair_stride(M), NG = PWS / 16, HS = pair_h1_stride(M);
+    // entry (P, Q) = (16 g + i, 4 s + k) at [s][g][i + 16 k]
+    auto at = [&](int P, int Q) -> cplx & { return f[((size_t)(Q / 4) * NG + P / 16) * 64 + P % 16 + 16 * (Q % 4)]; };
+    for (int Q = 0; Q < NP; Q++)
+        for (int P = 0; P < NP; P++) at(P, Q) = pw[(size_t)Q * PWS + P];
+    for (int k = 0; k < M; k++)
+        for (int l = 0; l < M; l++)
+            for (int s = 0; s < M; s++) {
+                cplx &w = at(pair_of2(k, s), pair_of2(s, l));
+                w = cadd(w, cscale(ph1[(size_t)l * HS + k], 1.0 / (N - 1)));
+            }
+}
+
 mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefDev *c, void **block,
-                               size_t *block_bytes, int N)
+                               size_t *block_bytes, int N, PairHost *keep)
 {
     const int64_t M2 = (int64_t)M * M, M3 = M2 * M;
     const int P = M * (M - 1) / 2;
@@ -187,24 +206,6 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
                     }
             }
     }
-    // the pair product's copy of W (HamCoefDev::pwf): h1[k][l] / (N - 1) added
-    // to W[{k, s}][{s, l}] for every s
-    std::vector<cplx> pwf;
-    if (pair && M <= MCPI_PAIR_MAXM && N >= 2) {
-        std::vector<cplx> W = pw;
-        for (int k = 0; k < M; k++)
-            for (int l = 0; l < M; l++)
-                for (int s = 0; s < M; s++) {
-                    cplx &w = W[(size_t)pair_of2(s, l) * PWS + pair_of2(k, s)];
-                    w = cadd(w, cscale(ph1[(size_t)l * HS + k], 1.0 / (N - 1)));
-                }
-        const int NP = pair_count(M), KS = pair_x_rows(M) / 4, NG = PWS / 16;
-        pwf.assign((size_t)KS * NG * 64, cmake(0, 0));
-        for (size_t x = 0; x < pwf.size(); x++) {
-            const int ln = (int)(x % 64), P = 16 * (int)(x / 64 % NG) + ln % 16, Q = 4 * (int)(x / 64 / NG) + ln / 16;
-            if (P < NP && Q < NP) pwf[x] = W[(size_t)Q * PWS + P];
-        }
-    }
     // the factorized pair form of schedule 7 (pair_factor.h)
     std::vector<cplx> za, zb;
     std::vector<int32_t> zblk, zord, zoff;
@@ -218,9 +219,18 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
             zoff = std::move(pf.zoff);
         }
     }
-    // the same term by term, for bases of few rows
+    // the pair product's tables, where the factorized form does not stand in
+    // for it; there they are laid out when schedule 6 is asked for
+    std::vector<cplx> pwf;
+    if (pair && M <= MCPI_PAIR_MAXM && N >= 2 && zblk.empty()) {
+        pwf.assign(fragment_entries(M), cmake(0, 0));
+        pair_fragments(N, M, pw.data(), ph1.data(), pwf.data());
+    }
+    // the factorized form term by term, for bases of few rows
     std::vector<PairTerm> zterm;
-    for (size_t r = 0; r + 1 < zoff.size() && zterm.size() <= (size_t)PAIR_TERMS; r++)
+    const bool terms = !zoff.empty() && N >= 2 && nc_of(N, M) <= pair_terms_rows();
+    if (terms) zterm.reserve(PAIR_TERMS + pair_count(M));
+    for (size_t r = 0; terms && r + 1 < zoff.size() && zterm.size() <= (size_t)PAIR_TERMS; r++)
         for (int x = zoff[r]; x < zoff[r + 1] && zterm.size() <= (size_t)PAIR_TERMS; x++)
             for (int y = zoff[r]; y < zoff[r + 1]; y++) {
                 const int P = zord[x], Q = zord[y], c2 = pair_hi(P), q2 = pair_hi(Q);
@@ -231,7 +241,7 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
                                  0});
             }
     const int nterm = zterm.size() <= (size_t)PAIR_TERMS ? (int)zterm.size() : 0;
-    if (!zoff.empty()) zterm.resize(PAIR_TERMS);
+    if (terms) zterm.resize(PAIR_TERMS);
     // blocks of one pair: a*_q a*_l a_q a_l is diagonal, so they need neither
     // of the two passes (Lieb-Liniger: the two lowest and the two highest
     // total momenta)
@@ -345,6 +355,10 @@ mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefD
     c->ttc = (cplx *)(dev + o_ttc);
     c->ph1 = pair ? (cplx *)(dev + o_ph1) : nullptr;
     c->pwf = pwf.empty() ? nullptr : (cplx *)(dev + o_pwf);
+    if (keep && pwf.empty() && pair && M <= MCPI_PAIR_MAXM && N >= 2) {
+        keep->w = std::move(pw);
+        keep->h1 = std::move(ph1);
+    }
     const bool fac = !zblk.empty();
     c->pza = fac ? (cplx *)(dev + o_za) : nullptr;
     c->pzb = fac ? (cplx *)(dev + o_zb) : nullptr;
@@ -706,6 +720,30 @@ static cplx *pair_workspace(mcpi_basis b, hipStream_t st, bool may_alloc, size_t
 
 static bool pair_schedule_ok(mcpi_ham h) { return pair_applicable(h->basis->d, h->c); }
 
+// lays out the pair product's tables of a factorized Hamiltonian, if they are
+// wanting and may be allocated (not under capture); without them schedule 6
+// does not apply
+static void pair_tables(mcpi_ham h, bool may_alloc)
+{
+    std::lock_guard<std::mutex> lock(h->pair_mu);
+    if (h->c.pwf || h->pair.w.empty() || !may_alloc) return;
+    const int N = h->basis->d.N, M = h->basis->d.M;
+    std::vector<cplx> f(fragment_entries(M), cmake(0, 0));
+    pair_fragments(N, M, h->pair.w.data(), h->pair.h1.data(), f.data());
+    void *p = nullptr;
+    if (hipMalloc(&p, sizeof(cplx) * f.size()) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    if (hipMemcpy(p, f.data(), sizeof(cplx) * f.size(), hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(p);
+        return;
+    }
+    h->pwf_block = (cplx *)p;
+    h->c.pwf = h->pwf_block;
+}
+
 // one H.v with schedule `sched`; 4 = specialised kernel reading the pattern
 // tables of the Hamiltonian's zero pattern (built on first use unless the
 // stream is capturing or memory is short; schedule 2 otherwise)
@@ -732,10 +770,10 @@ static mcpi_status launch_sched(mcpi_ham h, int sched, const cplx *C, cplx *out,
         return launch_apply_raw(bd, h->basis->maps, h->c, 1, 2, C, out, st);
     }
     if (sched == 6 || sched == 7) {
-        const bool ok = sched == 7 ? pairz_applicable(b, h->c) : pair_schedule_ok(h);
-        if (ok) {
-            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-            MCPI_HIP(hipStreamIsCapturing(st, &cs));
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        MCPI_HIP(hipStreamIsCapturing(st, &cs));
+        if (sched == 6) pair_tables(h, cs == hipStreamCaptureStatusNone);
+        if (sched == 7 ? pairz_applicable(b, h->c) : pair_schedule_ok(h)) {
             cplx *ws = pair_workspace(h->basis, st, cs == hipStreamCaptureStatusNone, pair_need(h, sched));
             if (ws) return sched == 7 ? launch_pairz(b, h->c, C, out, ws, st, e) : launch_pair(b, h->c, C, out, ws, st, e);
         }

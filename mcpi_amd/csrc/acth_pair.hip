@@ -212,6 +212,20 @@ mcpi_status launch_pair(const BasisDev &b, const HamCoefDev &c, const cplx *C, c
     return b.M <= 9 ? launch_pair_a(b, c, C, out, ws, st, e) : launch_pair_b(b, c, C, out, ws, st, e);
 }
 
+// By terms while every row's wavefront is resident at once (32 a CU); us a
+// H.v through the pair space and by terms: N = 6, M = 9 (3,003 rows) 8.5, 5.0;
+// N = 6, M = 11 (8,008) 9.4, 9.0; N = 8, M = 9 (12,870) 8.8, 11.0.
+int64_t pair_terms_rows()
+{
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return (int64_t)32 * ncu;
+}
+
 bool pairz_applicable(const BasisDev &b, const HamCoefDev &c)
 {
     return c.pza && c.pzR > 0 && b.occ2 && b.M >= 3 && b.M <= MCPI_PAIRZ_MAXM && !b.perm && b.IF && b.nc <= INT32_MAX &&
@@ -231,13 +245,7 @@ mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, 
                         hipStream_t st, PairEpi *e)
 {
     MCPI_ARG(pairz_applicable(b, c), "the factorized pair-space H.v does not apply to this basis and Hamiltonian");
-    // by terms while every row's wavefront is resident at once (32 a CU); us a
-    // H.v through the pair space and by terms: N = 6, M = 9 (3,003 rows) 8.5, 5.0;
-    // N = 6, M = 11 (8,008) 9.4, 9.0; N = 8, M = 9 (12,870) 8.8, 11.0
-    int dev = 0, ncu = 0;
-    MCPI_HIP(hipGetDevice(&dev));
-    MCPI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    if (c.pznt > 0 && b.nc <= (int64_t)32 * ncu)
+    if (c.pznt > 0)   // (there are terms on bases of few rows only)
         return b.M <= 8    ? launch_pair_terms<1>(b, c, C, out, st, e)
                : b.M <= 16 ? launch_pair_terms<2>(b, c, C, out, st, e)
                            : launch_pair_terms<3>(b, c, C, out, st, e);

@@ -151,7 +151,7 @@ mcpi_status mcpi_hip_ham_create(mcpi_basis b, const mcpi_cplx *Ho, const mcpi_cp
         }
     }
     mcpi_status st = build_coefficients(M, (const cplx *)Ho, (const cplx *)Hint, &h->c, &h->coef_block,
-                                        &h->coef_bytes, b->d.N);
+                                        &h->coef_bytes, b->d.N, &h->pair);
     // sector order: the zero-skipping kernel on the pattern tables is the one
     // H.v, so its term lists are walked even when most terms are non-zero
     if (st == MCPI_OK && b->sectored()) h->c.dense = 0;
@@ -176,6 +176,7 @@ mcpi_status mcpi_hip_ham_destroy(mcpi_ham h)
     if (!h) return MCPI_OK;
     (void)hipDeviceSynchronize();
     if (h->coef_block) (void)hipFree(h->coef_block);
+    if (h->pwf_block) (void)hipFree(h->pwf_block);
     if (h->Ho_dev) (void)hipFree(h->Ho_dev);
     if (h->Hint_dev) (void)hipFree(h->Hint_dev);
     delete h;

@@ -277,7 +277,8 @@ struct HamCoefDev {
     // w with the one-body part folded in for N >= 2 particles (a*_k a_l =
     // sum_s a*_k a*_s a_s a_l / (N - 1)), as the fragments of the pair product:
     // [s][g][lane] = w[16 g + lane % 16][4 s + lane / 16], zero past the pairs
-    // (M <= MCPI_PAIR_MAXM and N given to build_coefficients; null otherwise)
+    // (M <= MCPI_PAIR_MAXM and N given to build_coefficients; null otherwise, and
+    // for a factorized pair form until schedule 6 runs)
     cplx *pwf;
     // factorized pair form (schedule 7; null / 0 unless h1 is diagonal and
     // w is block diagonal with rank-one blocks): w[P][Q] = pza[P] pzb[Q]
@@ -296,8 +297,9 @@ struct HamCoefDev {
                      // start at pairs [w].j
     PairDiag *pzdiag;
     int pznd;
-    PairTerm *pzterm;   // w term by term, single pairs included, if there are
-    int pznt;           // at most PAIR_TERMS terms (else pznt is 0)
+    PairTerm *pzterm;   // w term by term, single pairs included, if the basis has
+    int pznt;           // at most pair_terms_rows() rows and w at most PAIR_TERMS
+                        // terms (else pznt is 0)
     int pzR;
     PairOff *pql;    // pairs P (with ph1; null otherwise)
     int real;        // 1 if every coefficient above has a zero imaginary part
@@ -330,7 +332,7 @@ __host__ __device__ inline HamCoefDev shift_coef(HamCoefDev c, ptrdiff_t d)
     c.nz_e = sh(c.nz_e);
     c.nz_c = sh(c.nz_c);
     if (c.ph1) c.ph1 = sh(c.ph1);
-    if (c.pwf) c.pwf = sh(c.pwf);
+    c.pwf = nullptr;   // (read by one Hamiltonian at a time only)
     if (c.pza) {
         c.pza = sh(c.pza);
         c.pzb = sh(c.pzb);
@@ -374,6 +376,12 @@ __host__ __device__ inline int pair_of2(int a, int b)
 // specialised kernels
 #define MCPI_PAIRZ_MULTI_MAXM 13
 
+// pair matrix and one-body table of a factorized Hamiltonian, kept on the host
+// for the pair product's tables
+struct PairHost {
+    std::vector<cplx> w, h1;
+};
+
 struct mcpi_ham_s {
     mcpi_basis basis;
     HamCoefDev c;
@@ -386,6 +394,11 @@ struct mcpi_ham_s {
     int skip_zero;
     int schedule;
     int tuned[2];       // autotuned schedule per skip_zero value (0 = not tuned)
+    // c.pwf of a factorized Hamiltonian: laid out from `pair` when schedule 6
+    // first runs, in an allocation of its own
+    PairHost pair;
+    cplx *pwf_block = nullptr;
+    std::mutex pair_mu;
 };
 
 namespace mcpi {
@@ -429,9 +442,11 @@ mcpi_status launch_comp(const BasisDev &b, const HamCoefDev &c, const cplx *C, c
 // wavefronts (Map and packed tables; 2 when the basis has no packed tables)
 mcpi_status launch_apply_raw(const BasisDev &b, int maps, const HamCoefDev &c, int skip_zero,
                              int schedule, const cplx *C, cplx *out, hipStream_t st);
-// N: particles, for the tables of the pair product (0: without them)
+// N: particles, for the tables of the pair product and of the terms (0: without
+// them); keep: receives what the pair product's tables are made of where they
+// are not made here
 mcpi_status build_coefficients(int M, const cplx *Ho, const cplx *Hint, HamCoefDev *c, void **block,
-                               size_t *block_bytes = nullptr, int N = 0);
+                               size_t *block_bytes = nullptr, int N = 0, PairHost *keep = nullptr);
 mcpi_status basis_upload_raw(int N, int M, const int32_t *IF, const int32_t *NCmat,
                              const int32_t *Map, const int32_t *MapOT, const int32_t *MapTT,
                              const int *strideOT, const int *strideTT, int64_t ot_len,
@@ -458,6 +473,8 @@ mcpi_status launch_pair(const BasisDev &b, const HamCoefDev &c, const cplx *C, c
 // the Hamiltonian's pair matrix factorizes, N >= 2); launch into a
 // workspace of (blocks) x pair_ld(NC(N-2, M)) complex entries
 bool pairz_applicable(const BasisDev &b, const HamCoefDev &c);
+// rows up to which schedule 7 goes term by term on the current device
+int64_t pair_terms_rows();
 mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
                          hipStream_t st, PairEpi *e = nullptr);
 // the same for chunks x mv (mv 2 or 4) Hamiltonians of one basis whose
