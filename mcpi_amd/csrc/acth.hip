@@ -774,8 +774,9 @@ static mcpi_status launch_sched(mcpi_ham h, int sched, const cplx *C, cplx *out,
         MCPI_HIP(hipStreamIsCapturing(st, &cs));
         if (sched == 6) pair_tables(h, cs == hipStreamCaptureStatusNone);
         if (sched == 7 ? pairz_applicable(b, h->c) : pair_schedule_ok(h)) {
-            cplx *ws = pair_workspace(h->basis, st, cs == hipStreamCaptureStatusNone, pair_need(h, sched));
-            if (ws) return sched == 7 ? launch_pairz(b, h->c, C, out, ws, st, e) : launch_pair(b, h->c, C, out, ws, st, e);
+            const bool terms = sched == 7 && pairz_by_terms(h->c);
+            cplx *ws = terms ? nullptr : pair_workspace(h->basis, st, cs == hipStreamCaptureStatusNone, pair_need(h, sched));
+            if (ws || terms) return sched == 7 ? launch_pairz(b, h->c, C, out, ws, st, e) : launch_pair(b, h->c, C, out, ws, st, e);
         }
         sched = 2;
     }
@@ -822,7 +823,7 @@ static mcpi_status autotune(mcpi_ham h, const cplx *C, cplx *out, hipStream_t st
     // factorized form, where it applies, does less work than the dense
     // product in a smaller workspace, and stands in for it
     if (h->skip_zero && pairz_applicable(b, h->c)) {
-        if (pair_workspace(h->basis, st, true, pair_need(h, 7))) cands[n++] = 7;
+        if (pairz_by_terms(h->c) || pair_workspace(h->basis, st, true, pair_need(h, 7))) cands[n++] = 7;
     } else if (h->skip_zero && has_fast_kernel(b.N, b.M) && pair_schedule_ok(h) &&
                pair_workspace(h->basis, st, true, pair_need(h, 6))) {
         cands[n++] = 6;

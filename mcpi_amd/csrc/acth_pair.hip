@@ -245,10 +245,11 @@ mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, 
                         hipStream_t st, PairEpi *e)
 {
     MCPI_ARG(pairz_applicable(b, c), "the factorized pair-space H.v does not apply to this basis and Hamiltonian");
-    if (c.pznt > 0)   // (there are terms on bases of few rows only)
+    if (pairz_by_terms(c))   // (there are terms on bases of few rows only)
         return b.M <= 8    ? launch_pair_terms<1>(b, c, C, out, st, e)
                : b.M <= 16 ? launch_pair_terms<2>(b, c, C, out, st, e)
                            : launch_pair_terms<3>(b, c, C, out, st, e);
+    MCPI_ARG(ws, "no workspace for the factorized pair-space H.v");
     return launch_pairz_any(b, c, 1, 1, C, out, 0, 0, ws, st, e);
 }
 

@@ -471,10 +471,12 @@ mcpi_status launch_pair(const BasisDev &b, const HamCoefDev &c, const cplx *C, c
                         hipStream_t st, PairEpi *e = nullptr);
 // schedule 7 (acth_pair.hip): the factorized pair form applies (as 6, and
 // the Hamiltonian's pair matrix factorizes, N >= 2); launch into a
-// workspace of (blocks) x pair_ld(NC(N-2, M)) complex entries
+// workspace of (blocks) x pair_ld(NC(N-2, M)) complex entries (null by terms)
 bool pairz_applicable(const BasisDev &b, const HamCoefDev &c);
 // rows up to which schedule 7 goes term by term on the current device
 int64_t pair_terms_rows();
+// it does so for this Hamiltonian, without a workspace
+inline bool pairz_by_terms(const HamCoefDev &c) { return c.pznt > 0; }
 mcpi_status launch_pairz(const BasisDev &b, const HamCoefDev &c, const cplx *C, cplx *out, cplx *ws,
                          hipStream_t st, PairEpi *e = nullptr);
 // the same for chunks x mv (mv 2 or 4) Hamiltonians of one basis whose
