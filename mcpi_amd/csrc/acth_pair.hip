@@ -265,10 +265,12 @@ mcpi_status launch_pairz_multi(const BasisDev &b, const HamCoefDev &c, int mv, i
 }  // namespace mcpi
 
 // H.v of h through the pair space on every size, as if it had more terms than
-// are kept (for tests; not part of the public interface).
+// are kept; what was tuned with them is tuned again (for tests; not part of the
+// public interface).
 extern "C" mcpi_status mcpi_hip_ham_drop_terms(mcpi_ham h)
 {
     MCPI_ARG(h, "null Hamiltonian");
     h->c.pznt = 0;
+    h->tuned[0] = h->tuned[1] = 0;
     return MCPI_OK;
 }

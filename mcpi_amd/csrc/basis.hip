@@ -1075,8 +1075,10 @@ mcpi_status mcpi_hip_basis_create(int N, int M, int maps, mcpi_basis *out)
 mcpi_status mcpi_hip_basis_drop_occ2(mcpi_basis b)
 {
     MCPI_ARG(b, "null basis");
-    if (b->d.occ2) MCPI_HIP(hipFree(b->d.occ2));
+    if (!b->d.occ2) return MCPI_OK;
+    MCPI_HIP(hipFree(b->d.occ2));
     b->d.occ2 = nullptr;
+    b->device_bytes -= nc_of(b->d.N - 2, b->d.M) * occ_stride(b->d.M);
     return MCPI_OK;
 }
 

@@ -491,3 +491,11 @@ mcpi_status launch_pairz_multi(const BasisDev &b, const HamCoefDev &c, int mv, i
 mcpi_status basis_build_parts(mcpi_basis b, int want_map, int want_ot, int want_tt);
 
 }  // namespace mcpi
+
+// Test hooks, outside the public interface.  The handle must not be in use: what
+// was captured or tuned with the tables is not told of it, beyond what the
+// hook says where it is defined.
+extern "C" {
+mcpi_status mcpi_hip_basis_drop_occ2(mcpi_basis b);
+mcpi_status mcpi_hip_ham_drop_terms(mcpi_ham h);
+}
