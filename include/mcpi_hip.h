@@ -290,15 +290,17 @@ mcpi_status mcpi_hip_ham_set_skip_zero(mcpi_ham h, int on);
  * map; 3 <= M <= 12, bases in the reference order; a workspace of about
  * M(M+1)/2 NC(N-2, M) complex entries per stream that runs
  * the schedule, allocated on that stream's first use outside stream capture,
- * is kept with the basis; falls back to 2 otherwise or when device memory
- * is short), 7 = 6 in the factorized pair form, for Hamiltonians whose
+ * is kept with the basis, as are, for a Hamiltonian to which 7 applies, the
+ * product's tables with the Hamiltonian; falls back to 2 otherwise or when
+ * device memory is short), 7 = 6 in the factorized pair form, for Hamiltonians whose
  * one-body part is diagonal and whose pair matrix is block diagonal with
  * blocks of rank one, W[P][Q] = a[P] b[Q] (contact interactions that conserve
  * a pair charge, such as Lieb-Liniger's): per block r, Z_r = sum_Q b[Q] a_Q C
  * is gathered over the states of N-2 particles and each row gathers its
  * a[P] Z_r back, with no matrix product (3 <= M <= 24, N >= 2; a
  * workspace of R NC(N-2, M) complex entries per stream, R the number of
- * blocks, kept likewise; a smaller workspace stays allocated beside a larger
+ * blocks, kept likewise, and none on bases of few rows, where it goes term by
+ * term; a smaller workspace stays allocated beside a larger
  * one until the basis is freed; falls back to 2 otherwise).  The autotuner
  * takes 6 and 7 among its candidates only with zero-skipping on, since they
  * read no map, and 7 in place of 6 where it applies.  Where

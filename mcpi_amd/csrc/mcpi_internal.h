@@ -97,7 +97,8 @@ struct BasisDev {
     int32_t *NCmat;     // (N+1)*(M+1), reference layout
     // occupations of the states with N - 2 particles, one byte per orbital in
     // rows of 16 (M <= 16) or 32 bytes; null for N < 2, or when the device had
-    // no memory for it (the pair amplitudes then unrank their rows)
+    // no memory for it (the densities then unrank their rows, and schedules 6 and
+    // 7 do not apply)
     uint8_t *occ2;
     // Wave-packed double-jump targets (full maps only; see basis.hip): for
     // each wavefront of 64 consecutive rows w, the slots of the jumps active

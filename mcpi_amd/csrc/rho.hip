@@ -31,19 +31,20 @@
 // S_d(x) = sum_{j=1}^{x} B[j][P_j(u) + d]:
 //   rank(u + e_q + e_l) = nc - 1 - S_2(M-1) - (S_0(q) - S_1(q)) - (S_1(l) - S_2(l))
 //   rank(u + e_k)       = nc - 1 - S_1(M-1) - (S_0(k) - S_1(k))
-// Each row u of a tile is unranked once (greedy over the same B table: the
-// combinatorial number system) and its two difference tables are kept in
-// LDS, so a gather costs two LDS reads and two subtractions.
+// Each row u of a tile has its two difference tables and the roots of its
+// occupations made once, in LDS (pair_rows.h), so a gather costs four LDS reads,
+// two subtractions and a product.
 //
 // Kernel k_gram: a block owns one tile pair (TI, TJ) of 80 x 80 entries of
 // the Gram matrix and loops over tiles of U rows of Phi (32 for rho2, 128
-// for rho1, whose Phi has at most 32 columns).  The tile's rows are
-// unranked (one thread per row, during the previous tile's products), its
-// entries gathered into LDS (lanes over consecutive rows of one column:
-// neighbouring targets; GB loads in flight per thread), and the product
-// runs on the FP64 matrix cores in 16 x 16 sub-blocks: the sub-blocks i <= j
-// of a diagonal tile pair, all of them off it, dealt out to the block's four
-// wavefronts.  Phi stays in LDS in one layout for both operands, because
+// for rho1, whose Phi has at most 32 columns).  The row tables come from the
+// basis's occupation table, two threads a row (without it, and for rho1, a
+// thread unranks a row: greedy over B, the combinatorial number system), during
+// the previous tile's products; the entries are gathered into LDS (lanes over
+// consecutive rows of one column: neighbouring targets; all of a thread's loads
+// in flight together), and the product runs on the FP64 matrix cores in 16 x 16
+// sub-blocks: the sub-blocks i <= j of a diagonal tile pair, all of them off it,
+// dealt out to the block's eight wavefronts (GramSplit).  Phi stays in LDS in one layout for both operands, because
 // v_mfma_f64_16x16x4f64 takes A[i][k] and B[k][j] from the same lanes
 // (i or j = lane % 16, k = lane / 16): lane (i, k) of step s reads column i of
 // row 4 s + k.
@@ -58,6 +59,14 @@
 // product 0.32 -> 0.18; N = 16 (4,457,400 rows) 5.26 -> 2.12 ms, the product
 // 4.2 -> 2.1 ms or 49 TFLOP/s issued (before: vector FMAs, unranked rows and a
 // Gram product of its own for rho1).
+// Rounding: the three products' errors are relative to |x| |y|, also in the part
+// of a product that is small beside the other.  Over random complex vectors the
+// result's relative error is 0.81 (rho2) and 0.62 (rho1) of that of the vector
+// FMAs before (against 80-bit sums, 13 sizes from N = 2, M = 24 to N = 60, M = 3), a
+// real vector has no imaginary part, but one whose imaginary parts are 1e-6 of
+// the real ones keeps them to 1e-9 of themselves instead of 1e-15.  Four real
+// products would keep them: 2.50 instead of 2.15 ms at N = 16, M = 12, 0.267
+// instead of 0.237 at N = 12.
 // Each block writes its sub-blocks once; two fixed-order stages sum the
 // blocks (deterministic result), the second one inside the kernel that
 // expands the Gram matrix into the full rho1 / rho2 arrays on the device.
